@@ -25,6 +25,7 @@
 #include "flow.h"
 #include "hier_logistic.h"
 #include "glm_large.h"
+#include "glm_wide.h"
 #include "nuts_types.h"
 
 using namespace nutsgpu;
@@ -128,8 +129,9 @@ struct ModelImpl {
   DevBuf<double> d_data;
   std::vector<int64_t> ds_off;
   // logistic regression batched paths (single dataset): glm for D <= 128 (FP64
-  // or FP32/BF16 contraction), glm_large for larger D (FP32/BF16 contraction)
-  bool glm = false, glm_large = false;
+  // or FP32/BF16 contraction), glm_large for larger D (FP32/BF16 contraction),
+  // glm_wide its FP64 kernel (D <= 1024)
+  bool glm = false, glm_large = false, glm_wide = false;
   int glmN = 0, glmD = 0;
   double glm_s2inv = 0;
   const double* d_X = nullptr;
@@ -738,8 +740,13 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   const bool hl_ok = M.kind == MK_HIER_LOGISTIC && nds == 1;
   // large-D logistic regression: two-pass FP32 matrix-core gradient (X FP32 or BF16)
   const bool gl_ok = (M.glm_large || small_as_large) && nds == 1 && cfg.precision != 0 && (cfg.fused != 1 || R.flow);
+  // the same in FP64: the column-split matrix-core kernel.  Against the per-chain
+  // functor on the fused kernel it wins at every table size: the functor takes
+  // about 0.3 us per column and 64 rows (40 us already at D = 129, N <= 64), a
+  // lockstep step of four launches about 30 us
+  const bool gw_ok = M.glm_wide && nds == 1 && cfg.precision == 0 && (cfg.fused != 1 || R.flow);
   if (M.plugin && cfg.fused == 1) throw std::invalid_argument("plugin models run on the lockstep kernels (fused=0)");
-  if (cfg.fused < 0) fused = !glm_ok && !hl_ok && !gl_ok && !M.plugin;
+  if (cfg.fused < 0) fused = !glm_ok && !hl_ok && !gl_ok && !gw_ok && !M.plugin;
   if (R.flow) {
     if (nds != 1 || R.flow->dim() != D[0] || R.flow->max_rows() < C)
       throw std::invalid_argument("flow: one dataset whose dimension matches the flow, at most max_rows chains");
@@ -823,7 +830,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   // flow: the GLM gradients read the packed rows x = T(z) and write packed
   // rows; the identity list maps position r to row r
   DevBuf<int> ident;
-  if (R.flow && (glm_ok || gl_ok)) {
+  if (R.flow && (glm_ok || gl_ok || gw_ok)) {
     std::vector<int> h(C);
     std::iota(h.begin(), h.end(), 0);
     ident.upload(h, st);
@@ -862,8 +869,25 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
       else xlow = M.low_x(cfg.precision, st);
     }
   }
+  GlmWidePlan gwplan;
+  if (!fused && gw_ok) {
+    act_idx.alloc(C);
+    n_act.alloc(1);
+    gwplan = glm_wide_plan(M.glmN, C, M.glmD, num_cus());
+    work.alloc(gwplan.work_doubles);
+    ga.X = M.d_X; ga.y = M.d_y; ga.N = M.glmN; ga.D = M.glmD; ga.C = C; ga.rows_per_chunk = 0;
+    ga.s2inv = M.glm_s2inv; ga.Q = Q.p; ga.ldq = Dp[0]; ga.G = G.p; ga.V = V.p; ga.work = work.p;
+    ga.idx = act_idx.p; ga.n_active = n_act.p;
+    if (R.flow) {
+      ga.Q = fX.p; ga.ldq = D[0]; ga.G = fGX.p; ga.V = fVX.p; ga.idx = ident.p;
+    }
+  }
   // the GLM gradient of the chosen kernel (FP64, FP32 or BF16-split)
   auto glm_grad = [&]() {
+    if (gw_ok) {
+      if (glm_grad_wide_f64(ga, gwplan, st)) throw std::runtime_error("GLM kernel: unsupported D");
+      return;
+    }
     const int rcg = cfg.precision == 0 ? glm_grad_mfma_f64(ga, gplan, st)
                     : xbf ? glm_grad_mfma_bf16(ga, gplan, xbf, cfg.precision, st)
                           : glm_grad_mfma_f32(ga, gplan, xlow, cfg.precision, kF32Layout, st);
@@ -930,7 +954,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
         R.flow->forward(Q.p, Dp[0], act_idx.p, n_act.p, C, fX.p, fLD.p);
         if (hl_ok) {
           hl_grad_launch(hla, hl_groups, st);
-        } else if (glm_ok) {
+        } else if (glm_ok || gw_ok) {
           ga.n_active = n_act.p;
           glm_grad();
         } else if (gl_ok) {
@@ -943,7 +967,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
         }
         R.flow->pullback(fGX.p, fVX.p, fLD.p, act_idx.p, n_act.p, C, G.p, Dp[0], V.p);
         if (with_events) HIPC(hipEventRecord(ev.b[k], st));
-      } else if (glm_ok) {
+      } else if (glm_ok || gw_ok) {
         launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
         ga.ev_begin = with_events ? ev.a[k] : nullptr;
         ga.ev_end = with_events ? ev.b[k] : nullptr;
@@ -1458,6 +1482,7 @@ nuts_model* nuts_model_create(const char* family, const nuts_data* const* datase
     if (M.kind == MK_LOGISTIC && num_datasets == 1) {
       M.glm = M.ds[0].D <= 128;
       M.glm_large = !M.glm;
+      M.glm_wide = glm_wide_ok(M.ds[0].D);
       M.glmN = (int)packed[0];
       M.glmD = (int)packed[1];
       M.glm_s2inv = packed[2];
@@ -1565,6 +1590,12 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
       gl_bind(M, a, gp, gs, precision, 0);
       a.C = C; a.Q = Q.p; a.ldq = Dp; a.G = G.p; a.V = V.p;
       gl_large_grad(a, gp, M.low_x(precision, 0), precision, 0);
+      HIPC(hipDeviceSynchronize());
+    } else if (M.glm_wide && dataset == 0) {
+      const GlmWidePlan gp = glm_wide_plan(M.glmN, C, D, num_cus());
+      DevBuf<double> work(gp.work_doubles);
+      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, C, 0, M.glm_s2inv, Q.p, Dp, G.p, V.p, work.p};
+      if (glm_grad_wide_f64(ga, gp, 0)) throw std::runtime_error("GLM kernel: unsupported D");
       HIPC(hipDeviceSynchronize());
     } else if (M.glm && dataset == 0) {
       // reduced precision: the kernel the sampler's autotuner picks for this many points
@@ -1909,6 +1940,11 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       need(gp.work_doubles);
       GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, gp.rows_per_chunk, M.glm_s2inv, d_q, D, d_grad, V, work};
       if (glm_grad_mfma_f64(ga, gp, st)) throw std::runtime_error("GLM kernel: unsupported D");
+    } else if (M.glm_wide && dataset == 0) {
+      const GlmWidePlan gp = glm_wide_plan(M.glmN, n, D, num_cus(), work_cap);
+      need(gp.work_doubles);
+      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, 0, M.glm_s2inv, d_q, D, d_grad, V, work};
+      if (glm_grad_wide_f64(ga, gp, st)) throw std::runtime_error("GLM kernel: unsupported D");
     } else if (M.kind == MK_HIER_LOGISTIC) {
       const Dataset& hd = M.ds[dataset];
       need(hl_work_doubles(hd.groups, hd.group_size, n));
