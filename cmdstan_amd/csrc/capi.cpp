@@ -254,7 +254,8 @@ Dataset make_dataset(const std::string& fam, const nuts_data& d, int& kind) {
     s.names = idx_names("x", D); s.unames = s.names;
     s.block.push_back(D);
     s.block.insert(s.block.end(), mu.begin(), mu.end());
-    s.block.insert(s.block.end(), P.begin(), P.end());
+    for (int j = 0; j < D; ++j)  // transposed: the gradient's lanes own rows
+      for (int i = 0; i < D; ++i) s.block.push_back(P[(size_t)i * D + j]);
   } else if (fam == "eight_schools_cp" || fam == "hier_normal_nc") {
     const bool nc = fam == "hier_normal_nc";
     kind = nc ? MK_HIER_NORMAL_NC : MK_EIGHT_SCHOOLS;
@@ -695,7 +696,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
 
   NutsBuffers B;
   std::memset(&B, 0, sizeof(B));
-  B.C = C; B.D = dD.p; B.Dp = dDp.p; B.off = doffb.p; B.moff = dmoff.p; B.uid = duid.p;
+  B.C = C; B.max_Dp = *std::max_element(Dp.begin(), Dp.end()); B.D = dD.p; B.Dp = dDp.p; B.off = doffb.p; B.moff = dmoff.p; B.uid = duid.p;
   B.Q = Q.p; B.G = G.p; B.V = V.p; B.pool = pool.p; B.st = dst.p; B.minv = minv.p;
   B.draws = draws.p; B.draw_off = ddoff.p; B.user_init = R.init ? uinit.p : nullptr;
   B.n_stopped = dstop.p; B.need = dneed.p;

@@ -56,17 +56,57 @@ __device__ __forceinline__ double stream_normal(uint64_t seed, uint32_t chain, u
 }
 
 // ----------------------------------------------------------------- reductions
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = NUTS_WAVE / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, NUTS_WAVE);
-  return v;
+// One butterfly step on both halves of a double by a rotation inside rows of 16
+// lanes: once lanes 8 apart hold the same value, rotating by 4 is the exchange
+// of lanes 4 apart, and so on down.
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xF, 0xF, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xF, 0xF, false);
+  return __hiloint2double(hi, lo);
 }
 
-__device__ __forceinline__ int wave_and(int v) {
-#pragma unroll
-  for (int off = NUTS_WAVE / 2; off > 0; off >>= 1) v &= __shfl_xor(v, off, NUTS_WAVE);
-  return v;
+__device__ __forceinline__ double uniform_value(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
 }
+
+// Sums of N values over the wave, every lane gets them: the lane-xor butterfly
+// (32, 16, 8, 4, 2, 1) with the additions of __shfl_xor's form -- the same bits
+// -- on the vector unit's lane moves instead of six dependent trips through the
+// LDS permute unit per value; the N chains interleave.
+template <int N>
+__device__ __forceinline__ void wave_sum_n(double (&v)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) {  // upper half of a copy swapped for the lower: (lower, lower) + (upper, upper)
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(v[k]), __double2loint(v[k]), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(v[k]), __double2hiint(v[k]), false, false);
+    v[k] = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) {  // the same with rows of 16
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(v[k]), __double2loint(v[k]), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(v[k]), __double2hiint(v[k]), false, false);
+    v[k] = __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+  }
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] += dpp_move<0x128>(v[k]);  // row_ror:8
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] += dpp_move<0x124>(v[k]);  // row_ror:4
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] += dpp_move<0x122>(v[k]);  // row_ror:2
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = uniform_value(v[k] + dpp_move<0x121>(v[k]));  // row_ror:1
+}
+
+__device__ __forceinline__ double wave_sum(double v) {
+  double a[1] = {v};
+  wave_sum_n(a);
+  return a[0];
+}
+
+// and of 0/1 flags
+__device__ __forceinline__ int wave_and(int v) { return __all(v != 0) ? 1 : 0; }
 
 // ------------------------------------------------------------ scalar math
 // 1/d for d in [1, 8]: the hardware reciprocal estimate refined by two Newton

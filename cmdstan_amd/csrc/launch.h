@@ -36,6 +36,9 @@ void launch_dense_factor(const NutsBuffers& B, int* failed, hipStream_t st);
 // dot products and tree weights stay FP64
 void launch_advance_fused(int kind, int metric, bool vec32, const NutsParams& P, const NutsBuffers& B,
                           const ModelDataDev& md, hipStream_t st);
+// the same with every chain's vectors in LDS (false: they do not fit, or too many chains)
+bool launch_advance_fused_lds(int kind, int metric, bool vec32, const NutsParams& P, const NutsBuffers& B,
+                              const ModelDataDev& md, hipStream_t st);
 // the same with one 256-thread block per chain (false: the model has no
 // block-wide gradient, or dense_e)
 bool launch_advance_fused_block(int kind, int metric, bool vec32, const NutsParams& P, const NutsBuffers& B,

@@ -5,7 +5,8 @@
 // stan::model::log_prob_grad<true, jacobian>) and writes gV = -grad log p.
 // Model data are packed per dataset into one double array; `off[c]` gives the
 // dataset block of chain c.  write_array maps an unconstrained draw to the
-// constrained outputs in Stan's column order.
+// constrained outputs in Stan's column order.  bind(c) names the chain the next
+// calls are for: it resolves the chain's block once, not once per gradient.
 #pragma once
 #include "device_common.h"
 
@@ -15,6 +16,7 @@ struct ModelData {
   const double* data;
   const int64_t* off;   // [C] offset of the chain's dataset block in data
   double jac;           // 1: add the log-Jacobian of the constraining transforms
+  const double* d;      // the bound chain's block (bind)
 };
 
 // examples/bernoulli/bernoulli.stan: theta ~ beta(1,1); y ~ bernoulli(theta);
@@ -24,13 +26,20 @@ struct BernoulliFn {
   static constexpr bool block_grad = false;
   static constexpr bool vec32 = true;  // FP32 vector storage supported
   ModelData md;
+  double N, s;
+  __device__ __forceinline__ void bind(int c) {
+    md.d = md.data + md.off[c];
+    N = md.d[0];
+    s = md.d[1];
+  }
   template <class T>
   __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
-    const double* d = md.data + md.off[c];
-    const double N = d[0], s = d[1];
+    // log1p_exp(u), log1p_exp(-u) and inv_logit(u) share e^-|u| and log1p of it
     const double u = q[0];
-    const double t = inv_logit(u);
-    const double lt = -log1p_exp(-u), l1t = -log1p_exp(u);
+    const double e = exp(u >= 0 ? -u : u);
+    const double l = log1p(e);
+    const double t = (u >= 0 ? 1.0 : e) / (1.0 + e);
+    const double lt = -(u < 0 ? -u + l : l), l1t = -(u > 0 ? u + l : l);
     double lp = s * lt + (N - s) * l1t;
     if (md.jac != 0) lp += lt + l1t;
     const double gr = (s + md.jac) * (1.0 - t) - (N - s + md.jac) * t;
@@ -41,30 +50,81 @@ struct BernoulliFn {
   __device__ void write_array(int, const double* q, double* out) const { out[0] = inv_logit(q[0]); }
 };
 
-// q ~ multi_normal_prec(mu, P); block = [D, mu[D], P[D*D] row-major]
+// q ~ multi_normal_prec(mu, P); block = [D, mu[D], P transposed [D*D] row-major]:
+// lanes own rows of P, so its transpose makes a column's read coalesced
 struct GaussFn {
   static constexpr bool fused = true;
   static constexpr bool block_grad = false;
   static constexpr bool vec32 = true;  // FP32 vector storage supported
   ModelData md;
+  __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
+  // rows i0 + lane + 64 r (r < RB) of P (q - mu), columns in order, 16 loads in
+  // flight; q - mu of 64 columns sits in the lanes and is broadcast by lane reads
+  template <int RB, class T>
+  __device__ __forceinline__ double rows(const T* __restrict__ q, T* __restrict__ gV, int D, int lane, int i0,
+                                         double acc) const {
+    const double* mu = md.d + 1;
+    const double* Pt = md.d + 1 + D;
+    constexpr int U = 16 / RB;
+    double si[RB];
+    int ii[RB];
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      si[r] = 0.0;
+      const int i = i0 + lane + NUTS_WAVE * r;
+      ii[r] = i < D ? i : D - 1;
+    }
+    for (int jb = 0; jb < D; jb += NUTS_WAVE) {
+      const int jl = jb + lane < D ? jb + lane : D - 1;
+      const double dl = (double)q[jl] - mu[jl];
+      auto diff = [&](int j) {
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(dl), j),
+                                __builtin_amdgcn_readlane(__double2loint(dl), j));
+      };
+      const int nj = D - jb < NUTS_WAVE ? D - jb : NUTS_WAVE;
+      int j = 0;
+      for (; j + U <= nj; j += U) {
+        double v[U][RB];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int r = 0; r < RB; ++r) v[u][r] = Pt[(int64_t)(jb + j + u) * D + ii[r]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const double x = diff(j + u);
+#pragma unroll
+          for (int r = 0; r < RB; ++r) si[r] += v[u][r] * x;
+        }
+      }
+      for (; j < nj; ++j) {
+        const double x = diff(j);
+#pragma unroll
+        for (int r = 0; r < RB; ++r) si[r] += Pt[(int64_t)(jb + j) * D + ii[r]] * x;
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const int i = i0 + lane + NUTS_WAVE * r;
+      if (i < D) {
+        gV[i] = si[r];
+        acc += (q[i] - mu[i]) * si[r];
+      }
+    }
+    return acc;
+  }
   template <class T>
-  __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int D, int lane) const {
-    const double* d = md.data + md.off[c];
-    const double* mu = d + 1;
-    const double* P = d + 1 + D;
+  __device__ double operator()(int, const T* __restrict__ q, T* __restrict__ gV, int D, int lane) const {
     double acc = 0;
-    for (int i = lane; i < D; i += NUTS_WAVE) {
-      double si = 0;
-      const double* Pi = P + (int64_t)i * D;
-      for (int j = 0; j < D; ++j) si += Pi[j] * (q[j] - mu[j]);
-      gV[i] = si;
-      acc += (q[i] - mu[i]) * si;
+    if (D <= NUTS_WAVE) {
+      acc = rows<1>(q, gV, D, lane, 0, acc);
+    } else {
+      for (int i0 = 0; i0 < D; i0 += 2 * NUTS_WAVE) acc = rows<2>(q, gV, D, lane, i0, acc);
     }
     return 0.5 * wave_sum(acc);
   }
-  __device__ int nout(int c) const { return (int)md.data[md.off[c]]; }
+  __device__ int nout(int c) const { return (int)md.d[0]; }
   __device__ void write_array(int c, const double* q, double* out) const {
-    const int D = (int)md.data[md.off[c]];
+    const int D = (int)md.d[0];
     for (int i = 0; i < D; ++i) out[i] = q[i];
   }
 };
@@ -77,9 +137,10 @@ struct EightSchoolsFn {
   static constexpr bool block_grad = false;
   static constexpr bool vec32 = true;  // FP32 vector storage supported
   ModelData md;
+  __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
   template <class T>
   __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
-    const double* d = md.data + md.off[c];
+    const double* d = md.d;
     const int J = (int)d[0];
     const double mu_s = d[1], tau_s = d[2];
     const double* y = d + 3;
@@ -104,9 +165,9 @@ struct EightSchoolsFn {
     if (lane == 0) { gV[0] = -gmu; gV[1] = -(md.jac + tau * gtau); }
     return -lp;
   }
-  __device__ int nout(int c) const { return (int)md.data[md.off[c]] + 2; }
+  __device__ int nout(int c) const { return (int)md.d[0] + 2; }
   __device__ void write_array(int c, const double* q, double* out) const {
-    const int J = (int)md.data[md.off[c]];
+    const int J = (int)md.d[0];
     out[0] = q[0]; out[1] = exp(q[1]);
     for (int j = 0; j < J; ++j) out[2 + j] = q[2 + j];
   }
@@ -120,11 +181,12 @@ struct HierNormalNCFn {
   static constexpr bool vec32 = true;       // FP32 vector storage supported
   static constexpr bool block_grad = true;  // gradient over a block per chain (group)
   ModelData md;
+  __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
   // the gradient with TPC threads per chain (thread tid); sum reduces a
   // per-thread partial over the chain's threads in a fixed order
   template <int TPC, class T, class Sum>
   __device__ double group(int c, const T* __restrict__ q, T* __restrict__ gV, int tid, const Sum& sum) const {
-    const double* d = md.data + md.off[c];
+    const double* d = md.d;
     const int J = (int)d[0];
     const double mu_s = d[1], tau_s = d[2];
     const double* y = d + 3;
@@ -155,9 +217,9 @@ struct HierNormalNCFn {
   __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
     return group<NUTS_WAVE>(c, q, gV, lane, [](double x) { return wave_sum(x); });
   }
-  __device__ int nout(int c) const { return 2 + 2 * (int)md.data[md.off[c]]; }
+  __device__ int nout(int c) const { return 2 + 2 * (int)md.d[0]; }
   __device__ void write_array(int c, const double* q, double* out) const {
-    const int J = (int)md.data[md.off[c]];
+    const int J = (int)md.d[0];
     const double tau = exp(q[1]);
     out[0] = q[0]; out[1] = tau;
     for (int j = 0; j < J; ++j) { out[2 + j] = q[2 + j]; out[2 + J + j] = q[0] + tau * q[2 + j]; }
@@ -173,9 +235,10 @@ struct HierLogisticFn {
   static constexpr bool block_grad = false;
   static constexpr bool vec32 = true;  // FP32 vector storage supported
   ModelData md;
+  __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
   template <class T>
   __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
-    const double* d = md.data + md.off[c];
+    const double* d = md.d;
     const int N = (int)d[0], K = (int)d[1], G = (int)d[2];
     const double mu_s = d[3];
     const double* gstart = d + 4;
@@ -225,11 +288,11 @@ struct HierLogisticFn {
     return -wave_sum(acc);
   }
   __device__ int nout(int c) const {
-    const double* d = md.data + md.off[c];
+    const double* d = md.d;
     return 2 * (int)d[1] + (int)d[1] * (int)d[2];
   }
   __device__ void write_array(int c, const double* q, double* out) const {
-    const double* d = md.data + md.off[c];
+    const double* d = md.d;
     const int K = (int)d[1], G = (int)d[2];
     for (int k = 0; k < K; ++k) { out[k] = q[k]; out[K + k] = exp(q[K + k]); }
     for (int k = 0; k < K; ++k)
@@ -245,8 +308,9 @@ struct LogisticFn {
   static constexpr bool block_grad = false;
   static constexpr bool vec32 = false;
   ModelData md;
+  __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
   __device__ double operator()(int c, const double* __restrict__ q, double* __restrict__ gV, int D, int lane) const {
-    const double* d = md.data + md.off[c];
+    const double* d = md.d;
     const int N = (int)d[0];
     const double s2inv = d[2];
     const double* X = d + 3;
@@ -278,11 +342,23 @@ struct LogisticFn {
     pr = wave_sum(pr);
     return -(wave_sum(acc) - 0.5 * s2inv * pr);
   }
-  __device__ int nout(int c) const { return (int)md.data[md.off[c] + 1]; }
+  __device__ int nout(int c) const { return (int)md.d[1]; }
   __device__ void write_array(int c, const double* q, double* out) const {
-    const int D = (int)md.data[md.off[c] + 1];
+    const int D = (int)md.d[1];
     for (int k = 0; k < D; ++k) out[k] = q[k];
   }
 };
+
+// runs CALL with `f`, the functor of the model kind over the data md
+#define NUTS_MODEL_SWITCH(kind, md, CALL)                       \
+  switch (kind) {                                               \
+    case MK_BERNOULLI: { BernoulliFn f{{md.data, md.off, md.jac}}; CALL; break; }    \
+    case MK_GAUSS: { GaussFn f{{md.data, md.off, md.jac}}; CALL; break; }            \
+    case MK_EIGHT_SCHOOLS: { EightSchoolsFn f{{md.data, md.off, md.jac}}; CALL; break; } \
+    case MK_HIER_NORMAL_NC: { HierNormalNCFn f{{md.data, md.off, md.jac}}; CALL; break; } \
+    case MK_HIER_LOGISTIC: { HierLogisticFn f{{md.data, md.off, md.jac}}; CALL; break; } \
+    case MK_LOGISTIC: { LogisticFn f{{md.data, md.off, md.jac}}; CALL; break; }      \
+    default: break;                                             \
+  }
 
 }  // namespace nutsgpu

@@ -362,6 +362,75 @@ __device__ __noinline__ void dense_matvec2(const double* __restrict__ M, const V
   }
 }
 
+// The same products (one or two at once) for a chain whose vectors are in LDS:
+// inlined, so x is read by LDS broadcasts, and only as many rows per lane as D
+// has (at D = 100 the eight-row form above loads eight columns' worth for two),
+// with 16 loads of M in flight.
+template <int NX, int RB, class VT>
+__device__ __forceinline__ void dense_matvec_lds_rows(const double* __restrict__ M, const VT* __restrict__ x1,
+                                                      const VT* __restrict__ x2, VT* __restrict__ out1,
+                                                      VT* __restrict__ out2, int D, int lane, int i0) {
+  constexpr int U = 16 / RB;
+  double a1[RB], a2[RB];
+  int ii[RB];
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    a1[r] = 0.0;
+    a2[r] = 0.0;
+    const int i = i0 + lane + NUTS_WAVE * r;
+    ii[r] = i < D ? i : D - 1;
+  }
+  int j = 0;
+  for (; j + U <= D; j += U) {
+    double v[U][RB];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double* col = M + (int64_t)(j + u) * D;
+#pragma unroll
+      for (int r = 0; r < RB; ++r) v[u][r] = col[ii[r]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const double y1 = x1[j + u];
+      const double y2 = NX > 1 ? (double)x2[j + u] : 0.0;
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        a1[r] += v[u][r] * y1;
+        if (NX > 1) a2[r] += v[u][r] * y2;
+      }
+    }
+  }
+  for (; j < D; ++j) {
+    const double y1 = x1[j];
+    const double y2 = NX > 1 ? (double)x2[j] : 0.0;
+    const double* col = M + (int64_t)j * D;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const double m = col[ii[r]];
+      a1[r] += m * y1;
+      if (NX > 1) a2[r] += m * y2;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    const int i = i0 + lane + NUTS_WAVE * r;
+    if (i < D) {
+      out1[i] = a1[r];
+      if (NX > 1) out2[i] = a2[r];
+    }
+  }
+}
+template <int NX, class VT>
+__device__ __forceinline__ void dense_matvec_lds(const double* __restrict__ M, const VT* __restrict__ x1,
+                                                 const VT* __restrict__ x2, VT* __restrict__ out1,
+                                                 VT* __restrict__ out2, int D, int lane) {
+  if (D <= NUTS_WAVE) {
+    dense_matvec_lds_rows<NX, 1>(M, x1, x2, out1, out2, D, lane, 0);
+  } else {
+    for (int i0 = 0; i0 < D; i0 += 2 * NUTS_WAVE) dense_matvec_lds_rows<NX, 2>(M, x1, x2, out1, out2, D, lane, i0);
+  }
+}
+
 // p = L⁻ᵀ z and ps = Minv p = L Lᵀ L⁻ᵀ z = L z in one pass over the packed
 // factor F (column-major D×D: L on and below the diagonal, row r of L⁻¹ in
 // column r above it, so F[j][i] (column j, row i < j) = (L⁻¹)[j][i] =
@@ -474,9 +543,12 @@ __device__ __noinline__ void dense_inverse(double* L, int D, int tid) {
   }
 }
 
-template <int METRIC, class GradFn, int TPC = NUTS_WAVE, class VT = double>
+// LV: the chain's vectors are in LDS (one wave per chain and block, see
+// nuts_advance_lds_body) instead of the Q, G, pool and metric buffers.
+template <int METRIC, class GradFn, int TPC = NUTS_WAVE, class VT = double, bool LV = false>
 struct NutsWave {
   static_assert(TPC % NUTS_WAVE == 0 && TPC <= 256, "threads per chain");
+  static_assert(!LV || TPC == NUTS_WAVE, "LDS vectors: one wave per chain");
   static constexpr bool DENSE = METRIC == METRIC_DENSE;
   static_assert(!DENSE || sizeof(VT) == sizeof(double), "dense_e keeps FP64 vectors");
   const NutsParams& P;
@@ -500,17 +572,25 @@ struct NutsWave {
   double v_new = 0;
   bool have_v = false;
 
-  __device__ NutsWave(const NutsParams& P_, const NutsBuffers& B_, ChainState& s_, const GradFn& g_, int c_, int lane_,
-                      int tid_)
+  // lv (LV only): LDS for q, g, minv and the pool block, Dp elements each but the pool's NV Dp
+  __device__ __forceinline__ NutsWave(const NutsParams& P_, const NutsBuffers& B_, ChainState& s_, const GradFn& g_,
+                                      int c_, int lane_, int tid_, VT* lv = nullptr)
       : P(P_), B(B_), s(s_), grad(g_), c(c_), lane(lane_), tid(tid_) {
     D = B.D[c];
     Dp = B.Dp[c];
     uid = B.uid[c];
-    // FP32 vectors use the first half of each buffer at the same element offsets
-    q = reinterpret_cast<VT*>(B.Q) + B.off[c];
-    g = reinterpret_cast<VT*>(B.G) + B.off[c];
-    blk = reinterpret_cast<VT*>(B.pool) + B.off[c] * (int64_t)P.NV;
-    minv = reinterpret_cast<VT*>(B.minv) + B.off[c];
+    if constexpr (LV) {
+      q = lv;
+      g = lv + Dp;
+      minv = lv + 2 * Dp;
+      blk = lv + 3 * Dp;
+    } else {
+      // FP32 vectors use the first half of each buffer at the same element offsets
+      q = reinterpret_cast<VT*>(B.Q) + B.off[c];
+      g = reinterpret_cast<VT*>(B.G) + B.off[c];
+      blk = reinterpret_cast<VT*>(B.pool) + B.off[c] * (int64_t)P.NV;
+      minv = reinterpret_cast<VT*>(B.minv) + B.off[c];
+    }
     if (DENSE) {
       dM = B.dM + B.moff[c];
       dL = B.dL + B.moff[c];
@@ -520,21 +600,32 @@ struct NutsWave {
     }
   }
 
-  // group reduction: every thread gets the same sum (fixed order)
-  static __device__ double gsum(double v) {
-    v = wave_sum(v);
-    if constexpr (TPC == NUTS_WAVE) {
-      return v;
-    } else {
-      __shared__ double red[TPC / NUTS_WAVE];
+  // group reductions: every thread gets the same sums (fixed order); several
+  // sums share one exchange
+  template <int N>
+  static __device__ __forceinline__ void gsum_n(double (&v)[N]) {
+    wave_sum_n(v);
+    if constexpr (TPC > NUTS_WAVE) {
+      __shared__ double red[TPC / NUTS_WAVE][N];
       __syncthreads();
-      if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-      __syncthreads();
-      double r = 0.0;
+      if ((threadIdx.x & 63) == 0) {
 #pragma unroll
-      for (int w = 0; w < TPC / NUTS_WAVE; ++w) r += red[w];
-      return r;
+        for (int k = 0; k < N; ++k) red[threadIdx.x >> 6][k] = v[k];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < N; ++k) {
+        double r = 0.0;
+#pragma unroll
+        for (int w = 0; w < TPC / NUTS_WAVE; ++w) r += red[w][k];
+        v[k] = uniform_value(r);
+      }
     }
+  }
+  static __device__ double gsum(double v) {
+    double a[1] = {v};
+    gsum_n(a);
+    return a[0];
   }
   // global vector writes of the group visible to its other threads
   static __device__ void gsync() {
@@ -592,7 +683,8 @@ struct NutsWave {
   // out = Minv x (dense)
   __device__ void matvec(const VT* x, VT* out) const {
     gsync();
-    dense_matvec<TPC, VT>(dM, x, out, D, tid);
+    if constexpr (LV) dense_matvec_lds<1>(dM, x, (const VT*)nullptr, out, (VT*)nullptr, D, lane);
+    else dense_matvec<TPC, VT>(dM, x, out, D, tid);
     gsync();
   }
   // T = 1/2 p·Minv p; for dense ps must hold Minv p
@@ -636,8 +728,8 @@ struct NutsWave {
     }
     // the reference solves Lᵀ p = z; p = L⁻ᵀ z with the stored inverse is the
     // same vector without D dependent steps, and Minv p = L z comes with it
-    __shared__ double sp[4][NUTS_WAVE * DENSE_RMAX];
-    double* zw = sp[TPC == NUTS_WAVE ? (threadIdx.x >> 6) : 0];
+    __shared__ double sp[LV ? 1 : 4][NUTS_WAVE * DENSE_RMAX];
+    double* zw = sp[TPC == NUTS_WAVE && !LV ? (threadIdx.x >> 6) : 0];
     for (int i = tid; i < D; i += TPC) zw[i] = normal_draw(i); converge();
     advance_normals();
     lsync();
@@ -700,7 +792,8 @@ struct NutsWave {
     for (int i = tid; i < D; i += TPC) p[i] = (double)p[i] - h * (double)gr[i];
     converge();
     gsync();
-    dense_matvec2<TPC, VT>(dM, p, g, vecp(PV_PS), vecp(PV_TMP), D, tid);
+    if constexpr (LV) dense_matvec_lds<2>(dM, p, g, vecp(PV_PS), vecp(PV_TMP), D, lane);
+    else dense_matvec2<TPC, VT>(dM, p, g, vecp(PV_PS), vecp(PV_TMP), D, tid);
     gsync();
   }
   // dense_e: begin_update_p(eps/2) and update_q(eps) of the next leaf, with
@@ -910,6 +1003,19 @@ struct NutsWave {
     return request(PH_LEAF);
   }
 
+  // pass_leaf_merge with its 1 + 6 F sums over the chain's threads
+  template <bool UNIT, int F>
+  __device__ __forceinline__ void leaf_sums(const VT* p, const VT* const (&lb)[3], const VT* const (&le)[3],
+                                            const VT* const (&lr)[3], VT* dp, VT* dr, VT* db, VT* edge, double h,
+                                            double* acc) const {
+    double v[1 + 6 * F];
+    pass_leaf_merge<TPC, UNIT, F>(p, g, minv, lb, le, lr, dp, dr, db, edge, D, tid, h, v);
+    converge();
+    gsum_n(v);
+#pragma unroll
+    for (int k = 0; k < 1 + 6 * F; ++k) acc[k] = v[k];
+  }
+
   // build_tree base case plus the merges that close at this leaf (unit/diag).
   // One pass completes the leapfrog, the kinetic energy and the U-turn sums of
   // up to three of the merges that close here, and stores the leaf's momentum
@@ -947,13 +1053,12 @@ struct NutsWave {
       }
       double acc[1 + 6 * FMAX];
       switch (F) {
-        case 0: pass_leaf_merge<TPC, UNIT, 0>(p, g, minv, lb, le, lr, dp, dr, db, edge, D, tid, hh, acc); break;
-        case 1: pass_leaf_merge<TPC, UNIT, 1>(p, g, minv, lb, le, lr, dp, dr, db, edge, D, tid, hh, acc); break;
-        case 2: pass_leaf_merge<TPC, UNIT, 2>(p, g, minv, lb, le, lr, dp, dr, db, edge, D, tid, hh, acc); break;
-        default: pass_leaf_merge<TPC, UNIT, 3>(p, g, minv, lb, le, lr, dp, dr, db, edge, D, tid, hh, acc); break;
+        case 0: leaf_sums<UNIT, 0>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+        case 1: leaf_sums<UNIT, 1>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+        case 2: leaf_sums<UNIT, 2>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+        default: leaf_sums<UNIT, 3>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
       }
-      converge();
-      double h = 0.5 * gsum(acc[0]) + s.Vz;
+      double h = 0.5 * acc[0] + s.Vz;
       if (isnan(h)) h = __builtin_inf();
       if ((h - s.H0) > P.max_deltaH) s.divergent = 1;
       s.max_abs_dH = fmax(s.max_abs_dH, fabs(h - s.H0));
@@ -974,9 +1079,10 @@ struct NutsWave {
         else { free_slot(s.s_prop); s.s_prop = s.L_prop[k]; }
         double a1, b1, a2, b2, a3, b3;
         if (k < F) {
-          const double* ak = acc + 1 + 6 * k;
-          a1 = gsum(ak[0]); b1 = gsum(ak[1]); a2 = gsum(ak[2]);
-          b2 = gsum(ak[3]); a3 = gsum(ak[4]); b3 = gsum(ak[5]);
+          // selects, not an index: acc stays in registers
+          auto at = [&](int j) { return k == 0 ? acc[1 + j] : (k == 1 ? acc[7 + j] : acc[13 + j]); };
+          a1 = at(0); b1 = at(1); a2 = at(2);
+          b2 = at(3); a3 = at(4); b3 = at(5);
         } else {
           // deeper merges: the separate pass over the stored leaf momentum and
           // the rho merged so far (k >= F >= 1, so the begin is level k-1's)
@@ -984,8 +1090,9 @@ struct NutsWave {
           pass_merge<TPC, METRIC, VT>(Lbeg(k), Lend(k), Lrho(k), Lbeg(k - 1), dp, dr, minv, nullptr, nullptr,
                                       nullptr, nullptr, D, tid, am);
           converge();
-          a1 = gsum(am[0]); b1 = gsum(am[1]); a2 = gsum(am[2]);
-          b2 = gsum(am[3]); a3 = gsum(am[4]); b3 = gsum(am[5]);
+          gsum_n(am);
+          a1 = am[0]; b1 = am[1]; a2 = am[2];
+          b2 = am[3]; a3 = am[4]; b3 = am[5];
         }
         const bool ok = (b1 > 0 && a1 > 0) && (b2 > 0 && a2 > 0) && (b3 > 0 && a3 > 0);
         s.S_logw = lsw_sub;
@@ -1078,8 +1185,9 @@ struct NutsWave {
       double acc[6];
       pass_merge<TPC, METRIC>(lb, le, lr, sb, p, srho, minv, lbs, les, sbs, DENSE ? ps : nullptr, D, tid, acc);
       converge();
-      const double a1 = gsum(acc[0]), b1 = gsum(acc[1]), a2 = gsum(acc[2]);
-      const double b2 = gsum(acc[3]), a3 = gsum(acc[4]), b3 = gsum(acc[5]);
+      gsum_n(acc);
+      const double a1 = acc[0], b1 = acc[1], a2 = acc[2];
+      const double b2 = acc[3], a3 = acc[4], b3 = acc[5];
       const bool ok = (b1 > 0 && a1 > 0) && (b2 > 0 && a2 > 0) && (b3 > 0 && a3 > 0);
       s.S_logw = lsw_sub;
       if (!ok) { free_slot(s.s_prop); trans_end(); return false; }
@@ -1161,8 +1269,9 @@ struct NutsWave {
     double acc[6];
     pass_doubling<TPC, METRIC>(fwd, rho, srho, bb, ff, pfb, pbf, minv, bbs, ffs, psfb, psbf, D, tid, acc);
     converge();
-    const double a1 = gsum(acc[0]), b1 = gsum(acc[1]), a2 = gsum(acc[2]);
-    const double b2 = gsum(acc[3]), a3 = gsum(acc[4]), b3 = gsum(acc[5]);
+    gsum_n(acc);
+    const double a1 = acc[0], b1 = acc[1], a2 = acc[2];
+    const double b2 = acc[3], a3 = acc[4], b3 = acc[5];
     const bool ok = (b1 > 0 && a1 > 0) && (b2 > 0 && a2 > 0) && (b3 > 0 && a3 > 0);
     if (!ok || s.depth >= P.max_depth) trans_end();
     else s.phase = PH_DOUBLING_BEGIN;
@@ -1386,16 +1495,6 @@ struct NutsWave {
   }
 };
 
-// Initial factorisation of every chain's dense inverse metric (one wave per chain).
-__global__ void __launch_bounds__(256) dense_factor_kernel(NutsBuffers B, int* failed) {
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (c >= B.C) return;
-  const int D = B.D[c];
-  const bool ok = NutsWave<METRIC_DENSE, ExternalGrad>::dense_factor(B.dM + B.moff[c], B.dL + B.moff[c], D, lane);
-  if (!ok && lane == 0) atomicAdd(failed, 1);
-}
-
 // Stage ChainState in LDS, run, write back.  TPC == 64: one wave per chain, 4
 // chains per block; TPC == 256: one chain per block, each wave with its own
 // identical copy of the state, wave 0 writes it back.
@@ -1409,6 +1508,8 @@ __device__ __forceinline__ void nuts_advance_body(const NutsParams& P, const Nut
   const int c = TPC == NUTS_WAVE ? blockIdx.x * 4 + w : blockIdx.x;
   const int tid = TPC == NUTS_WAVE ? lane : (int)threadIdx.x;
   if (c >= B.C) return;
+  GradFn f = grad;
+  if constexpr (GradFn::fused) f.bind(c);
   ChainState& s = sst[w];
   {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(B.st + c);
@@ -1420,7 +1521,7 @@ __device__ __forceinline__ void nuts_advance_body(const NutsParams& P, const Nut
   // every wave has its copy of the state before wave 0 may write the new one back
   if (TPC > NUTS_WAVE) __syncthreads();
   if (s.phase < PH_PAUSED) {
-    NutsWave<METRIC, GradFn, TPC, VT> wv(P, B, s, grad, c, lane, tid);
+    NutsWave<METRIC, GradFn, TPC, VT> wv(P, B, s, f, c, lane, tid);
     wv.run();
   }
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -1430,6 +1531,69 @@ __device__ __forceinline__ void nuts_advance_body(const NutsParams& P, const Nut
     const uint32_t* src = reinterpret_cast<const uint32_t*>(&s);
     for (int i = lane; i < (int)(sizeof(ChainState) / 4); i += 64) dst[i] = src[i];
   }
+}
+
+// LDS of one chain's vectors: q, g, minv and the NV pool vectors, Dp elements each
+__host__ __device__ inline size_t nuts_lds_vector_bytes(int Dp, int NV, size_t elem) {
+  return (size_t)(NV + 3) * Dp * elem;
+}
+
+// Fused machine for chains whose vectors fit LDS: one wave per block and chain.
+// The vectors are copied in at the start of a launch and back at its end, and
+// the up to fused_budget gradients between them touch global memory only for
+// the model's data, a dense metric and the draw rows: a leaf of a small chain
+// is a chain of dependent passes over its vectors, each an LDS round trip
+// here and a global one in nuts_advance_body.  Same operations in the same
+// order, so the draws are the same bits.
+template <int METRIC, class GradFn, class VT>
+__device__ __forceinline__ void nuts_advance_lds_body(const NutsParams& P, const NutsBuffers& B, const GradFn& grad) {
+  extern __shared__ __attribute__((aligned(16))) char lds_vectors[];
+  __shared__ ChainState sst;
+  const int lane = threadIdx.x;
+  const int c = blockIdx.x;
+  GradFn f = grad;
+  f.bind(c);
+  {
+    const uint32_t* src = reinterpret_cast<const uint32_t*>(B.st + c);
+    uint32_t* dst = reinterpret_cast<uint32_t*>(&sst);
+    for (int i = lane; i < (int)(sizeof(ChainState) / 4); i += NUTS_WAVE) dst[i] = src[i];
+  }
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  if (sst.phase >= PH_PAUSED) return;  // nothing to do, nothing to write back
+  VT* lv = reinterpret_cast<VT*>(lds_vectors);
+  const int Dp = B.Dp[c];
+  const int64_t off = B.off[c];
+  VT* gq = reinterpret_cast<VT*>(B.Q) + off;
+  VT* gg = reinterpret_cast<VT*>(B.G) + off;
+  VT* gm = reinterpret_cast<VT*>(B.minv) + off;
+  VT* gp = reinterpret_cast<VT*>(B.pool) + off * (int64_t)P.NV;
+  for (int i = lane; i < Dp; i += NUTS_WAVE) {
+    lv[i] = gq[i];
+    lv[Dp + i] = gg[i];
+    lv[2 * Dp + i] = gm[i];
+  }
+#pragma unroll 8
+  for (int i = lane; i < P.NV * Dp; i += NUTS_WAVE) lv[3 * Dp + i] = gp[i];
+  __builtin_amdgcn_wave_barrier();
+  wave_sync();
+  {
+    NutsWave<METRIC, GradFn, NUTS_WAVE, VT, true> wv(P, B, sst, f, c, lane, lane, lv);
+    wv.run();
+  }
+  wave_sync();
+  for (int i = lane; i < Dp; i += NUTS_WAVE) {
+    gq[i] = lv[i];
+    gg[i] = lv[Dp + i];
+    gm[i] = lv[2 * Dp + i];
+  }
+#pragma unroll 8
+  for (int i = lane; i < P.NV * Dp; i += NUTS_WAVE) gp[i] = lv[3 * Dp + i];
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  uint32_t* dst = reinterpret_cast<uint32_t*>(B.st + c);
+  const uint32_t* src = reinterpret_cast<const uint32_t*>(&sst);
+  for (int i = lane; i < (int)(sizeof(ChainState) / 4); i += NUTS_WAVE) dst[i] = src[i];
 }
 
 }  // namespace nutsgpu

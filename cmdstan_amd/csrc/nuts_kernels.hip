@@ -31,6 +31,16 @@ __global__ void __launch_bounds__(256) advance_fused_block_kernel(NutsParams P, 
   nuts_advance_body<METRIC, F, 256, VT>(P, B, f);
 }
 
+// Initial factorisation of every chain's dense inverse metric (one wave per chain).
+__global__ void __launch_bounds__(256) dense_factor_kernel(NutsBuffers B, int* failed) {
+  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  if (c >= B.C) return;
+  const int D = B.D[c];
+  const bool ok = NutsWave<METRIC_DENSE, ExternalGrad>::dense_factor(B.dM + B.moff[c], B.dL + B.moff[c], D, lane);
+  if (!ok && lane == 0) atomicAdd(failed, 1);
+}
+
 template <class F>
 __global__ void __launch_bounds__(256) model_grad_kernel(F f, int C, const int* D, const int64_t* off, const double* Q,
                                                          double* G, double* V, int* need) {
@@ -38,6 +48,7 @@ __global__ void __launch_bounds__(256) model_grad_kernel(F f, int C, const int* 
   const int lane = threadIdx.x & 63;
   if (c >= C) return;
   if (need && !need[c]) return;
+  f.bind(c);
   const double v = f(c, Q + off[c], G + off[c], D[c], lane);
   if (lane == 0) {
     V[c] = v;
@@ -54,6 +65,7 @@ __global__ void __launch_bounds__(256) model_grad_rows_kernel(F f, const int* id
   const int nr = n_dev ? min(n, *n_dev) : n;
   if (r >= nr) return;
   const int c = idx ? idx[r] : r;
+  f.bind(c);
   const double v = f(c, X + (int64_t)r * D, GX + (int64_t)r * D, D, lane);
   if (lane == 0) VX[r] = v;
 }
@@ -67,6 +79,7 @@ __global__ void write_array_kernel(F f, int C, int rows, const int* D, const int
   const double* src = in + in_off[c] + (int64_t)r * (7 + D[c]);
   double* dst = out + out_off[c] + (int64_t)r * (7 + nout[c]);
   for (int i = 0; i < 7; ++i) dst[i] = src[i];
+  f.bind(c);
   f.write_array(c, src + 7, dst + 7);
 }
 
@@ -133,19 +146,9 @@ static bool fused_block_for_metric(int metric, bool vec32, const NutsParams& P, 
   }
 }
 
-#define NUTS_MODEL_SWITCH(kind, md, CALL)                       \
-  switch (kind) {                                               \
-    case MK_BERNOULLI: { BernoulliFn f{{md.data, md.off, md.jac}}; CALL; break; }    \
-    case MK_GAUSS: { GaussFn f{{md.data, md.off, md.jac}}; CALL; break; }            \
-    case MK_EIGHT_SCHOOLS: { EightSchoolsFn f{{md.data, md.off, md.jac}}; CALL; break; } \
-    case MK_HIER_NORMAL_NC: { HierNormalNCFn f{{md.data, md.off, md.jac}}; CALL; break; } \
-    case MK_HIER_LOGISTIC: { HierLogisticFn f{{md.data, md.off, md.jac}}; CALL; break; } \
-    case MK_LOGISTIC: { LogisticFn f{{md.data, md.off, md.jac}}; CALL; break; }      \
-    default: break;                                             \
-  }
-
 void launch_advance_fused(int kind, int metric, bool vec32, const NutsParams& P, const NutsBuffers& B,
                           const ModelDataDev& md, hipStream_t st) {
+  if (launch_advance_fused_lds(kind, metric, vec32, P, B, md, st)) return;
   NUTS_MODEL_SWITCH(kind, md, fused_for_metric(metric, vec32, P, B, f, st));
 }
 

@@ -91,7 +91,7 @@ struct NutsParams {
 
 // Device pointers (kernel argument by value).
 struct NutsBuffers {
-  int C, pad;
+  int C, max_Dp;            // chains, the largest Dp among them
   const int* D;             // [C]
   const int* Dp;            // [C]
   const int64_t* off;       // [C] offset into Q/G/minv (diag)
