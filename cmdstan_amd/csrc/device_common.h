@@ -45,8 +45,10 @@ __device__ __forceinline__ double stream_uniform(uint64_t seed, uint32_t chain, 
   return bits_to_unit(r.x, r.y);
 }
 
-// Box-Muller; element `which` (0: cos, 1: sin) of pair `idx`.
-__device__ __forceinline__ double stream_normal(uint64_t seed, uint32_t chain, uint64_t idx, int which) {
+// Box-Muller; element `which` (0: cos, 1: sin) of pair `idx`.  Out of line: the
+// logarithm and the two angle reductions are 6 KB of instructions, and the
+// state machine draws momenta in two places.
+static __device__ __noinline__ double stream_normal(uint64_t seed, uint32_t chain, uint64_t idx, int which) {
   U4 r = stream_block(seed, chain, STREAM_NORMAL, idx);
   const double u1 = bits_to_unit(r.x, r.y);
   const double u2 = bits_to_unit(r.z, r.w);
@@ -148,8 +150,9 @@ __device__ __forceinline__ double log_sum_exp2(double a, double b) {
   const double inf = __builtin_inf();
   if (a == -inf) return b;
   if (a == inf && b == inf) return inf;
-  if (a > b) return a + log1p_exp(b - a);
-  return b + log1p_exp(a - b);
+  // one exponential and one logarithm in the code: the difference is not positive
+  const double d = a > b ? b - a : a - b;
+  return (a > b ? a : b) + log1p(exp(d));
 }
 
 __device__ __forceinline__ double inv_logit(double x) {

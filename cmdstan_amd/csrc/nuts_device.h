@@ -185,12 +185,12 @@ __device__ __forceinline__ void pass_leaf_merge(const VT* __restrict__ p, const 
 // unit/diag: the leaf's (q, g, p) proposal slot when it is kept, then
 // begin_update_p(eps/2) and update_q(eps) of the next leaf from the closed
 // subtree's end momentum po
-template <int TPC, bool UNIT, bool SLOT, class VT>
+template <int UN, int TPC, bool UNIT, bool SLOT, class VT>
 __device__ __forceinline__ void pass_leaf_next(const VT* __restrict__ po_src, VT* __restrict__ p, VT* __restrict__ q,
                                                const VT* __restrict__ g, const VT* __restrict__ minv,
                                                VT* __restrict__ sq, VT* __restrict__ sg, VT* __restrict__ sp, int D,
                                                int tid, double h, double e) {
-#pragma unroll 4
+#pragma unroll(UN)
   for (int i = tid; i < D; i += TPC) {
     const VT po = po_src[i], qo = q[i], gi = g[i];
     if (SLOT) {
@@ -206,7 +206,7 @@ __device__ __forceinline__ void pass_leaf_next(const VT* __restrict__ po_src, VT
 
 // the three generalized U-turn checks of a merge inside a subtree (rho of the
 // merged subtree written back into srho): partial dot products per thread
-template <int TPC, int METRIC, class VT>
+template <int UN, int TPC, int METRIC, class VT>
 __device__ __forceinline__ void pass_merge(const VT* __restrict__ lb, const VT* __restrict__ le,
                                            const VT* __restrict__ lr, const VT* __restrict__ sb,
                                            const VT* __restrict__ p, VT* __restrict__ srho,
@@ -214,7 +214,7 @@ __device__ __forceinline__ void pass_merge(const VT* __restrict__ lb, const VT* 
                                            const VT* __restrict__ les, const VT* __restrict__ sbs,
                                            const VT* __restrict__ ps, int D, int tid, double* acc) {
   double a1 = 0, b1 = 0, a2 = 0, b2 = 0, a3 = 0, b3 = 0;
-#pragma unroll 4
+#pragma unroll(UN)
   for (int i = tid; i < D; i += TPC) {
     const double l = lr[i], r = srho[i];
     const VT rsv = l + r;
@@ -232,7 +232,7 @@ __device__ __forceinline__ void pass_merge(const VT* __restrict__ lb, const VT* 
 
 // the same checks for the top-level merge of a doubling (rho of the whole
 // trajectory updated in place)
-template <int TPC, int METRIC, class VT>
+template <int UN, int TPC, int METRIC, class VT>
 __device__ __forceinline__ void pass_doubling(bool fwd, VT* __restrict__ rho, const VT* __restrict__ srho,
                                               const VT* __restrict__ bb, const VT* __restrict__ ff,
                                               const VT* __restrict__ pfb, const VT* __restrict__ pbf,
@@ -240,7 +240,7 @@ __device__ __forceinline__ void pass_doubling(bool fwd, VT* __restrict__ rho, co
                                               const VT* __restrict__ ffs, const VT* __restrict__ psfb,
                                               const VT* __restrict__ psbf, int D, int tid, double* acc) {
   double a1 = 0, b1 = 0, a2 = 0, b2 = 0, a3 = 0, b3 = 0;
-#pragma unroll 4
+#pragma unroll(UN)
   for (int i = tid; i < D; i += TPC) {
     const double old = rho[i], nw = srho[i];
     const VT rnv = fwd ? old + nw : nw + old;  // rho_bck + rho_fwd
@@ -550,6 +550,9 @@ struct NutsWave {
   static_assert(TPC % NUTS_WAVE == 0 && TPC <= 256, "threads per chain");
   static_assert(!LV || TPC == NUTS_WAVE, "LDS vectors: one wave per chain");
   static constexpr bool DENSE = METRIC == METRIC_DENSE;
+  // elements per step of the strided passes: loads of several in flight from
+  // global memory, one from LDS (a pass is a few elements per lane there)
+  static constexpr int UN = LV ? 1 : 4;
   static_assert(!DENSE || sizeof(VT) == sizeof(double), "dense_e keeps FP64 vectors");
   const NutsParams& P;
   const NutsBuffers& B;
@@ -692,7 +695,7 @@ struct NutsWave {
     const VT* __restrict__ pr = p;
     const VT* __restrict__ sr = DENSE ? ps : (METRIC == METRIC_UNIT ? p : minv);
     double a = 0;
-#pragma unroll 4
+#pragma unroll(UN)
     for (int i = tid; i < D; i += TPC) {
       const double pv = pr[i];
       a += pv * (DENSE ? (double)sr[i] : (METRIC == METRIC_UNIT ? pv : (double)sr[i] * pv));
@@ -743,7 +746,7 @@ struct NutsWave {
   // the pool vectors never alias each other: restrict lets the unrolled loops
   // issue several independent loads before their stores
   __device__ void copy(VT* __restrict__ dst, const VT* __restrict__ src) const {
-#pragma unroll 4
+#pragma unroll(UN)
     for (int i = tid; i < D; i += TPC) dst[i] = src[i];
     converge();
   }
@@ -764,7 +767,7 @@ struct NutsWave {
     VT* __restrict__ pr = p;
     VT* __restrict__ qr = q;
     const VT* __restrict__ gr = g;
-#pragma unroll 4
+#pragma unroll(UN)
     for (int i = tid; i < D; i += TPC) {
       const VT pi = (double)pr[i] - h * (double)gr[i];
       pr[i] = pi;
@@ -777,7 +780,7 @@ struct NutsWave {
     VT* __restrict__ p = vecp(PV_P);
     const VT* __restrict__ gr = g;
     const double h = 0.5 * e;
-#pragma unroll 4
+#pragma unroll(UN)
     for (int i = tid; i < D; i += TPC) p[i] = (double)p[i] - h * (double)gr[i];
     converge();
     if (DENSE) matvec(p, vecp(PV_PS));
@@ -839,6 +842,13 @@ struct NutsWave {
     s.phase = next;
     s.n_grad++;
     return true;
+  }
+  // the machine goes on at `phase`: steps reached from several places are
+  // phases of their own, so their code is there once (the loop's instructions
+  // are fetched through a 64 KB cache)
+  __device__ bool then(int phase) {
+    s.phase = phase;
+    return false;
   }
   __device__ void stop(int phase) {
     s.phase = phase;
@@ -905,7 +915,7 @@ struct NutsWave {
     const double e = s.nom_eps;
     if (e == 0 || e > 1e7 || isnan(e)) { ss_finish(); return false; }
     s.ss_first = 1;
-    return ss_probe_begin();
+    return then(PH_SS_BEGIN);
   }
   __device__ bool ss_probe() {
     s.Vz = pending_V();
@@ -917,14 +927,14 @@ struct NutsWave {
     if (s.ss_first) {
       s.ss_dir = dH > l08 ? 1 : -1;
       s.ss_first = 0;
-      return ss_probe_begin();
+      return then(PH_SS_BEGIN);
     }
     if ((s.ss_dir == 1) && !(dH > l08)) { ss_finish(); return false; }
     if ((s.ss_dir == -1) && !(dH < l08)) { ss_finish(); return false; }
     s.nom_eps = s.ss_dir == 1 ? s.nom_eps * 2 : s.nom_eps * 0.5;
     if (s.nom_eps > 1e7) { fail(FAIL_STEPSIZE_IMPROPER); return false; }
     if (s.nom_eps == 0) { fail(FAIL_STEPSIZE_ZERO); return false; }
-    return ss_probe_begin();
+    return then(PH_SS_BEGIN);
   }
   __device__ void ss_finish() {
     if (s.ss_return == SS_RET_WINDOW) {
@@ -1028,7 +1038,8 @@ struct NutsWave {
       return leaf_dense();
     } else {
       constexpr bool UNIT = METRIC == METRIC_UNIT;
-      constexpr int FMAX = 3;
+      // LDS vectors: every merge in a pass of its own (one copy of its code)
+      constexpr int FMAX = LV ? 0 : 3;
       const double e = s.dir * s.eps;
       s.Vz = pending_V();
       s.n_leapfrog++;
@@ -1041,9 +1052,9 @@ struct NutsWave {
       VT* edge = s.leaf_idx == 0 ? (s.z_is_fwd ? vecp(PV_PFB) : vecp(PV_PBF)) : nullptr;
       const double hh = 0.5 * e;
       const int F = K < FMAX ? K : FMAX;
-      const VT* lb[FMAX];
-      const VT* le[FMAX];
-      const VT* lr[FMAX];
+      const VT* lb[3] = {};
+      const VT* le[3] = {};
+      const VT* lr[3] = {};
 #pragma unroll
       for (int k = 0; k < FMAX; ++k) {
         const int kk = k < F ? k : 0;
@@ -1051,12 +1062,16 @@ struct NutsWave {
         le[k] = Lend(kk);
         lr[k] = Lrho(kk);
       }
-      double acc[1 + 6 * FMAX];
-      switch (F) {
-        case 0: leaf_sums<UNIT, 0>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
-        case 1: leaf_sums<UNIT, 1>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
-        case 2: leaf_sums<UNIT, 2>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
-        default: leaf_sums<UNIT, 3>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+      double acc[1 + 6 * 3];
+      if constexpr (LV) {
+        leaf_sums<UNIT, 0>(p, lb, le, lr, dp, dr, db, edge, hh, acc);
+      } else {
+        switch (F) {
+          case 0: leaf_sums<UNIT, 0>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+          case 1: leaf_sums<UNIT, 1>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+          case 2: leaf_sums<UNIT, 2>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+          default: leaf_sums<UNIT, 3>(p, lb, le, lr, dp, dr, db, edge, hh, acc); break;
+        }
       }
       double h = 0.5 * acc[0] + s.Vz;
       if (isnan(h)) h = __builtin_inf();
@@ -1066,7 +1081,7 @@ struct NutsWave {
       if (s.H0 - h > 0) s.sum_metro += 1;
       else s.sum_metro += exp(s.H0 - h);
       s.leaf_h = h;
-      if (s.divergent) { trans_end(); return false; }
+      if (s.divergent) return then(PH_TRANS_END);
       s.S_logw = lw;
       s.s_prop = PROP_LEAF;
       int k = 0;
@@ -1078,16 +1093,16 @@ struct NutsWave {
         if (take) free_slot(s.L_prop[k]);
         else { free_slot(s.s_prop); s.s_prop = s.L_prop[k]; }
         double a1, b1, a2, b2, a3, b3;
-        if (k < F) {
+        if (!LV && k < F) {
           // selects, not an index: acc stays in registers
           auto at = [&](int j) { return k == 0 ? acc[1 + j] : (k == 1 ? acc[7 + j] : acc[13 + j]); };
           a1 = at(0); b1 = at(1); a2 = at(2);
           b2 = at(3); a3 = at(4); b3 = at(5);
         } else {
           // deeper merges: the separate pass over the stored leaf momentum and
-          // the rho merged so far (k >= F >= 1, so the begin is level k-1's)
+          // the rho merged so far (the begin is level k-1's, the leaf at level 0)
           double am[6];
-          pass_merge<TPC, METRIC, VT>(Lbeg(k), Lend(k), Lrho(k), Lbeg(k - 1), dp, dr, minv, nullptr, nullptr,
+          pass_merge<UN, TPC, METRIC, VT>(Lbeg(k), Lend(k), Lrho(k), k == 0 ? dp : Lbeg(k - 1), dp, dr, minv, nullptr, nullptr,
                                       nullptr, nullptr, D, tid, am);
           converge();
           gsum_n(am);
@@ -1096,10 +1111,10 @@ struct NutsWave {
         }
         const bool ok = (b1 > 0 && a1 > 0) && (b2 > 0 && a2 > 0) && (b3 > 0 && a3 > 0);
         s.S_logw = lsw_sub;
-        if (!ok) { free_slot(s.s_prop); trans_end(); return false; }
+        if (!ok) { free_slot(s.s_prop); return then(PH_TRANS_END); }
         ++k;
       }
-      if (last) { doubling_end(); return false; }
+      if (last) return then(PH_DOUBLING_END);
       // the closed subtree is the open left sibling at level K: its end and rho
       // are stored there; its begin is level K-1's begin vector (the oldest
       // subtree merged), taken over by a swap, or the leaf itself (K = 0)
@@ -1112,8 +1127,8 @@ struct NutsWave {
       VT* sq = slot >= 0 ? Sq(slot) : nullptr;
       VT* sg = slot >= 0 ? Sg(slot) : nullptr;
       VT* spp = slot >= 0 && P.diag ? Sp(slot) : nullptr;
-      if (sq) pass_leaf_next<TPC, UNIT, true>(dp, p, q, g, minv, sq, sg, spp, D, tid, hh, e);
-      else pass_leaf_next<TPC, UNIT, false>(dp, p, q, g, minv, sq, sg, spp, D, tid, hh, e);
+      if (sq) pass_leaf_next<UN, TPC, UNIT, true>(dp, p, q, g, minv, sq, sg, spp, D, tid, hh, e);
+      else pass_leaf_next<UN, TPC, UNIT, false>(dp, p, q, g, minv, sq, sg, spp, D, tid, hh, e);
       converge();
       if (slot >= 0) {
         s.slot_V[slot] = s.Vz;
@@ -1162,7 +1177,7 @@ struct NutsWave {
       copy(s.z_is_fwd ? vecp(PV_PFB) : vecp(PV_PBF), p);
       copy(s.z_is_fwd ? vecp(PV_PSFB) : vecp(PV_PSBF), ps);
     }
-    if (s.divergent) { trans_end(); return false; }
+    if (s.divergent) return then(PH_TRANS_END);
 
     if (DENSE) copy(srho, p);
     s.S_logw = lw;
@@ -1183,17 +1198,17 @@ struct NutsWave {
       const VT* les = DENSE ? LSend(k) : nullptr;
       const VT* sbs = DENSE ? (k == 0 ? ps : LSbeg(k - 1)) : nullptr;
       double acc[6];
-      pass_merge<TPC, METRIC>(lb, le, lr, sb, p, srho, minv, lbs, les, sbs, DENSE ? ps : nullptr, D, tid, acc);
+      pass_merge<UN, TPC, METRIC>(lb, le, lr, sb, p, srho, minv, lbs, les, sbs, DENSE ? ps : nullptr, D, tid, acc);
       converge();
       gsum_n(acc);
       const double a1 = acc[0], b1 = acc[1], a2 = acc[2];
       const double b2 = acc[3], a3 = acc[4], b3 = acc[5];
       const bool ok = (b1 > 0 && a1 > 0) && (b2 > 0 && a2 > 0) && (b3 > 0 && a3 > 0);
       s.S_logw = lsw_sub;
-      if (!ok) { free_slot(s.s_prop); trans_end(); return false; }
+      if (!ok) { free_slot(s.s_prop); return then(PH_TRANS_END); }
       ++k;
     }
-    if (s.leaf_idx == (1 << s.depth) - 1) { doubling_end(); return false; }
+    if (s.leaf_idx == (1 << s.depth) - 1) return then(PH_DOUBLING_END);
     // the closed subtree becomes the open left sibling at level k
     if (DENSE) {
       copy(Lbeg(k), k == 0 ? p : Lbeg(k - 1));
@@ -1267,14 +1282,13 @@ struct NutsWave {
     const VT* bbs = fwd ? ops : ps;
     const VT* ffs = fwd ? ps : ops;
     double acc[6];
-    pass_doubling<TPC, METRIC>(fwd, rho, srho, bb, ff, pfb, pbf, minv, bbs, ffs, psfb, psbf, D, tid, acc);
+    pass_doubling<UN, TPC, METRIC>(fwd, rho, srho, bb, ff, pfb, pbf, minv, bbs, ffs, psfb, psbf, D, tid, acc);
     converge();
     gsum_n(acc);
     const double a1 = acc[0], b1 = acc[1], a2 = acc[2];
     const double b2 = acc[3], a3 = acc[4], b3 = acc[5];
     const bool ok = (b1 > 0 && a1 > 0) && (b2 > 0 && a2 > 0) && (b3 > 0 && a3 > 0);
-    if (!ok || s.depth >= P.max_depth) trans_end();
-    else s.phase = PH_DOUBLING_BEGIN;
+    s.phase = !ok || s.depth >= P.max_depth ? PH_TRANS_END : PH_DOUBLING_BEGIN;
   }
 
   // window logic of stan::mcmc::windowed_adaptation (unsigned arithmetic)
@@ -1438,10 +1452,13 @@ struct NutsWave {
       case PH_INIT_TRY: return init_try();
       case PH_INIT_CHECK: return init_check();
       case PH_SS_START: return ss_start();
+      case PH_SS_BEGIN: return ss_probe_begin();
       case PH_SS_PROBE: return ss_probe();
       case PH_TRANS_BEGIN: trans_begin(); return false;
       case PH_DOUBLING_BEGIN: return doubling_begin();
       case PH_LEAF: return leaf();
+      case PH_DOUBLING_END: doubling_end(); return false;
+      case PH_TRANS_END: trans_end(); return false;
       default: return false;
     }
   }

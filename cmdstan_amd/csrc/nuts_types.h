@@ -23,10 +23,13 @@ enum Phase : int {
   PH_INIT_TRY = 0,
   PH_INIT_CHECK,
   PH_SS_START,
+  PH_SS_BEGIN,  // the next step-size probe's momentum and half step
   PH_SS_PROBE,
   PH_TRANS_BEGIN,
   PH_DOUBLING_BEGIN,
   PH_LEAF,
+  PH_DOUBLING_END,
+  PH_TRANS_END,
   PH_PAUSED,   // reached the host's iteration target (warmup end)
   PH_DONE,
   PH_FAILED,
