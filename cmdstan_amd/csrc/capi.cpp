@@ -46,16 +46,89 @@ struct HipError : std::runtime_error {
                      std::to_string(__LINE__));                                                         \
   } while (0)
 
+// Device workspace of a handle (a model or a flow), kept from call to call: a
+// call's buffers cost a hipMalloc and a hipFree each (tens of microseconds, and
+// hipFree waits for the device), more than a small call's kernels.  Blocks are
+// the handle's own -- one handle is used by one host thread -- and go with it;
+// at most kKeep bytes stay cached, larger buffers are freed at once.
+class DevPool {
+ public:
+  static constexpr size_t kKeep = (size_t)1 << 30;
+  DevPool() {}
+  DevPool(const DevPool&) = delete;
+  DevPool& operator=(const DevPool&) = delete;
+  ~DevPool() { clear(); }
+  // Around a call's use.  A call that left by an exception may have work in
+  // flight on its buffers: the next one waits for the device first.
+  void begin() {
+    if (open_) (void)hipDeviceSynchronize();
+    open_ = true;
+  }
+  void end() { open_ = false; }
+  void* get(size_t bytes, size_t* got) {
+    size_t best = free_.size();
+    for (size_t i = 0; i < free_.size(); ++i)
+      if (free_[i].n >= bytes && free_[i].n <= 2 * bytes + 65536 && (best == free_.size() || free_[i].n < free_[best].n))
+        best = i;
+    if (best < free_.size()) {
+      void* p = free_[best].p;
+      *got = free_[best].n;
+      held_ -= free_[best].n;
+      free_.erase(free_.begin() + best);
+      return p;
+    }
+    bytes = (bytes + 511) & ~size_t(511);
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      clear();
+      HIPC(hipMalloc(&p, bytes));
+    }
+    *got = bytes;
+    return p;
+  }
+  void put(void* p, size_t n) {
+    if (held_ + n > kKeep) {
+      (void)hipFree(p);
+      return;
+    }
+    free_.push_back({p, n});
+    held_ += n;
+  }
+
+ private:
+  struct Block { void* p; size_t n; };
+  void clear() {
+    for (auto& b : free_) (void)hipFree(b.p);
+    free_.clear();
+    held_ = 0;
+  }
+  std::vector<Block> free_;
+  size_t held_ = 0;
+  bool open_ = false;
+};
+
+// a call's span of the handle's workspace: done() once its work has finished
+struct PoolSpan {
+  DevPool& p;
+  explicit PoolSpan(DevPool& p_) : p(p_) { p.begin(); }
+  void done() { p.end(); }
+};
+
 template <class T>
 struct DevBuf {
   T* p = nullptr;
   size_t n = 0;
   DevBuf() {}
   explicit DevBuf(size_t n_) { alloc(n_); }
+  explicit DevBuf(DevPool* pool) : pool_(pool) {}
+  DevBuf(DevPool* pool, size_t n_) : pool_(pool) { alloc(n_); }
   void alloc(size_t n_) {
     free();
     n = n_;
-    if (n) HIPC(hipMalloc(&p, n * sizeof(T)));
+    if (!n) return;
+    if (pool_) p = static_cast<T*>(pool_->get(n * sizeof(T), &bytes_));
+    else HIPC(hipMalloc(&p, n * sizeof(T)));
   }
   void upload(const T* h, size_t cnt, hipStream_t st = 0) {
     if (cnt) HIPC(hipMemcpyAsync(p, h, cnt * sizeof(T), hipMemcpyHostToDevice, st));
@@ -65,13 +138,18 @@ struct DevBuf {
     upload(h.data(), h.size(), st);
   }
   void free() {
-    if (p) (void)hipFree(p);
+    if (p && pool_) pool_->put(p, bytes_);
+    else if (p) (void)hipFree(p);
     p = nullptr;
     n = 0;
   }
   ~DevBuf() { free(); }
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
+
+ private:
+  DevPool* pool_ = nullptr;
+  size_t bytes_ = 0;
 };
 
 // ------------------------------------------------------------------ data
@@ -123,6 +201,7 @@ struct Dataset {
 };
 
 struct ModelImpl {
+  DevPool ws;  // workspace of this handle's calls
   std::string family;
   int kind = 0;
   std::vector<Dataset> ds;
@@ -191,6 +270,7 @@ struct GlScratch {
   DevBuf<float> qf, r;
   DevBuf<unsigned short> qb, rb;
   DevBuf<double> wg, wlp;
+  explicit GlScratch(DevPool* p) : qf(p), r(p), qb(p), rb(p), wg(p), wlp(p) {}
 };
 bool gl_bf16_enabled(int precision, int D) {
   if (precision != 2 || !gl_large_bf16_ok(D)) return false;
@@ -387,6 +467,9 @@ struct RunSpec {
   bool diagnostics = false;                     // record q, p, g of every saved draw
   bool energy_error = false;                    // record each saved row's max |H - H0|
   int block_mode = -1;                          // lockstep state machine: -1 by dimension, 0 wave, 1 block per chain
+  bool want_last = false;                       // RunResult::z_last
+  // results go here when given (else into RunResult's vectors)
+  double *out_draws = nullptr, *out_minv = nullptr, *out_diag = nullptr, *out_eerr = nullptr;
   int fused_block = -1;                         // fused kernel, block per chain: -1 once few chains remain, 0 never, 1 always
 };
 
@@ -514,7 +597,7 @@ ModelImpl::GlmTune glm_autotune(ModelImpl& M, int C, int precision, hipStream_t 
       if (ms < best.ms) { best.ms = ms; best.path = 2; best.blocks_per_cu = bpc; }
     }
     const GlLargePlan gp = gl_large_plan(N, C, D, num_cus());
-    GlScratch gs;
+    GlScratch gs(&M.ws);
     GlLargeArgs a;
     gl_bind(M, a, gp, gs, precision, st);
     a.C = C; a.Q = Q.p; a.ldq = Dp; a.G = G.p; a.V = V.p;
@@ -575,6 +658,8 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     }
   }
 
+  DevPool* const ws = &M.ws;
+  PoolSpan span(M.ws);
   hipStream_t st;
   HIPC(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   struct StreamGuard { hipStream_t s; ~StreamGuard() { (void)hipStreamDestroy(s); } } sg{st};
@@ -584,20 +669,21 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     ~FlowBind() { if (f) f->bind_stream(old); }
   } fb{R.flow, R.flow ? R.flow->bind_stream(st) : nullptr};
 
-  DevBuf<int> dD(C), dDp(C), dneed(C), dstop(1);
-  DevBuf<int64_t> doffb(C), dmoff(C), ddoff(C), ddsoff(C), dooff(C);
-  DevBuf<uint32_t> duid(C);
-  DevBuf<double> Q(tot), G(tot), V(C), pool((size_t)tot * NV), minv(tot), draws(std::max<int64_t>(dtot, 1));
-  DevBuf<ChainState> dst(C);
-  DevBuf<double> uinit, du, dz;
+  DevBuf<int> dD(ws, C), dDp(ws, C), dneed(ws, C), dstop(ws, 1);
+  DevBuf<int64_t> doffb(ws, C), dmoff(ws, C), ddoff(ws, C), ddsoff(ws, C), dooff(ws, C);
+  DevBuf<uint32_t> duid(ws, C);
+  DevBuf<double> Q(ws, tot), G(ws, tot), V(ws, C), pool(ws, (size_t)tot * NV), minv(ws, tot),
+      draws(ws, std::max<int64_t>(dtot, 1));
+  DevBuf<ChainState> dst(ws, C);
+  DevBuf<double> uinit(ws), du(ws), dz(ws);
   std::vector<int64_t> diag_off(C);
   int64_t diag_tot = 0;
   for (int c = 0; c < C; ++c) {
     diag_off[c] = diag_tot;
     diag_tot += (int64_t)rows * (7 + 3 * D[c]);
   }
-  DevBuf<double> ddiag;
-  DevBuf<int64_t> ddiag_off;
+  DevBuf<double> ddiag(ws);
+  DevBuf<int64_t> ddiag_off(ws);
   if (R.diagnostics) {
     ddiag.alloc(std::max<int64_t>(diag_tot, 1));
     ddiag_off.alloc(C);
@@ -611,41 +697,45 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   HIPC(hipMemsetAsync(pool.p, 0, (size_t)tot * NV * sizeof(double), st));
   HIPC(hipMemsetAsync(dneed.p, 0, C * sizeof(int), st));
   HIPC(hipMemsetAsync(dstop.p, 0, sizeof(int), st));
-  std::vector<double> hm(tot, 1.0);  // diagonal inverse metric as uploaded
-  {
-    if (R.inv_metric && cfg.metric == NUTS_METRIC_DIAG_E) {
-      for (int c = 0; c < C; ++c)
-        for (int i = 0; i < D[c]; ++i) {
-          const double v = R.inv_metric[(size_t)c * D[0] + i];
-          if (!(v > 0) || !std::isfinite(v)) throw std::invalid_argument("inverse metric must be positive and finite");
-          hm[off[c] + i] = v;
-        }
-    }
+  // rows a failed chain does not reach read as zero
+  HIPC(hipMemsetAsync(draws.p, 0, draws.n * sizeof(double), st));
+  if (ddiag.p) HIPC(hipMemsetAsync(ddiag.p, 0, ddiag.n * sizeof(double), st));
+  std::vector<double> hm;  // diagonal inverse metric as given
+  if (R.inv_metric && cfg.metric == NUTS_METRIC_DIAG_E) {
+    hm.assign(tot, 1.0);
+    for (int c = 0; c < C; ++c)
+      for (int i = 0; i < D[c]; ++i) {
+        const double v = R.inv_metric[(size_t)c * D[0] + i];
+        if (!(v > 0) || !std::isfinite(v)) throw std::invalid_argument("inverse metric must be positive and finite");
+        hm[off[c] + i] = v;
+      }
     minv.upload(hm, st);
-    HIPC(hipStreamSynchronize(st));
+  } else {
+    launch_fill(minv.p, tot, 1.0, st);
   }
-  DevBuf<double> dMb, dLb, dWb;
+  int maxD = 0;
+  for (int c = 0; c < C; ++c) maxD = std::max(maxD, D[c]);
+  DevBuf<double> dMb(ws), dLb(ws), dWb(ws);
   if (dense) {
-    // column-major (i, j) at [j*D + i]; the metric file holds a symmetric matrix
-    std::vector<double> hm(mtot, 0.0);
-    for (int c = 0; c < C; ++c) {
-      const int d = D[c];
-      for (int j = 0; j < d; ++j)
-        for (int i = 0; i < d; ++i) {
-          double v = (i == j) ? 1.0 : 0.0;
-          if (R.inv_metric) {
-            v = R.inv_metric[(size_t)c * d * d + (size_t)i * d + j];
-            if (!std::isfinite(v)) throw std::invalid_argument("inverse metric must be finite");
-          }
-          hm[moff[c] + (int64_t)j * d + i] = v;
-        }
-    }
-    dMb.upload(hm, st);
+    dMb.alloc(mtot);
     dLb.alloc(mtot);
-    // the identity start metric is its own Cholesky factor: no factorisation
-    if (!R.inv_metric) dLb.upload(hm.data(), hm.size(), st);
-    HIPC(hipStreamSynchronize(st));
     dWb.alloc(mtot);
+    if (R.inv_metric) {
+      // column-major (i, j) at [j*D + i] from the given rows (one dimension: the
+      // callers check), staged in the Welford buffer
+      DevBuf<int> bad(ws, 1);
+      HIPC(hipMemsetAsync(bad.p, 0, sizeof(int), st));
+      dWb.upload(R.inv_metric, mtot, st);
+      launch_metric_transpose(dWb.p, dMb.p, C, D[0], bad.p, st);
+      int nbad = 0;
+      HIPC(hipMemcpyAsync(&nbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, st));
+      HIPC(hipStreamSynchronize(st));
+      if (nbad) throw std::invalid_argument("inverse metric must be finite");
+    } else {
+      // the identity start metric is its own Cholesky factor: no factorisation
+      launch_metric_identity(dMb.p, dD.p, dmoff.p, C, maxD, st);
+      launch_metric_identity(dLb.p, dD.p, dmoff.p, C, maxD, st);
+    }
     HIPC(hipMemsetAsync(dWb.p, 0, mtot * sizeof(double), st));
   }
   if (R.init) {
@@ -704,13 +794,14 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   B.n_inj_u = R.n_u; B.n_inj_z = R.n_z;
   B.dM = dMb.p; B.dL = dLb.p; B.dW = dWb.p;
   B.diag = ddiag.p; B.diag_off = ddiag_off.p;
-  DevBuf<double> deerr;
+  DevBuf<double> deerr(ws);
   if (R.energy_error && rows > 0) {
     deerr.alloc((size_t)C * rows);
+    HIPC(hipMemsetAsync(deerr.p, 0, deerr.n * sizeof(double), st));
     B.eerr = deerr.p;
   }
   if (dense && R.inv_metric) {
-    DevBuf<int> nfail(1);
+    DevBuf<int> nfail(ws, 1);
     HIPC(hipMemsetAsync(nfail.p, 0, sizeof(int), st));
     launch_dense_factor(B, nfail.p, st);
     int nf = 0;
@@ -763,20 +854,22 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     throw std::invalid_argument("precision=bf16 applies to the logistic regression design matrix only");
   if (vec32) {
     // same element offsets, FP32 values in the first half of each buffer
-    std::vector<float> hf(hm.begin(), hm.end());
-    HIPC(hipMemcpyAsync(minv.p, hf.data(), hf.size() * sizeof(float), hipMemcpyHostToDevice, st));
-    HIPC(hipStreamSynchronize(st));
+    if (hm.empty()) {
+      launch_fill(reinterpret_cast<float*>(minv.p), tot, 1.0f, st);
+    } else {
+      std::vector<float> hf(hm.begin(), hm.end());
+      HIPC(hipMemcpyAsync(minv.p, hf.data(), hf.size() * sizeof(float), hipMemcpyHostToDevice, st));
+      HIPC(hipStreamSynchronize(st));
+    }
   }
 
-  DevBuf<double> work;
-  DevBuf<int> act_idx, n_act;
+  DevBuf<double> work(ws);
+  DevBuf<int> act_idx(ws), n_act(ws);
   const void* xlow = nullptr;
   const unsigned short* xbf = nullptr;  // BF16 terms of X (path 2)
   GlmArgs ga;
   GlmPlan gplan;
   // large chains: one 256-thread block per chain for the state machine
-  int maxD = 0;
-  for (int c = 0; c < C; ++c) maxD = std::max(maxD, D[c]);
   const char* bpc = std::getenv("CMDSTAN_AMD_BLOCK_PER_CHAIN");
   bool block_per_chain =
       !fused && (R.block_mode >= 0 ? R.block_mode == 1 : (bpc ? std::atoi(bpc) != 0 : maxD >= 512));
@@ -800,7 +893,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     throw std::invalid_argument("this model has no block-per-chain fused kernel");
   const char* fbc = std::getenv("CMDSTAN_AMD_FUSED_BLOCK_CHAINS");  // threshold override (chains still running)
   const int fused_block_chains = fbc ? std::atoi(fbc) : 2 * num_cus();
-  DevBuf<double> hlwork;
+  DevBuf<double> hlwork(ws);
   HlArgs hla{};
   if (hl_ok && !fused) {
     const Dataset& hd = M.ds[R.first_dataset];
@@ -817,7 +910,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     }
   }
   const int hl_groups = hl_ok ? M.ds[R.first_dataset].groups : 0;
-  DevBuf<double> fX, fGX, fVX, fLD;
+  DevBuf<double> fX(ws), fGX(ws), fVX(ws), fLD(ws);
   if (R.flow) {
     if (!act_idx.p) {
       act_idx.alloc(C);
@@ -830,7 +923,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   }
   // flow: the GLM gradients read the packed rows x = T(z) and write packed
   // rows; the identity list maps position r to row r
-  DevBuf<int> ident;
+  DevBuf<int> ident(ws);
   if (R.flow && (glm_ok || gl_ok || gw_ok)) {
     std::vector<int> h(C);
     std::iota(h.begin(), h.end(), 0);
@@ -842,7 +935,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   }
   GlLargeArgs gla;
   GlLargePlan glp;
-  GlScratch gls;
+  GlScratch gls(&M.ws);
   if (!fused && gl_ok) {
     act_idx.alloc(C);
     n_act.alloc(1);
@@ -919,7 +1012,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   // grow through early warmup) weighs on both modes alike
   int tune_left = tune_threads ? 4 : 0;
   double tune_s[2] = {0, 0};
-  DevBuf<long long> tally;
+  DevBuf<long long> tally(ws);
   if (!fused) {
     for (int k = 0; k < kCheck; ++k) {
       HIPC(hipEventCreate(&ev.a[k]));
@@ -935,7 +1028,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   const char* lim = std::getenv("CMDSTAN_AMD_MAX_SECONDS");
   const double max_seconds = lim ? std::atof(lim) : 3600.0;
   const auto t_begin = std::chrono::steady_clock::now();
-  DevBuf<int> miter(1);
+  DevBuf<int> miter(ws, 1);
   int min_it = 0;
   int next_report = cfg.refresh > 0 ? cfg.refresh : 0;
   // One check interval of lockstep work: kCheck x (advance, gradient).  With
@@ -1123,38 +1216,55 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
 
   res.st.resize(C);
   HIPC(hipMemcpyAsync(res.st.data(), dst.p, C * sizeof(ChainState), hipMemcpyDeviceToHost, st));
-  if (dense) {
-    std::vector<double> hm(mtot);
-    HIPC(hipMemcpyAsync(hm.data(), dMb.p, mtot * sizeof(double), hipMemcpyDeviceToHost, st));
+  // results straight into the caller's arrays where it gave them
+  auto result = [&](double* user, std::vector<double>& own, int64_t n) {
+    if (user) return user;
+    own.resize(n);
+    return own.data();
+  };
+  {
+    DevBuf<double> packed(ws);
+    const double* src = packed.p;
+    int64_t n = 0;
+    if (dense) {
+      n = mtot;
+      bool uni = true;
+      for (int c = 1; c < C; ++c) uni = uni && D[c] == D[0];
+      for (int c = 0; c < (uni ? 1 : C); ++c)  // rows of the metric, in the Welford buffer (its run is over)
+        launch_metric_transpose(dMb.p + moff[c], dWb.p + moff[c], uni ? C : 1, D[c], nullptr, st);
+      src = dWb.p;
+    } else {
+      std::vector<int64_t> to(C);
+      for (int c = 0; c < C; ++c) { to[c] = n; n += D[c]; }
+      DevBuf<int64_t> dto(ws, C);
+      dto.upload(to, st);
+      packed.alloc(n);
+      launch_pack_rows(minv.p, vec32, doffb.p, dD.p, dto.p, C, packed.p, st);
+      src = packed.p;
+      HIPC(hipStreamSynchronize(st));
+    }
+    HIPC(hipMemcpyAsync(result(R.out_minv, res.minv, n), src, n * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
-    for (int c = 0; c < C; ++c)
-      for (int i = 0; i < D[c]; ++i)
-        for (int j = 0; j < D[c]; ++j) res.minv.push_back(hm[moff[c] + (int64_t)j * D[c] + i]);
-  } else if (vec32) {
-    std::vector<float> hf(tot);
-    HIPC(hipMemcpyAsync(hf.data(), minv.p, tot * sizeof(float), hipMemcpyDeviceToHost, st));
-    HIPC(hipStreamSynchronize(st));
-    for (int c = 0; c < C; ++c) for (int i = 0; i < D[c]; ++i) res.minv.push_back(hf[off[c] + i]);
-  } else {
-    std::vector<double> hmo(tot);
-    HIPC(hipMemcpyAsync(hmo.data(), minv.p, tot * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPC(hipStreamSynchronize(st));
-    for (int c = 0; c < C; ++c) for (int i = 0; i < D[c]; ++i) res.minv.push_back(hmo[off[c] + i]);
   }
-  if (rows > 0 && (msp < 0 || msp >= D[0])) {
+  if (R.want_last && rows > 0 && (msp < 0 || msp >= D[0])) {
     bool uni = true;
     for (int c = 1; c < C; ++c) uni = uni && D[c] == D[0];
     if (uni) {
       // last saved row of each chain, unconstrained (the state a later run resumes from)
       const int ld = 7 + nsave_of(D[0]);
-      std::vector<double> last((size_t)C * ld);
-      for (int c = 0; c < C; ++c)
-        HIPC(hipMemcpyAsync(last.data() + (size_t)c * ld, draws.p + doff[c] + (int64_t)(rows - 1) * ld,
-                            ld * sizeof(double), hipMemcpyDeviceToHost, st));
-      HIPC(hipStreamSynchronize(st));
+      std::vector<int64_t> from(C), to(C);
+      for (int c = 0; c < C; ++c) {
+        from[c] = doff[c] + (int64_t)(rows - 1) * ld + 7;
+        to[c] = (int64_t)c * D[0];
+      }
+      DevBuf<int64_t> dfrom(ws, C), dto(ws, C);
+      dfrom.upload(from, st);
+      dto.upload(to, st);
+      DevBuf<double> last(ws, (size_t)C * D[0]);
+      launch_pack_rows(draws.p, false, dfrom.p, dD.p, dto.p, C, last.p, st);
       res.z_last.resize((size_t)C * D[0]);
-      for (int c = 0; c < C; ++c)
-        for (int i = 0; i < D[0]; ++i) res.z_last[(size_t)c * D[0] + i] = last[(size_t)c * ld + 7 + i];
+      HIPC(hipMemcpyAsync(res.z_last.data(), last.p, res.z_last.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+      HIPC(hipStreamSynchronize(st));
     }
   }
   if (R.flow) {
@@ -1172,11 +1282,11 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     std::vector<double> un(dtot);
     HIPC(hipMemcpyAsync(un.data(), draws.p, dtot * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
-    res.draws.assign(otot, 0.0);
+    double* const od = result(R.out_draws, res.draws, otot);
     std::vector<double> q((size_t)rows * D[0]), o((size_t)rows * nout[0]);
     for (int c = 0; c < C; ++c) {
       const double* src = un.data() + doff[c];
-      double* dst = res.draws.data() + ooff[c];
+      double* dst = od + ooff[c];
       for (int r = 0; r < rows; ++r)
         for (int i = 0; i < D[c]; ++i) q[(size_t)r * D[c] + i] = src[(int64_t)r * (7 + D[c]) + 7 + i];
       if (M.pl.write_array) {
@@ -1192,30 +1302,29 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     res.draw_off = ooff;
     for (int c = 0; c < C; ++c) res.cols.push_back(7 + nout[c]);
   } else if (R.constrain && msp < 0) {
-    DevBuf<double> out(std::max<int64_t>(otot, 1));
-    DevBuf<int> dn(C);
+    DevBuf<double> out(ws, std::max<int64_t>(otot, 1));
+    DevBuf<int> dn(ws, C);
     dn.upload(nout, st);
     launch_write_array(M.kind, C, rows, dD.p, ddoff.p, dooff.p, dn.p, draws.p, out.p, md, st);
-    res.draws.resize(otot);
-    HIPC(hipMemcpyAsync(res.draws.data(), out.p, otot * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPC(hipMemcpyAsync(result(R.out_draws, res.draws, otot), out.p, otot * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPC(hipStreamSynchronize(st));  // before `out` goes back to the workspace
     res.draw_off = ooff;
     for (int c = 0; c < C; ++c) res.cols.push_back(7 + nout[c]);
   } else {
-    res.draws.resize(dtot);
-    HIPC(hipMemcpyAsync(res.draws.data(), draws.p, dtot * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPC(hipMemcpyAsync(result(R.out_draws, res.draws, dtot), draws.p, dtot * sizeof(double), hipMemcpyDeviceToHost, st));
     res.draw_off = doff;
     for (int c = 0; c < C; ++c) res.cols.push_back(7 + nsave_of(D[c]));
   }
   if (R.diagnostics) {
-    res.diag.resize(diag_tot);
-    HIPC(hipMemcpyAsync(res.diag.data(), ddiag.p, diag_tot * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPC(hipMemcpyAsync(result(R.out_diag, res.diag, diag_tot), ddiag.p, diag_tot * sizeof(double), hipMemcpyDeviceToHost, st));
   }
   if (B.eerr) {
-    res.eerr.resize((size_t)C * rows);
-    HIPC(hipMemcpyAsync(res.eerr.data(), deerr.p, res.eerr.size() * sizeof(double), hipMemcpyDeviceToHost, st));
+    HIPC(hipMemcpyAsync(result(R.out_eerr, res.eerr, (int64_t)C * rows), deerr.p, (size_t)C * rows * sizeof(double),
+                        hipMemcpyDeviceToHost, st));
   }
   HIPC(hipStreamSynchronize(st));
   HIPC(hipGetLastError());
+  span.done();
   return res;
 }
 
@@ -1281,6 +1390,8 @@ RunResult run_with_flow(ModelImpl& M, const RunSpec& R0, FlowReport& rep) {
   A.cfg.flow = 0; A.cfg.save_warmup = 1; A.cfg.thin = 1; A.cfg.num_samples = P; A.cfg.max_saved_params = -1;
   A.constrain = false;
   A.energy_error = false;
+  A.want_last = true;
+  A.out_draws = A.out_minv = A.out_diag = A.out_eerr = nullptr;
   RunResult ra = run_batch(M, A);
   add_counts(ra);
   for (int c = 0; c < C; ++c) {
@@ -1337,6 +1448,8 @@ RunResult run_with_flow(ModelImpl& M, const RunSpec& R0, FlowReport& rep) {
   Bs.cfg.thin = 1; Bs.cfg.max_saved_params = -1;
   Bs.init = z0.data(); Bs.inv_metric = nullptr; Bs.flow = &net; Bs.constrain = false;
   Bs.energy_error = false;
+  Bs.want_last = true;
+  Bs.out_draws = Bs.out_minv = Bs.out_diag = Bs.out_eerr = nullptr;
   RunResult rb = run_batch(M, Bs);
   add_counts(rb);
   const bool flow_ok = all_done(rb);
@@ -1557,92 +1670,6 @@ int nuts_model_unconstrained_name(const nuts_model* m, int dataset, int i, char*
   return guarded([&]() { return copy_name(m->impl.ds.at(dataset).unames.at(i), buf, buflen); });
 }
 
-static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n_points, int jacobian,
-                              int precision, double* lp, double* grad) {
-  return guarded([&]() {
-    ModelImpl& M = m->impl;
-    if (dataset < 0 || dataset >= (int)M.ds.size()) throw std::out_of_range("dataset index");
-    if (n_points < 1) return NUTS_OK;
-    const int D = M.ds[dataset].D;
-    const int Dp = (D + 15) / 16 * 16;
-    const int C = n_points;
-    std::vector<int> Dv(C, D);
-    std::vector<int64_t> off(C), dso(C, M.ds_off[dataset]);
-    std::vector<double> hq((size_t)C * Dp, 0.0);
-    for (int c = 0; c < C; ++c) {
-      off[c] = (int64_t)c * Dp;
-      for (int i = 0; i < D; ++i) hq[(size_t)c * Dp + i] = q[(size_t)c * D + i];
-    }
-    DevBuf<int> dD(C);
-    DevBuf<int64_t> doff(C), ddso(C);
-    DevBuf<double> Q(hq.size()), G(hq.size()), V(C);
-    dD.upload(Dv); doff.upload(off); ddso.upload(dso); Q.upload(hq);
-    ModelDataDev md{M.d_data.p, ddso.p, jacobian ? 1.0 : 0.0};
-    if (precision != 0 && !((M.glm || M.glm_large) && dataset == 0))
-      throw std::invalid_argument("reduced precision is available for the batched logistic regression only");
-    if (M.plugin) {
-      if (M.pl.log_prob_grad(M.pl.user, Q.p, Dp, nullptr, nullptr, C, jacobian ? 1 : 0, G.p, V.p, nullptr))
-        throw std::runtime_error("plugin log_prob_grad failed");
-      HIPC(hipDeviceSynchronize());
-    } else if (M.glm_large && dataset == 0 && precision != 0) {
-      const GlLargePlan gp = gl_large_plan(M.glmN, C, D, num_cus());
-      GlScratch gs;
-      GlLargeArgs a;
-      gl_bind(M, a, gp, gs, precision, 0);
-      a.C = C; a.Q = Q.p; a.ldq = Dp; a.G = G.p; a.V = V.p;
-      gl_large_grad(a, gp, M.low_x(precision, 0), precision, 0);
-      HIPC(hipDeviceSynchronize());
-    } else if (M.glm_wide && dataset == 0) {
-      const GlmWidePlan gp = glm_wide_plan(M.glmN, C, D, num_cus());
-      DevBuf<double> work(gp.work_doubles);
-      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, C, 0, M.glm_s2inv, Q.p, Dp, G.p, V.p, work.p};
-      if (glm_grad_wide_f64(ga, gp, 0)) throw std::runtime_error("GLM kernel: unsupported D");
-      HIPC(hipDeviceSynchronize());
-    } else if (M.glm && dataset == 0) {
-      // reduced precision: the kernel the sampler's autotuner picks for this many points
-      const ModelImpl::GlmTune tn = precision != 0 ? glm_autotune(M, C, precision, 0) : ModelImpl::GlmTune{};
-      if (tn.path == 1) {
-        const GlLargePlan gp = gl_large_plan(M.glmN, C, D, num_cus());
-        GlScratch gs;
-        GlLargeArgs a;
-        gl_bind(M, a, gp, gs, precision, 0);
-        a.C = C; a.Q = Q.p; a.ldq = Dp; a.G = G.p; a.V = V.p;
-        gl_large_grad(a, gp, M.low_x(precision, 0), precision, 0);
-      } else {
-        const GlmPlan gp = glm_mfma_plan(M.glmN, C, D, num_cus());
-        DevBuf<double> work(gp.work_doubles);
-        GlmArgs ga{M.d_X, M.d_y, M.glmN, D, C, gp.rows_per_chunk, M.glm_s2inv, Q.p, Dp, G.p, V.p, work.p};
-        const int rcg = precision == 0 ? glm_grad_mfma_f64(ga, gp, 0)
-                        : tn.path == 2 ? glm_grad_mfma_bf16(ga, gp, M.bf16_x(precision, 0), precision, 0)
-                                       : glm_grad_mfma_f32(ga, gp, M.low_x(precision, 0), precision, kF32Layout, 0);
-        if (rcg) throw std::runtime_error("GLM kernel: unsupported D");
-      }
-      HIPC(hipDeviceSynchronize());
-    } else if (M.kind == MK_HIER_LOGISTIC) {
-      // the sampler's batched group kernel (lane = point)
-      const Dataset& hd = M.ds[dataset];
-      DevBuf<double> work(hl_work_doubles(hd.groups, hd.group_size, C));
-      HlArgs a{};
-      a.block = M.d_data.p + M.ds_off[dataset];
-      a.Q = Q.p; a.ldq = Dp; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = C;
-      a.Gout = G.p; a.ldg = Dp; a.Vout = V.p; a.work = work.p; a.jac = jacobian ? 1.0 : 0.0;
-      hl_grad_launch(a, hd.groups, 0);
-      HIPC(hipDeviceSynchronize());
-    } else {
-      launch_model_grad(M.kind, C, dD.p, doff.p, Q.p, G.p, V.p, nullptr, md, 0);
-    }
-    HIPC(hipGetLastError());
-    std::vector<double> hg(hq.size()), hv(C);
-    HIPC(hipMemcpy(hg.data(), G.p, hg.size() * sizeof(double), hipMemcpyDeviceToHost));
-    HIPC(hipMemcpy(hv.data(), V.p, C * sizeof(double), hipMemcpyDeviceToHost));
-    for (int c = 0; c < C; ++c) {
-      lp[c] = -hv[c];
-      for (int i = 0; i < D; ++i) grad[(size_t)c * D + i] = -hg[(size_t)c * Dp + i];
-    }
-    return NUTS_OK;
-  });
-}
-
 // stan::model::model_base::transform_inits for the registered families: the
 // named constrained values of `inits` to the unconstrained vector (D values);
 // parameters absent from `inits` are NaN (drawn at random by initialize).
@@ -1699,16 +1726,6 @@ int nuts_model_transform_inits(nuts_model* m, int dataset, const nuts_data* init
   });
 }
 
-int nuts_log_prob_grad(nuts_model* m, int dataset, const double* q, int n_points, int jacobian, double* lp,
-                       double* grad) {
-  return log_prob_grad_impl(m, dataset, q, n_points, jacobian, 0, lp, grad);
-}
-
-int nuts_log_prob_grad_precision(nuts_model* m, int dataset, const double* q, int n_points, int jacobian,
-                                 int precision, double* lp, double* grad) {
-  return log_prob_grad_impl(m, dataset, q, n_points, jacobian, precision, lp, grad);
-}
-
 void nuts_config_default(nuts_config* c) {
   std::memset(c, 0, sizeof(*c));
   c->num_samples = 1000; c->num_warmup = 1000; c->save_warmup = 0; c->thin = 1;
@@ -1737,6 +1754,10 @@ int nuts_sample(nuts_model* m, const nuts_config* cfg, const double* init, const
     R.inv_metric = inv_metric;
     R.diagnostics = out && out->diagnostics;
     R.energy_error = out && out->energy_error;
+    if (out) {
+      R.out_draws = out->draws; R.out_minv = out->inv_metric; R.out_diag = out->diagnostics;
+      R.out_eerr = out->energy_error;
+    }
     if (R.diagnostics && cfg->flow) throw std::invalid_argument("diagnostic rows are not available with the flow");
     if (init || inv_metric) {
       // per-chain arrays index with a uniform stride: require one dimension
@@ -1747,7 +1768,8 @@ int nuts_sample(nuts_model* m, const nuts_config* cfg, const double* init, const
     RunResult r = cfg->flow ? run_with_flow(m->impl, R, rep) : run_batch(m->impl, R);
     const int C = (int)r.st.size();
     if (out) {
-      if (out->draws) std::memcpy(out->draws, r.draws.data(), r.draws.size() * sizeof(double));
+      // vectors that are not empty: results of an earlier phase of a flow run
+      if (out->draws && !r.draws.empty()) std::memcpy(out->draws, r.draws.data(), r.draws.size() * sizeof(double));
       int64_t moff = 0;
       for (int c = 0; c < C; ++c) {
         const ChainState& s = r.st[c];
@@ -1756,9 +1778,8 @@ int nuts_sample(nuts_model* m, const nuts_config* cfg, const double* init, const
         if (out->grad_evals) out->grad_evals[c] = cfg->flow ? rep.ngrad[c] : s.n_grad;
         if (out->status) out->status[c] = s.phase == PH_DONE ? 0 : (s.failure ? s.failure : -1);
       }
-      if (out->inv_metric) std::memcpy(out->inv_metric, r.minv.data(), r.minv.size() * sizeof(double));
-      if (out->diagnostics) std::memcpy(out->diagnostics, r.diag.data(), r.diag.size() * sizeof(double));
-      if (out->energy_error) std::memcpy(out->energy_error, r.eerr.data(), r.eerr.size() * sizeof(double));
+      if (out->inv_metric && !r.minv.empty())
+        std::memcpy(out->inv_metric, r.minv.data(), r.minv.size() * sizeof(double));
       if (out->init_rejections)
         for (int c = 0; c < C; ++c) {
           out->init_rejections[2 * c] = cfg->flow ? rep.rej_lp[c] : r.st[c].init_rej_lp;
@@ -1900,6 +1921,92 @@ __global__ void noalloc_finish(const double* V, double* lp, double* grad, int n,
 
 }  // namespace
 
+// The host entry: points up, the same kernels as the allocation-free entry
+// (rows of D doubles), results down, on the handle's workspace.
+static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n_points, int jacobian,
+                              int precision, double* lp, double* grad) {
+  return guarded([&]() {
+    ModelImpl& M = m->impl;
+    if (dataset < 0 || dataset >= (int)M.ds.size()) throw std::out_of_range("dataset index");
+    if (n_points < 1) return NUTS_OK;
+    const int D = M.ds[dataset].D, C = n_points;
+    if (precision != 0 && !((M.glm || M.glm_large) && dataset == 0))
+      throw std::invalid_argument("reduced precision is available for the batched logistic regression only");
+    PoolSpan span(M.ws);
+    DevPool* const ws = &M.ws;
+    DevBuf<double> Q(ws, (size_t)C * D), G(ws, (size_t)C * D), V(ws, C), L(ws, C), work(ws);
+    DevBuf<int> dD(ws);
+    DevBuf<int64_t> doff(ws), ddso(ws);
+    GlScratch gs(ws);
+    Q.upload(q, (size_t)C * D);
+    if (M.plugin) {
+      if (M.pl.log_prob_grad(M.pl.user, Q.p, D, nullptr, nullptr, C, jacobian ? 1 : 0, G.p, V.p, nullptr))
+        throw std::runtime_error("plugin log_prob_grad failed");
+      HIPC(hipDeviceSynchronize());  // whatever stream the callback worked on
+    } else if ((M.glm || (M.glm_large && (precision != 0 || M.glm_wide))) && dataset == 0) {
+      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, C, 0, M.glm_s2inv, Q.p, D, G.p, V.p, nullptr};
+      // reduced precision: the kernel the sampler's autotuner picks for this many points
+      const ModelImpl::GlmTune tn = M.glm && precision != 0 ? glm_autotune(M, C, precision, 0) : ModelImpl::GlmTune{};
+      int rcg = 0;
+      if (precision != 0 && (M.glm_large || tn.path == 1)) {
+        const GlLargePlan gp = gl_large_plan(M.glmN, C, D, num_cus());
+        GlLargeArgs a;
+        gl_bind(M, a, gp, gs, precision, 0);
+        a.C = C; a.Q = Q.p; a.ldq = D; a.G = G.p; a.V = V.p;
+        gl_large_grad(a, gp, M.low_x(precision, 0), precision, 0);
+      } else if (M.glm_wide) {
+        const GlmWidePlan gp = glm_wide_plan(M.glmN, C, D, num_cus());
+        work.alloc(gp.work_doubles);
+        ga.work = work.p;
+        rcg = glm_grad_wide_f64(ga, gp, 0);
+      } else {
+        const GlmPlan gp = glm_mfma_plan(M.glmN, C, D, num_cus());
+        work.alloc(gp.work_doubles);
+        ga.work = work.p;
+        ga.rows_per_chunk = gp.rows_per_chunk;
+        rcg = precision == 0 ? glm_grad_mfma_f64(ga, gp, 0)
+              : tn.path == 2 ? glm_grad_mfma_bf16(ga, gp, M.bf16_x(precision, 0), precision, 0)
+                             : glm_grad_mfma_f32(ga, gp, M.low_x(precision, 0), precision, kF32Layout, 0);
+      }
+      if (rcg) throw std::runtime_error("GLM kernel: unsupported D");
+    } else if (M.kind == MK_HIER_LOGISTIC) {
+      // the sampler's batched group kernel (lane = point)
+      const Dataset& hd = M.ds[dataset];
+      work.alloc(hl_work_doubles(hd.groups, hd.group_size, C));
+      HlArgs a{};
+      a.block = M.d_data.p + M.ds_off[dataset];
+      a.Q = Q.p; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = C;
+      a.Gout = G.p; a.ldg = D; a.Vout = V.p; a.work = work.p; a.jac = jacobian ? 1.0 : 0.0;
+      hl_grad_launch(a, hd.groups, 0);
+    } else {
+      dD.alloc(C);
+      doff.alloc(C);
+      ddso.alloc(C);
+      hipLaunchKernelGGL(noalloc_tables, dim3((C + 255) / 256), dim3(256), 0, 0, dD.p, doff.p, ddso.p, C, D,
+                         M.ds_off[dataset]);
+      ModelDataDev md{M.d_data.p, ddso.p, jacobian ? 1.0 : 0.0};
+      launch_model_grad(M.kind, C, dD.p, doff.p, Q.p, G.p, V.p, nullptr, md, 0);
+    }
+    const int64_t tot = std::max<int64_t>((int64_t)C * D, C);
+    hipLaunchKernelGGL(noalloc_finish, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, 0, V.p, L.p, G.p, C, D);
+    HIPC(hipGetLastError());
+    HIPC(hipMemcpy(grad, G.p, (size_t)C * D * sizeof(double), hipMemcpyDeviceToHost));
+    HIPC(hipMemcpy(lp, L.p, C * sizeof(double), hipMemcpyDeviceToHost));
+    span.done();
+    return NUTS_OK;
+  });
+}
+
+extern "C" int nuts_log_prob_grad(nuts_model* m, int dataset, const double* q, int n_points, int jacobian, double* lp,
+                                  double* grad) {
+  return log_prob_grad_impl(m, dataset, q, n_points, jacobian, 0, lp, grad);
+}
+
+extern "C" int nuts_log_prob_grad_precision(nuts_model* m, int dataset, const double* q, int n_points, int jacobian,
+                                            int precision, double* lp, double* grad) {
+  return log_prob_grad_impl(m, dataset, q, n_points, jacobian, precision, lp, grad);
+}
+
 extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const double* d_q, int n_points, int jacobian,
                                           double* d_lp, double* d_grad, void* stream) {
   return guarded([&]() {
@@ -1969,6 +2076,7 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
 
 // ------------------------------------------------------------------ flow
 struct nuts_flow {
+  DevPool ws;  // workspace of this handle's calls
   std::unique_ptr<FlowNet> net;
 };
 
@@ -2012,13 +2120,15 @@ int nuts_flow_forward(nuts_flow* f, const double* z, int n, double* x, double* l
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
-    DevBuf<double> dz((size_t)n * D), dx((size_t)n * D), dl(n);
+    PoolSpan span(f->ws);
+    DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dl(&f->ws, n);
     dz.upload(z, (size_t)n * D, st);
     f->net->forward(dz.p, D, nullptr, nullptr, n, dx.p, dl.p);
     HIPC(hipMemcpyAsync(x, dx.p, (size_t)n * D * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipMemcpyAsync(logdet, dl.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
     f->net->check_barriers();
+    span.done();
     return NUTS_OK;
   });
 }
@@ -2028,12 +2138,14 @@ int nuts_flow_inverse(nuts_flow* f, const double* x, int n, double* z, double* l
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
-    DevBuf<double> dz((size_t)n * D), dx((size_t)n * D), dl(n);
+    PoolSpan span(f->ws);
+    DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dl(&f->ws, n);
     dx.upload(x, (size_t)n * D, st);
     f->net->inverse(dx.p, n, dz.p, dl.p);
     HIPC(hipMemcpyAsync(z, dz.p, (size_t)n * D * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipMemcpyAsync(logdet, dl.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
+    span.done();
     return NUTS_OK;
   });
 }
@@ -2043,7 +2155,8 @@ int nuts_flow_pullback_grad(nuts_flow* f, const double* z, const double* gx, int
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
-    DevBuf<double> dz((size_t)n * D), dx((size_t)n * D), dgx((size_t)n * D), dgz((size_t)n * D), dl(n), dvx(n), dv(n);
+    PoolSpan span(f->ws);
+    DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dgx(&f->ws, (size_t)n * D), dgz(&f->ws, (size_t)n * D), dl(&f->ws, n), dvx(&f->ws, n), dv(&f->ws, n);
     dz.upload(z, (size_t)n * D, st);
     dgx.upload(gx, (size_t)n * D, st);
     HIPC(hipMemsetAsync(dvx.p, 0, n * sizeof(double), st));
@@ -2052,6 +2165,7 @@ int nuts_flow_pullback_grad(nuts_flow* f, const double* z, const double* gx, int
     HIPC(hipMemcpyAsync(gz, dgz.p, (size_t)n * D * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
     f->net->check_barriers();
+    span.done();
     return NUTS_OK;
   });
 }
@@ -2061,10 +2175,12 @@ int nuts_flow_loss_grad(nuts_flow* f, const double* x, int n, double* loss, floa
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
-    DevBuf<double> dx((size_t)n * D);
+    PoolSpan span(f->ws);
+    DevBuf<double> dx(&f->ws, (size_t)n * D);
     dx.upload(x, (size_t)n * D, st);
     const double l = f->net->loss_grad(dx.p, n, grad);
     if (loss) *loss = l;
+    span.done();
     return NUTS_OK;
   });
 }
@@ -2076,11 +2192,13 @@ int nuts_flow_train(nuts_flow* f, const double* x, int64_t n, int steps, int bat
       throw std::invalid_argument("flow: bad training arguments");
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
-    DevBuf<double> dx((size_t)n * D);
+    PoolSpan span(f->ws);
+    DevBuf<double> dx(&f->ws, (size_t)n * D);
     dx.upload(x, (size_t)n * D, st);
     HIPC(hipStreamSynchronize(st));
     const double l = f->net->train(dx.p, n, steps, batch, (float)lr, seed, std::min(20, std::max(1, steps)));
     if (final_loss) *final_loss = l;
+    span.done();
     return NUTS_OK;
   });
 }

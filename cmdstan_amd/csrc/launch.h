@@ -46,6 +46,16 @@ bool launch_advance_fused_block(int kind, int metric, bool vec32, const NutsPara
 bool model_supports_fused_block(int kind, int metric);
 bool model_supports_vec32(int kind);
 
+// Run set-up and results (batch_kernels.hip): C contiguous D x D blocks
+// transposed (*bad set when an element is not finite), identity metrics, fills,
+// rows of D[c] values (FP32 or FP64) at src + off[c] packed at out + to[c].
+void launch_metric_transpose(const double* A, double* M, int C, int D, int* bad, hipStream_t st);
+void launch_metric_identity(double* M, const int* D, const int64_t* moff, int C, int maxD, hipStream_t st);
+void launch_fill(double* p, int64_t n, double v, hipStream_t st);
+void launch_fill(float* p, int64_t n, float v, hipStream_t st);
+void launch_pack_rows(const void* src, bool f32, const int64_t* off, const int* D, const int64_t* to, int C,
+                      double* out, hipStream_t st);
+
 // Per-chain model gradient: V[c], G row c at Q row c for chains with need[c]
 // (need == nullptr: all chains).  Clears need[c].
 void launch_model_grad(int kind, int C, const int* D, const int64_t* off, const double* Q, double* G, double* V,
