@@ -31,16 +31,6 @@ __global__ void __launch_bounds__(256) advance_fused_block_kernel(NutsParams P, 
   nuts_advance_body<METRIC, F, 256, VT>(P, B, f);
 }
 
-// Initial factorisation of every chain's dense inverse metric (one wave per chain).
-__global__ void __launch_bounds__(256) dense_factor_kernel(NutsBuffers B, int* failed) {
-  const int c = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (c >= B.C) return;
-  const int D = B.D[c];
-  const bool ok = NutsWave<METRIC_DENSE, ExternalGrad>::dense_factor(B.dM + B.moff[c], B.dL + B.moff[c], D, lane);
-  if (!ok && lane == 0) atomicAdd(failed, 1);
-}
-
 template <class F>
 __global__ void __launch_bounds__(256) model_grad_kernel(F f, int C, const int* D, const int64_t* off, const double* Q,
                                                          double* G, double* V, int* need) {
@@ -98,10 +88,6 @@ void launch_advance_external_block(int metric, const NutsParams& P, const NutsBu
   else if (metric == METRIC_DENSE)
     hipLaunchKernelGGL(advance_external_block_kernel<METRIC_DENSE>, grid, blk, 0, st, P, B);
   else hipLaunchKernelGGL(advance_external_block_kernel<METRIC_DIAG>, grid, blk, 0, st, P, B);
-}
-
-void launch_dense_factor(const NutsBuffers& B, int* failed, hipStream_t st) {
-  hipLaunchKernelGGL(dense_factor_kernel, dim3(blocks_for(B.C)), dim3(256), 0, st, B, failed);
 }
 
 // vec32: the sampler's vectors in FP32 (unit/diag metrics, models with F::vec32)
