@@ -263,46 +263,79 @@ __device__ __forceinline__ void pass_doubling(bool fwd, VT* __restrict__ rho, co
 // loading the next; here the loads of four columns issue together.  Rows past
 // D read a valid element (row D-1) and are never stored, so the loads carry
 // no branches.
+template <int TPC, int NX, int RB, int U, class VT>
+__device__ __forceinline__ void dense_matvec_rows(const double* __restrict__ M, const VT* __restrict__ x1,
+                                                  const VT* __restrict__ x2, VT* __restrict__ out1,
+                                                  VT* __restrict__ out2, int D, int tid, int i0) {
+  double a1[RB], a2[RB];
+  int ii[RB];
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    a1[r] = 0.0;
+    a2[r] = 0.0;
+    const int i = i0 + tid + TPC * r;
+    ii[r] = i < D ? i : D - 1;
+  }
+  int j = 0;
+  for (; j + U <= D; j += U) {
+    double v[U][RB], y1[U], y2[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      y1[u] = x1[j + u];
+      if (NX > 1) y2[u] = x2[j + u];
+      const double* col = M + (int64_t)(j + u) * D;
+#pragma unroll
+      for (int r = 0; r < RB; ++r) v[u][r] = col[ii[r]];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int r = 0; r < RB; ++r) {
+        a1[r] += v[u][r] * y1[u];
+        if (NX > 1) a2[r] += v[u][r] * y2[u];
+      }
+  }
+  for (; j < D; ++j) {
+    const double y1j = x1[j], y2j = NX > 1 ? (double)x2[j] : 0.0;
+    const double* col = M + (int64_t)j * D;
+#pragma unroll
+    for (int r = 0; r < RB; ++r) {
+      const double m = col[ii[r]];
+      a1[r] += m * y1j;
+      if (NX > 1) a2[r] += m * y2j;
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RB; ++r) {
+    const int i = i0 + tid + TPC * r;
+    if (i < D) {
+      out1[i] = a1[r];
+      if (NX > 1) out2[i] = a2[r];
+    }
+  }
+}
+
+// As many rows per thread as D needs (block mode: a chain's matvec is a chain
+// of D / U waits for memory, so fewer rows buy more columns in flight; with
+// four rows and four columns at D = 520 half the loads were of rows past D).
+template <int TPC, int NX, class VT>
+__device__ __forceinline__ void dense_matvec_all(const double* __restrict__ M, const VT* __restrict__ x1,
+                                                 const VT* __restrict__ x2, VT* __restrict__ out1,
+                                                 VT* __restrict__ out2, int D, int tid) {
+  if constexpr (TPC >= 256) {
+    if (D <= TPC) dense_matvec_rows<TPC, NX, 1, 16>(M, x1, x2, out1, out2, D, tid, 0);
+    else if (D <= 2 * TPC) dense_matvec_rows<TPC, NX, 2, 8>(M, x1, x2, out1, out2, D, tid, 0);
+    else if (D <= 3 * TPC) dense_matvec_rows<TPC, NX, 3, 8>(M, x1, x2, out1, out2, D, tid, 0);
+    else for (int i0 = 0; i0 < D; i0 += 4 * TPC) dense_matvec_rows<TPC, NX, 4, 4>(M, x1, x2, out1, out2, D, tid, i0);
+  } else {
+    for (int i0 = 0; i0 < D; i0 += 8 * TPC) dense_matvec_rows<TPC, NX, 8, 4>(M, x1, x2, out1, out2, D, tid, i0);
+  }
+}
+
 template <int TPC, class VT>
 __device__ __noinline__ void dense_matvec(const double* __restrict__ M, const VT* __restrict__ x,
                                           VT* __restrict__ out, int D, int tid) {
-  constexpr int RB = TPC >= 256 ? 4 : 8;  // TPC * RB rows per pass (dense_e: D <= 1024)
-  for (int i0 = 0; i0 < D; i0 += TPC * RB) {
-    double acc[RB];
-    int ii[RB];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      acc[r] = 0.0;
-      const int i = i0 + tid + TPC * r;
-      ii[r] = i < D ? i : D - 1;
-    }
-    int j = 0;
-    for (; j + 4 <= D; j += 4) {
-      double v[4][RB], xv[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        xv[u] = x[j + u];
-        const double* col = M + (int64_t)(j + u) * D;
-#pragma unroll
-        for (int r = 0; r < RB; ++r) v[u][r] = col[ii[r]];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int r = 0; r < RB; ++r) acc[r] += v[u][r] * xv[u];
-    }
-    for (; j < D; ++j) {
-      const double xj = x[j];
-      const double* col = M + (int64_t)j * D;
-#pragma unroll
-      for (int r = 0; r < RB; ++r) acc[r] += col[ii[r]] * xj;
-    }
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const int i = i0 + tid + TPC * r;
-      if (i < D) out[i] = acc[r];
-    }
-  }
+  dense_matvec_all<TPC, 1, VT>(M, x, x, out, out, D, tid);
 }
 
 // out1 = M x1 and out2 = M x2 in one pass over M (same order of summation as
@@ -311,55 +344,7 @@ template <int TPC, class VT>
 __device__ __noinline__ void dense_matvec2(const double* __restrict__ M, const VT* __restrict__ x1,
                                            const VT* __restrict__ x2, VT* __restrict__ out1, VT* __restrict__ out2,
                                            int D, int tid) {
-  constexpr int RB = TPC >= 256 ? 4 : 8;
-  for (int i0 = 0; i0 < D; i0 += TPC * RB) {
-    double a1[RB], a2[RB];
-    int ii[RB];
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      a1[r] = 0.0;
-      a2[r] = 0.0;
-      const int i = i0 + tid + TPC * r;
-      ii[r] = i < D ? i : D - 1;
-    }
-    int j = 0;
-    for (; j + 4 <= D; j += 4) {
-      double v[4][RB], y1[4], y2[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        y1[u] = x1[j + u];
-        y2[u] = x2[j + u];
-        const double* col = M + (int64_t)(j + u) * D;
-#pragma unroll
-        for (int r = 0; r < RB; ++r) v[u][r] = col[ii[r]];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int r = 0; r < RB; ++r) {
-          a1[r] += v[u][r] * y1[u];
-          a2[r] += v[u][r] * y2[u];
-        }
-    }
-    for (; j < D; ++j) {
-      const double y1j = x1[j], y2j = x2[j];
-      const double* col = M + (int64_t)j * D;
-#pragma unroll
-      for (int r = 0; r < RB; ++r) {
-        const double m = col[ii[r]];
-        a1[r] += m * y1j;
-        a2[r] += m * y2j;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < RB; ++r) {
-      const int i = i0 + tid + TPC * r;
-      if (i < D) {
-        out1[i] = a1[r];
-        out2[i] = a2[r];
-      }
-    }
-  }
+  dense_matvec_all<TPC, 2, VT>(M, x1, x2, out1, out2, D, tid);
 }
 
 // The same products (one or two at once) for a chain whose vectors are in LDS:
@@ -1062,7 +1047,7 @@ struct NutsWave {
         le[k] = Lend(kk);
         lr[k] = Lrho(kk);
       }
-      double acc[1 + 6 * 3];
+      double acc[1 + 6 * 3] = {};
       if constexpr (LV) {
         leaf_sums<UNIT, 0>(p, lb, le, lr, dp, dr, db, edge, hh, acc);
       } else {
@@ -1094,10 +1079,11 @@ struct NutsWave {
         else { free_slot(s.s_prop); s.s_prop = s.L_prop[k]; }
         double a1, b1, a2, b2, a3, b3;
         if (!LV && k < F) {
-          // selects, not an index: acc stays in registers
-          auto at = [&](int j) { return k == 0 ? acc[1 + j] : (k == 1 ? acc[7 + j] : acc[13 + j]); };
-          a1 = at(0); b1 = at(1); a2 = at(2);
-          b2 = at(3); a3 = at(4); b3 = at(5);
+          a1 = acc[1]; b1 = acc[2]; a2 = acc[3];
+          b2 = acc[4]; a3 = acc[5]; b3 = acc[6];
+          // the next level's sums move up: no index, so acc stays in registers
+#pragma unroll
+          for (int j = 1; j < 13; ++j) acc[j] = acc[j + 6];
         } else {
           // deeper merges: the separate pass over the stored leaf momentum and
           // the rho merged so far (the begin is level k-1's, the leaf at level 0)
