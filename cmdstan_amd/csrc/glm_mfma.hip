@@ -1,9 +1,9 @@
-// Batched logistic-regression gradient on FP64 matrix cores (gfx950).
+// Batched logistic-regression gradient on FP64 matrix cores (gfx950), D <= 128.
 //
-// For a tile of 64 observations and 64 chains (4 waves x 16 chains):
-//   phase 1  Eta = X_tile · Qᵀ            v_mfma_f64_16x16x4: M = rows, N = chains, K = D
-//   pointwise R = sigmoid(Eta) - y, lp += y·Eta - log1p(e^Eta)   (in registers)
-//   phase 2  Gᵀ += Rᵀ · X_tile             M = chains, N = D, K = rows
+// For a tile of rows and 16 points per wave (v_mfma_f64_16x16x4):
+//   phase 1  Eta = X_tile . Q^T           M = rows, N = points, K = D
+//   pointwise R = sigmoid(Eta) - y, lp += y.Eta - log1p(e^Eta)   (in registers)
+//   phase 2  G^T += R^T . X_tile           M = points, N = D, K = rows
 // The 16x16x4 f64 result layout puts element (4i + l/16, l%16) in register i of
 // lane l.  Phase 2 walks the rows of the tile in the order (block rb, register
 // i, lane group l/16), so the A operand of each phase-2 step is exactly register
@@ -11,9 +11,25 @@
 // B operand of phase 2 reads X in that same row order from the LDS tile that
 // phase 1 used.
 //
-// Work split: blocks own (row chunk, 64-chain group); the linear block id is
-// remapped so that the chain groups sharing one row chunk run on the same XCD
-// and share its L2.  Chunk partials go to a workspace reduced in fixed order
+// Two ways to share a block's four waves:
+//   SPLIT = 1  64 points, 16 per wave, on a common 32-row tile, double-buffered
+//              in LDS (more than 16 points)
+//   SPLIT = 4  16 points, the waves on row tiles of their own (16 rows each, in
+//              wave-private LDS: no barriers), summed at the end (at most 16
+//              points: three of four waves would multiply padding)
+// The next tile's loads are issued before the current tile's products and wait
+// in registers (2 D / 16 doubles per thread) until they are done.
+//
+// The step counts are template parameters (DT 16-column tiles, KS = 4 DT - R
+// four-column steps), so the products are straight-line code whose operand
+// reads run ahead of them.  With runtime counts every step was a branch, an LDS
+// read waited for at once, and -- the tile being copied straight to LDS -- a
+// wait for the whole copy of the next tile: 45-50% of the FP64 matrix peak at
+// N = 100000, D = 100, 1024 points.
+//
+// Work split: blocks own (row chunk, 64-point group); the linear block id is
+// remapped so that the groups sharing one row chunk run on the same XCD and
+// share its L2.  Chunk partials go to a workspace reduced in fixed order
 // (deterministic, no atomics).
 #include "device_common.h"
 #include "glm_split.h"
@@ -24,20 +40,37 @@ namespace nutsgpu {
 typedef double d4 __attribute__((ext_vector_type(4)));
 
 
-#define GM_TN 64            // rows per tile
-#define GM_TC 64            // chains per block
-#define GM_KMAX 128         // D capacity (K of phase 1, N of phase 2)
-#define GM_XS (GM_KMAX + 2) // LDS row stride in doubles (== 2 mod 32: conflict-free phase-1 reads)
+#define GM_TC 64    // points per group of the work split
+#define GM_KMAX 128 // D capacity
 
-template <int KMAX>
+// The residual and the log-likelihood term of one observation; a row past the
+// chunk (live false) counts as zero.
+__device__ __forceinline__ double gm_residual(double e, double yy, bool live, double& lp) {
+  // t = e^{-|e|}: log1p_exp(e) = max(e,0) + log1p(t), sigmoid(e) from 1 / (1 + t)
+  const double t = exp(-fabs(e));
+  double r1;
+  const double l1p = log1p_recip_unit(t, r1);
+  const double term = yy * e - ((e > 0.0 ? e : 0.0) + l1p);
+  const double r = (e >= 0.0 ? r1 : t * r1) - yy;
+  lp += live ? term : 0.0;
+  return live ? r : 0.0;
+}
+
+template <int DT, int R, int SPLIT>
 __global__ void __launch_bounds__(256, 2)
 glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, int D, int total_blocks,
              const double* __restrict__ Q, int64_t ldq, int C, const int* __restrict__ idx,
              const int* __restrict__ n_active, double* __restrict__ Wg, double* __restrict__ Wlp) {
-  __shared__ double sX[GM_TN * GM_XS];
-  __shared__ double sY[GM_TN];
+  constexpr int KS = 4 * DT - R;              // phase-1 steps
+  constexpr int XS = 16 * DT + 2;             // LDS row stride
+  constexpr int TR = SPLIT == 1 ? 32 : 16;    // rows per tile
+  constexpr int RB = TR / 16;
+  constexpr int STEP = SPLIT == 1 ? 32 : 64;  // rows per iteration of the block
+  constexpr int FR = SPLIT == 1 ? 2 : 4;      // prefetched rows per thread
+  __shared__ double sX[SPLIT == 1 ? 2 : 4][TR * XS];
+  __shared__ double sY[SPLIT == 1 ? 2 : 4][TR];
   const int tid = threadIdx.x;
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63;
   const int lr = l & 15;   // m/n index inside a 16-wide tile
   const int lk = l >> 4;   // k index inside a 4-deep step
@@ -52,244 +85,131 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
   const int group = j % sp.groups;
   if (chunk >= sp.chunks || group * GM_TC >= n_act) return;
 
-  const int c0 = group * GM_TC + 16 * w;  // this wave's 16 positions
-  const int KS = (D + 3) >> 2;            // phase-1 k-steps
-  const int DT = (D + 15) >> 4;           // phase-2 output tiles
-
+  const int c0 = group * GM_TC + (SPLIT == 1 ? 16 * w : 0);  // this wave's 16 positions
   // phase-1 B operand for all k-steps: Q[c0 + lr][4 ks + lk]
-  double qreg[KMAX / 4];
+  double qreg[KS];
   {
     const int pos = c0 + lr;
     const int c = pos < n_act ? (idx ? idx[pos] : pos) : -1;
+    const double* qr = Q + (int64_t)(c < 0 ? 0 : c) * ldq;
 #pragma unroll
-    for (int ks = 0; ks < KMAX / 4; ++ks) {
+    for (int ks = 0; ks < KS; ++ks) {
       const int k = 4 * ks + lk;
-      qreg[ks] = (ks < KS && c >= 0 && k < D) ? Q[(int64_t)c * ldq + k] : 0.0;
+      const double v = qr[k < D ? k : 0];
+      qreg[ks] = c >= 0 && k < D ? v : 0.0;
     }
   }
-  d4 gacc[KMAX / 16];
+  d4 gacc[DT];
 #pragma unroll
-  for (int t = 0; t < KMAX / 16; ++t) gacc[t] = d4{0, 0, 0, 0};
+  for (int t = 0; t < DT; ++t) gacc[t] = d4{0, 0, 0, 0};
   double lp = 0.0;
-
   const int n_begin = chunk * sp.rows;
   const int n_end = min(N, n_begin + sp.rows);
-  const int ncols = DT * 16;
 
-  for (int nb = n_begin; nb < n_end; nb += GM_TN) {
-    __syncthreads();
-    // 16 lanes cover 16 consecutive columns of a row: 128-byte segments
+  // prefetch: 16 lanes cover 16 consecutive columns of a row (128-byte
+  // segments); rows and columns outside read a clamped address and count as zero
+  const int pr = SPLIT == 1 ? tid >> 4 : lk;      // first row of this thread in the tile
+  constexpr int PS = SPLIT == 1 ? 16 : 4;         // its row step
+  const int roff = SPLIT == 1 ? 0 : 16 * w;       // the wave's rows inside an iteration
+  double xr[FR][DT], yr = 0.0;
+  auto fetch = [&](int nb) {
 #pragma unroll
-    for (int m = 0; m < GM_TN / 16; ++m) {
-      const int r = (tid >> 4) + 16 * m;
-      const int n = nb + r;
-      const bool rowok = n < n_end;
-      const double* xr = X + (int64_t)n * D;
+    for (int m = 0; m < FR; ++m) {
+      const int n = nb + roff + pr + PS * m;
+      const double* row = X + (int64_t)(n < n_end ? n : n_end - 1) * D;
 #pragma unroll
-      for (int jj = 0; jj < KMAX / 16; ++jj) {
-        const int k = (tid & 15) + 16 * jj;
-        if (k < ncols) sX[r * GM_XS + k] = (rowok && k < D) ? xr[k] : 0.0;
+      for (int t = 0; t < DT; ++t) {
+        const int k = 16 * t + lr;
+        const double v = row[t < DT - 1 || k < D ? k : 0];
+        xr[m][t] = n < n_end && (t < DT - 1 || k < D) ? v : 0.0;
       }
     }
-    if (tid < GM_TN) sY[tid] = (nb + tid < n_end) ? y[nb + tid] : 0.0;
-    __syncthreads();
-
-    d4 eta[4];
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) eta[rb] = d4{0, 0, 0, 0};
-#pragma unroll
-    for (int ks = 0; ks < KMAX / 4; ++ks) {
-      if (ks < KS) {
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-          const double a = sX[(16 * rb + lr) * GM_XS + 4 * ks + lk];
-          eta[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, qreg[ks], eta[rb], 0, 0, 0);
-        }
-      }
-    }
-    // R = sigmoid(eta) - y in place; rows past the chunk contribute nothing
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int rr = 16 * rb + 4 * i + lk;
-        const double e = eta[rb][i];
-        double r = 0.0;
-        if (nb + rr < n_end) {
-          // one exp: log1p_exp(e) = max(e,0) + log1p(t), sigmoid(e) from t = e^{-|e|}
-          const double yy = sY[rr];
-          const double t = exp(-fabs(e));
-          double r1;
-          const double l1p = log1p_recip_unit(t, r1);
-          lp += yy * e - ((e > 0.0 ? e : 0.0) + l1p);
-          r = (e >= 0.0 ? r1 : t * r1) - yy;
-        }
-        eta[rb][i] = r;
-      }
-    }
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const double a = eta[rb][i];
-        const double* xrow = sX + (16 * rb + 4 * i + lk) * GM_XS + lr;
-#pragma unroll
-        for (int t = 0; t < KMAX / 16; ++t) {
-          if (t < DT) gacc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, xrow[16 * t], gacc[t], 0, 0, 0);
-        }
-      }
-    }
-  }
-
-  // gacc[t] register i of lane l = G[chain c0 + 4i + lk][d 16t + lr]
-#pragma unroll
-  for (int t = 0; t < KMAX / 16; ++t) {
-    if (t < DT) {
-      const int d = 16 * t + lr;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int pos = c0 + 4 * i + lk;
-        if (pos < n_act && d < D) Wg[((int64_t)chunk * sp.stride + pos) * D + d] = gacc[t][i];
-      }
-    }
-  }
-  // lp: lanes l, l+16, l+32, l+48 hold the same chain
-  lp += __shfl_xor(lp, 16, 64);
-  lp += __shfl_xor(lp, 32, 64);
-  if (lk == 0 && c0 + lr < n_act) Wlp[(int64_t)chunk * sp.stride + c0 + lr] = lp;
-}
-
-// Even D: the same products on 32-row tiles double-buffered in LDS.  The next
-// tile's rows are copied global -> LDS by global_load_lds_dwordx4 (16 bytes
-// per lane, lane l at row base + 16 l, exec-masked lanes leave their slots
-// alone -- checked on the device), one instruction per row, issued before the
-// current tile's products and waited for (vmcnt, then the barrier) after
-// them: the copy needs no registers and overlaps the matrix work.  Columns
-// past D stay zero from the initial clear; rows past the chunk hold finite
-// data of an earlier tile and contribute nothing (their residual is 0).  Rows
-// are summed in the order of the 64-row kernel, so the products match it bit
-// for bit; the per-observation terms use two reciprocals instead of divisions.
-typedef __attribute__((address_space(3))) void lds_void;
-#define GL_TN 32  // rows per double-buffered tile
-
-template <int KMAX>
-__global__ void __launch_bounds__(256, 2)
-glm_mfma_f64_lds(const double* __restrict__ X, const double* __restrict__ y, int N, int D, int total_blocks,
-                 const double* __restrict__ Q, int64_t ldq, int C, const int* __restrict__ idx,
-                 const int* __restrict__ n_active, double* __restrict__ Wg, double* __restrict__ Wlp) {
-  __shared__ __attribute__((aligned(16))) double sX[2][GL_TN * GM_XS];
-  __shared__ double sY[2][GL_TN];
-  const int tid = threadIdx.x;
-  const int w = tid >> 6;
-  const int l = tid & 63;
-  const int lr = l & 15;
-  const int lk = l >> 4;
-
-  const int n_act = idx ? *n_active : C;
-  const GlmSplit sp = glm_split(n_act, N, total_blocks);
-  const int lin = blockIdx.x;
-  const int xcd = lin & 7;
-  const int j = lin >> 3;
-  const int chunk = xcd + 8 * (j / sp.groups);
-  const int group = j % sp.groups;
-  if (chunk >= sp.chunks || group * GM_TC >= n_act) return;
-
-  const int c0 = group * GM_TC + 16 * w;
-  const int KS = (D + 3) >> 2;
-  const int DT = (D + 15) >> 4;
-  double qreg[KMAX / 4];
-  {
-    const int pos = c0 + lr;
-    const int c = pos < n_act ? (idx ? idx[pos] : pos) : -1;
-#pragma unroll
-    for (int ks = 0; ks < KMAX / 4; ++ks) {
-      const int k = 4 * ks + lk;
-      qreg[ks] = (ks < KS && c >= 0 && k < D) ? Q[(int64_t)c * ldq + k] : 0.0;
-    }
-  }
-  d4 gacc[KMAX / 16];
-#pragma unroll
-  for (int t = 0; t < KMAX / 16; ++t) gacc[t] = d4{0, 0, 0, 0};
-  double lp = 0.0;
-
-  const int n_begin = chunk * sp.rows;
-  const int n_end = min(N, n_begin + sp.rows);
-  for (int i = tid; i < 2 * GL_TN * GM_XS; i += 256) (&sX[0][0])[i] = 0.0;
-  const int nch = D >> 1;  // 16-byte chunks per row
-  // wave w copies rows 8 w .. 8 w + 7 of the tile
-  auto issue = [&](int nb, int b) {
-#pragma unroll
-    for (int rr = 0; rr < GL_TN / 4; ++rr) {
-      const int r = w * (GL_TN / 4) + rr;
-      const int n = nb + r;
-      if (n < n_end && l < nch)
-        __builtin_amdgcn_global_load_lds(X + (int64_t)n * D + 2 * l, (lds_void*)&sX[b][r * GM_XS], 16, 0, 0);
-    }
+    const int ny = nb + roff + (SPLIT == 1 ? (tid & 31) : lr);
+    yr = ny < n_end ? y[ny] : 0.0;
   };
-  __syncthreads();
-  if (tid < GL_TN) sY[0][tid] = (n_begin + tid < n_end) ? y[n_begin + tid] : 0.0;
-  issue(n_begin, 0);
-  int b = 0;
-  for (int nb = n_begin; nb < n_end; nb += GL_TN, b ^= 1) {
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    const int nxt = nb + GL_TN;
-    double yn = 0.0;
-    if (nxt < n_end) {
-      issue(nxt, b ^ 1);
-      if (tid < GL_TN) yn = (nxt + tid < n_end) ? y[nxt + tid] : 0.0;
+  auto stash = [&](int b) {
+    double* sx = sX[b];
+#pragma unroll
+    for (int m = 0; m < FR; ++m)
+#pragma unroll
+      for (int t = 0; t < DT; ++t) sx[(pr + PS * m) * XS + 16 * t + lr] = xr[m][t];
+    if (SPLIT == 1 ? tid < TR : l < TR) sY[b][SPLIT == 1 ? tid : l] = yr;
+  };
+  int b = SPLIT == 1 ? 0 : w;
+  if (n_begin < n_end) {
+    fetch(n_begin);
+    stash(b);
+  }
+  for (int nb = n_begin; nb < n_end; nb += STEP) {
+    if constexpr (SPLIT == 1) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+      __builtin_amdgcn_wave_barrier();
     }
+    const bool more = nb + STEP < n_end;
+    if (more) fetch(nb + STEP);
     const double* sx = sX[b];
-    d4 eta[2];
+    const double* sy = sY[b];
+    d4 eta[RB];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) eta[rb] = d4{0, 0, 0, 0};
+    for (int rb = 0; rb < RB; ++rb) eta[rb] = d4{0, 0, 0, 0};
 #pragma unroll
-    for (int ks = 0; ks < KMAX / 4; ++ks) {
-      if (ks < KS) {
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int rb = 0; rb < 2; ++rb) {
-          const double a = sx[(16 * rb + lr) * GM_XS + 4 * ks + lk];
-          eta[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, qreg[ks], eta[rb], 0, 0, 0);
-        }
-      }
-    }
+      for (int rb = 0; rb < RB; ++rb)
+        eta[rb] = __builtin_amdgcn_mfma_f64_16x16x4f64(sx[(16 * rb + lr) * XS + 4 * ks + lk], qreg[ks], eta[rb], 0, 0, 0);
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int rr = 16 * rb + 4 * i + lk;
-        const double e = eta[rb][i];
-        double r = 0.0;
-        if (nb + rr < n_end) {
-          // t = e^{-|e|}: log1p_exp(e) = max(e,0) + log1p(t), sigmoid(e) from 1 / (1 + t)
-          const double yy = sY[b][rr];
-          const double t = exp(-fabs(e));
-          double r1;
-          const double l1p = log1p_recip_unit(t, r1);
-          lp += yy * e - ((e > 0.0 ? e : 0.0) + l1p);
-          r = (e >= 0.0 ? r1 : t * r1) - yy;
-        }
-        eta[rb][i] = r;
+        eta[rb][i] = gm_residual(eta[rb][i], sy[rr], nb + roff + rr < n_end, lp);
       }
-    }
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
+    for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const double a = eta[rb][i];
-        const double* xrow = sx + (16 * rb + 4 * i + lk) * GM_XS + lr;
+        const double* xrow = sx + (16 * rb + 4 * i + lk) * XS + lr;
 #pragma unroll
-        for (int t = 0; t < KMAX / 16; ++t) {
-          if (t < DT) gacc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, xrow[16 * t], gacc[t], 0, 0, 0);
-        }
+        for (int t = 0; t < DT; ++t)
+          gacc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(eta[rb][i], xrow[16 * t], gacc[t], 0, 0, 0);
       }
+    if (more) {
+      if constexpr (SPLIT == 1) b ^= 1;  // the other buffer: its readers passed this iteration's barrier
+      else {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+      stash(b);
     }
-    if (tid < GL_TN) sY[b ^ 1][tid] = yn;
   }
 
+  lp += __shfl_xor(lp, 16, 64);
+  lp += __shfl_xor(lp, 32, 64);
+  if constexpr (SPLIT == 4) {
+    // the four waves' sums: tile by tile through LDS, wave 0 + 1 + 2 + 3
+    __shared__ double red[4][256];
+    __shared__ double redlp[4][16];
+    if (lk == 0) redlp[w][lr] = lp;
 #pragma unroll
-  for (int t = 0; t < KMAX / 16; ++t) {
-    if (t < DT) {
+    for (int t = 0; t < DT; ++t) {
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 4; ++i) red[w][64 * i + l] = gacc[t][i];
+      __syncthreads();
+      const int pos = c0 + (tid >> 4), d = 16 * t + (tid & 15);  // element tid: point tid / 16, column tid % 16
+      if (pos < n_act && d < D)
+        Wg[((int64_t)chunk * sp.stride + pos) * D + d] = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
+    }
+    if (tid < 16 && c0 + tid < n_act)
+      Wlp[(int64_t)chunk * sp.stride + c0 + tid] =
+          ((redlp[0][tid] + redlp[1][tid]) + redlp[2][tid]) + redlp[3][tid];
+  } else {
+    // gacc[t] register i of lane l = G[chain c0 + 4i + lk][d 16t + lr]; lanes l,
+    // l + 16, l + 32, l + 48 hold the same chain's lp
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
       const int d = 16 * t + lr;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -297,16 +217,19 @@ glm_mfma_f64_lds(const double* __restrict__ X, const double* __restrict__ y, int
         if (pos < n_act && d < D) Wg[((int64_t)chunk * sp.stride + pos) * D + d] = gacc[t][i];
       }
     }
+    if (lk == 0 && c0 + lr < n_act) Wlp[(int64_t)chunk * sp.stride + c0 + lr] = lp;
   }
-  lp += __shfl_xor(lp, 16, 64);
-  lp += __shfl_xor(lp, 32, 64);
-  if (lk == 0 && c0 + lr < n_act) Wlp[(int64_t)chunk * sp.stride + c0 + lr] = lp;
 }
 
-__global__ void glm_mfma_reduce(const double* __restrict__ Wg, const double* __restrict__ Wlp, int N,
-                                int total_blocks, int C, int D, double s2inv, const double* __restrict__ Q,
-                                int64_t ldq, const int* __restrict__ idx, const int* __restrict__ n_active,
-                                double* __restrict__ G, double* __restrict__ V) {
+// G and V of every point from the chunk partials: 64 columns x 8 chunk slices
+// per block, a fixed order (slice z takes chunks z, z + 8, ...), eight loads in
+// flight per thread.  A few points have few blocks and many chunks: one thread
+// per column walking all chunks took 8.0 us at 160 chunks.
+__global__ void __launch_bounds__(512)
+glm_mfma_reduce(const double* __restrict__ Wg, const double* __restrict__ Wlp, int N, int total_blocks, int C, int D,
+                double s2inv, const double* __restrict__ Q, int64_t ldq, const int* __restrict__ idx,
+                const int* __restrict__ n_active, double* __restrict__ G, double* __restrict__ V) {
+  __shared__ double red[8][64];
   const int pos = blockIdx.x;
   const int n_act = idx ? *n_active : C;
   if (pos >= n_act) return;
@@ -314,20 +237,28 @@ __global__ void glm_mfma_reduce(const double* __restrict__ Wg, const double* __r
   const int c = idx ? idx[pos] : pos;
   const double* q = Q + (int64_t)c * ldq;
   double* g = G + (int64_t)c * ldq;
-  for (int k = threadIdx.x; k < D; k += blockDim.x) {
-    double s = 0.0;
-    // chunk order kept; sixteen loads in flight instead of one
-#pragma unroll 16
-    for (int ch = 0; ch < sp.chunks; ++ch) s += Wg[((int64_t)ch * sp.stride + pos) * D + k];
-    g[k] = s + s2inv * q[k];
+  const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
+  const int k = blockIdx.y * 64 + lane;
+  double s = 0.0;
+  if (k < D) {
+#pragma unroll 8
+    for (int ch = z; ch < sp.chunks; ch += 8) s += Wg[((int64_t)ch * sp.stride + pos) * D + k];
   }
-  if (threadIdx.x < 64) {
+  red[z][lane] = s;
+  __syncthreads();
+  if (z == 0 && k < D) {
+    double t = 0.0;
+#pragma unroll
+    for (int v = 0; v < 8; v += 2) t += red[v][lane] + red[v + 1][lane];
+    g[k] = t + s2inv * q[k];
+  }
+  if (blockIdx.y == 0 && z == 1) {
     double lpv = 0.0, pr = 0.0;
-    for (int ch = threadIdx.x; ch < sp.chunks; ch += 64) lpv += Wlp[(int64_t)ch * sp.stride + pos];
-    for (int k = threadIdx.x; k < D; k += 64) pr += q[k] * q[k];
+    for (int ch = lane; ch < sp.chunks; ch += 64) lpv += Wlp[(int64_t)ch * sp.stride + pos];
+    for (int i = lane; i < D; i += 64) pr += q[i] * q[i];
     lpv = wave_sum(lpv);
     pr = wave_sum(pr);
-    if (threadIdx.x == 0) V[c] = -(lpv - 0.5 * s2inv * pr);
+    if (lane == 0) V[c] = -(lpv - 0.5 * s2inv * pr);
   }
 }
 
@@ -390,28 +321,42 @@ GlmPlan glm_mfma_plan(int N, int C, int D, int num_cus, int blocks_per_cu) {
   return p;
 }
 
+template <int DT, int R>
+static void gm_launch(const GlmArgs& a, const GlmPlan& p, double* Wg, double* Wlp, hipStream_t st) {
+  // at most 16 points: the waves split the rows (see the top of the file)
+  if (a.C <= 16)
+    hipLaunchKernelGGL((glm_mfma_f64<DT, R, 4>), dim3(p.total_blocks), dim3(256), 0, st, a.X, a.y, a.N, a.D,
+                       p.total_blocks, a.Q, a.ldq, a.C, a.idx, a.n_active, Wg, Wlp);
+  else
+    hipLaunchKernelGGL((glm_mfma_f64<DT, R, 1>), dim3(p.total_blocks), dim3(256), 0, st, a.X, a.y, a.N, a.D,
+                       p.total_blocks, a.Q, a.ldq, a.C, a.idx, a.n_active, Wg, Wlp);
+}
+
+template <int DT>
+static void gm_launch_tiles(const GlmArgs& a, const GlmPlan& p, double* Wg, double* Wlp, hipStream_t st) {
+  switch (4 * DT - (a.D + 3) / 4) {  // four-column steps the last tile leaves out
+    case 0: gm_launch<DT, 0>(a, p, Wg, Wlp, st); break;
+    case 1: gm_launch<DT, 1>(a, p, Wg, Wlp, st); break;
+    case 2: gm_launch<DT, 2>(a, p, Wg, Wlp, st); break;
+    default: gm_launch<DT, 3>(a, p, Wg, Wlp, st); break;
+  }
+}
+
 int glm_grad_mfma_f64(const GlmArgs& a, const GlmPlan& p, hipStream_t st) {
   if (a.D > GM_KMAX || a.D < 1) return 1;
   double* Wg = a.work;
   double* Wlp = a.work + (size_t)p.total_blocks * GM_TC * a.D;
-  // even D: rows are whole 16-byte chunks, so the double-buffered LDS copy applies
-#define GM_LAUNCH(K)                                                                                                \
-  do {                                                                                                              \
-    if ((a.D & 1) == 0)                                                                                             \
-      hipLaunchKernelGGL(glm_mfma_f64_lds<K>, dim3(p.total_blocks), dim3(256), 0, st, a.X, a.y, a.N, a.D,           \
-                         p.total_blocks, a.Q, a.ldq, a.C, a.idx, a.n_active, Wg, Wlp);                              \
-    else                                                                                                            \
-      hipLaunchKernelGGL(glm_mfma_f64<K>, dim3(p.total_blocks), dim3(256), 0, st, a.X, a.y, a.N, a.D,               \
-                         p.total_blocks, a.Q, a.ldq, a.C, a.idx, a.n_active, Wg, Wlp);                              \
-  } while (0)
   if (a.ev_begin) (void)hipEventRecord(a.ev_begin, st);
-  // operand registers scale with the D bucket (a 64 bucket spilled registers:
-  // 33 <= D <= 112 share the 112 instance, whose extra operands are zero)
-  if (a.D <= 16) GM_LAUNCH(16);
-  else if (a.D <= 32) GM_LAUNCH(32);
-  else if (a.D <= 112) GM_LAUNCH(112);
-  else GM_LAUNCH(128);
-#undef GM_LAUNCH
+  switch ((a.D + 15) / 16) {
+    case 1: gm_launch_tiles<1>(a, p, Wg, Wlp, st); break;
+    case 2: gm_launch_tiles<2>(a, p, Wg, Wlp, st); break;
+    case 3: gm_launch_tiles<3>(a, p, Wg, Wlp, st); break;
+    case 4: gm_launch_tiles<4>(a, p, Wg, Wlp, st); break;
+    case 5: gm_launch_tiles<5>(a, p, Wg, Wlp, st); break;
+    case 6: gm_launch_tiles<6>(a, p, Wg, Wlp, st); break;
+    case 7: gm_launch_tiles<7>(a, p, Wg, Wlp, st); break;
+    default: gm_launch_tiles<8>(a, p, Wg, Wlp, st); break;
+  }
   if (a.ev_end) (void)hipEventRecord(a.ev_end, st);
   glm_reduce_launch(a, p, st);
   return 0;
@@ -420,9 +365,8 @@ int glm_grad_mfma_f64(const GlmArgs& a, const GlmPlan& p, hipStream_t st) {
 void glm_reduce_launch(const GlmArgs& a, const GlmPlan& p, hipStream_t st) {
   double* Wg = a.work;
   double* Wlp = a.work + (size_t)p.total_blocks * GM_TC * a.D;
-  hipLaunchKernelGGL(glm_mfma_reduce, dim3(a.C), dim3(128), 0, st, Wg, Wlp, a.N, p.total_blocks, a.C, a.D, a.s2inv,
-                     a.Q, a.ldq,
-                     a.idx, a.n_active, a.G, a.V);
+  hipLaunchKernelGGL(glm_mfma_reduce, dim3(a.C, (a.D + 63) / 64), dim3(512), 0, st, Wg, Wlp, a.N, p.total_blocks, a.C,
+                     a.D, a.s2inv, a.Q, a.ldq, a.idx, a.n_active, a.G, a.V);
 }
 
 }  // namespace nutsgpu
