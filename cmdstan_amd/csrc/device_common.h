@@ -141,6 +141,22 @@ __device__ __forceinline__ double log1p_recip_unit(double t, double& r1) {
   return __builtin_fma(2.0 * s, p, hi ? 0.69314718055994531 : 0.0);
 }
 
+// Sum of log(1 + t) over many t in [0, 1] as the logarithm of their product: a
+// multiplication per term and one logarithm at the end.  fold() after at most
+// 900 terms keeps the mantissa in range.  Each factor and product rounds by
+// 1e-16 of itself, so the sum is off by about 2e-16 per term, below the rounding
+// of adding the terms up one by one.
+struct LogProduct {
+  double m = 1.0;
+  int e = 0;
+  __device__ __forceinline__ void times(double one_plus_t) { m *= one_plus_t; }
+  __device__ __forceinline__ void fold() {
+    e += __builtin_amdgcn_frexp_exp(m);
+    m = __builtin_amdgcn_frexp_mant(m);
+  }
+  __device__ __forceinline__ double log_value() const { return log(m) + (double)e * 0.69314718055994531; }
+};
+
 __device__ __forceinline__ double log1p_exp(double a) {
   return a > 0.0 ? a + log1p(exp(-a)) : log1p(exp(a));
 }

@@ -43,16 +43,17 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 #define GM_TC 64    // points per group of the work split
 #define GM_KMAX 128 // D capacity
 
-// The residual and the log-likelihood term of one observation; a row past the
-// chunk (live false) counts as zero.
-__device__ __forceinline__ double gm_residual(double e, double yy, bool live, double& lp) {
-  // t = e^{-|e|}: log1p_exp(e) = max(e,0) + log1p(t), sigmoid(e) from 1 / (1 + t)
+// The residual and the log-likelihood of one observation; a row past the chunk
+// (live false) counts as zero.  lp takes y e - max(e, 0), lg the log1p term (as
+// a factor): the vector unit's FP64 work shares its pipes with the FP64 matrix
+// products, so these operations add to the products' time instead of hiding
+// behind it -- a series of log1p per observation was a third of them.
+__device__ __forceinline__ double gm_residual(double e, double yy, bool live, double& lp, LogProduct& lg) {
   const double t = exp(-fabs(e));
-  double r1;
-  const double l1p = log1p_recip_unit(t, r1);
-  const double term = yy * e - ((e > 0.0 ? e : 0.0) + l1p);
-  const double r = (e >= 0.0 ? r1 : t * r1) - yy;
-  lp += live ? term : 0.0;
+  const double d = 1.0 + t;
+  const double r = (e >= 0.0 ? 1.0 : t) * recip_small(d) - yy;
+  lp += live ? yy * e - (e > 0.0 ? e : 0.0) : 0.0;
+  lg.times(live ? d : 1.0);
   return live ? r : 0.0;
 }
 
@@ -103,6 +104,7 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
 #pragma unroll
   for (int t = 0; t < DT; ++t) gacc[t] = d4{0, 0, 0, 0};
   double lp = 0.0;
+  LogProduct lg;
   const int n_begin = chunk * sp.rows;
   const int n_end = min(N, n_begin + sp.rows);
 
@@ -164,8 +166,9 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int rr = 16 * rb + 4 * i + lk;
-        eta[rb][i] = gm_residual(eta[rb][i], sy[rr], nb + roff + rr < n_end, lp);
+        eta[rb][i] = gm_residual(eta[rb][i], sy[rr], nb + roff + rr < n_end, lp, lg);
       }
+    lg.fold();
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -185,6 +188,7 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
     }
   }
 
+  lp -= lg.log_value();
   lp += __shfl_xor(lp, 16, 64);
   lp += __shfl_xor(lp, 32, 64);
   if constexpr (SPLIT == 4) {

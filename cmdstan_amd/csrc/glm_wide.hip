@@ -124,6 +124,7 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
   // round the waves: wave w finishes items w, w + W, ...
   constexpr int IT = (4 * NG + W - 1) / W;
   double lp[IT];
+  LogProduct lg[IT];
 #pragma unroll
   for (int m = 0; m < IT; ++m) lp[m] = 0.0;
   if (n_begin < n_end) fetch(n_begin);
@@ -164,10 +165,11 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
         if (n < n_end) {
           const double yy = a.y[n];
           const double t = exp(-fabs(e));
-          double r1;
-          const double l1p = log1p_recip_unit(t, r1);
-          lp[m] += yy * e - ((e > 0.0 ? e : 0.0) + l1p);
-          r = (e >= 0.0 ? r1 : t * r1) - yy;
+          const double d = 1.0 + t;
+          lp[m] += yy * e - (e > 0.0 ? e : 0.0);
+          lg[m].times(d);
+          lg[m].fold();
+          r = (e >= 0.0 ? 1.0 : t) * recip_small(d) - yy;
         }
         sR[64 * item + l] = r;
       }
@@ -210,7 +212,7 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
 #pragma unroll
   for (int m = 0; m < IT; ++m) {
     const int item = w + W * m;
-    double v = lp[m];
+    double v = lp[m] - lg[m].log_value();
     v += __shfl_xor(v, 16, 64);
     v += __shfl_xor(v, 32, 64);
     if (item < 4 * NG && lk == 0) sR[16 * item + lr] = v;
