@@ -910,6 +910,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     }
   }
   const int hl_groups = hl_ok ? M.ds[R.first_dataset].groups : 0;
+  const int hl_k = hl_ok ? M.ds[R.first_dataset].group_size : 0;
   DevBuf<double> fX(ws), fGX(ws), fVX(ws), fLD(ws);
   if (R.flow) {
     if (!act_idx.p) {
@@ -1047,7 +1048,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
         if (with_events) HIPC(hipEventRecord(ev.a[k], st));
         R.flow->forward(Q.p, Dp[0], act_idx.p, n_act.p, C, fX.p, fLD.p);
         if (hl_ok) {
-          hl_grad_launch(hla, hl_groups, st);
+          hl_grad_launch(hla, hl_groups, hl_k, st);
         } else if (glm_ok || gw_ok) {
           ga.n_active = n_act.p;
           glm_grad();
@@ -1074,7 +1075,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
       } else if (hl_ok) {
         launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
         if (with_events) HIPC(hipEventRecord(ev.a[k], st));
-        hl_grad_launch(hla, hl_groups, st);
+        hl_grad_launch(hla, hl_groups, hl_k, st);
         if (with_events) HIPC(hipEventRecord(ev.b[k], st));
       } else if (M.plugin) {
         launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
@@ -1977,7 +1978,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
       a.block = M.d_data.p + M.ds_off[dataset];
       a.Q = Q.p; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = C;
       a.Gout = G.p; a.ldg = D; a.Vout = V.p; a.work = work.p; a.jac = jacobian ? 1.0 : 0.0;
-      hl_grad_launch(a, hd.groups, 0);
+      hl_grad_launch(a, hd.groups, hd.group_size, 0);
     } else {
       dD.alloc(C);
       doff.alloc(C);
@@ -2060,7 +2061,7 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       a.block = M.d_data.p + M.ds_off[dataset];
       a.Q = d_q; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = n;
       a.Gout = d_grad; a.ldg = D; a.Vout = V; a.work = work; a.jac = jacobian ? 1.0 : 0.0;
-      hl_grad_launch(a, hd.groups, st);
+      hl_grad_launch(a, hd.groups, hd.group_size, st);
     } else {
       hipLaunchKernelGGL(noalloc_tables, dim3((n + 255) / 256), dim3(256), 0, st, Dv, off, dso, n, D,
                          M.ds_off[dataset]);

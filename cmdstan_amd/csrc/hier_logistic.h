@@ -22,7 +22,7 @@ struct HlArgs {
   double jac;            // 1: add the log-Jacobian of tau = exp(v)
 };
 
-void hl_grad_launch(const HlArgs& a, int G, hipStream_t st);
+void hl_grad_launch(const HlArgs& a, int G, int K, hipStream_t st);
 size_t hl_work_doubles(int G, int K, int n_rows);
 
 }  // namespace nutsgpu

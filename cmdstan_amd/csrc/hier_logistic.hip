@@ -2,37 +2,37 @@
 // (one dataset):
 //   mu_k ~ N(0, mu_s), tau_k = exp(v_k) ~ HalfNormal(1) (+ v_k Jacobian),
 //   beta[g][k] ~ N(mu_k, tau_k), y_n ~ bernoulli_logit(x_n . beta[group_n]).
-// Kernel 1 takes one group and 64 chains per block: lane = chain, the group's
-// observations are staged in LDS and read as broadcasts, each lane keeps its
-// chain's beta[g] and gradient in registers (K <= 16), the four waves split the
-// observations and combine through LDS.  It writes the beta[g] gradient
-// directly and per-group partials for the hyperparameters; kernel 2 reduces
-// those over groups in a fixed order (deterministic, no atomics).
+// Kernel 1 takes one group and a tile of points per block: a lane owns one point
+// and keeps its beta[g] and gradient in registers (K <= 16, a template parameter:
+// the K products of an observation are straight-line code on broadcast LDS reads),
+// and the block's other lanes split the observations -- four ways for a tile of
+// 64 points (one wave each), sixteen ways for a tile of 16, where most lanes of a
+// 64-point tile would have no point.  It writes the beta[g] gradient directly and
+// per-group partials for the hyperparameters; kernel 2 reduces those over groups
+// in a fixed order (deterministic, no atomics).
+// Bound: the FP64 vector unit (4 K + some 45 operations per observation and
+// point).  log(1 + e^eta) is a factor of one product per lane, its logarithm
+// taken once at the end (LogProduct).
 // Dataset block (host layout): [N, K, G, mu_s, gstart[G+1], X[N*K] sorted by group, y[N]].
 #include "device_common.h"
 #include "hier_logistic.h"
 
 namespace nutsgpu {
 
-#define HL_TC 64     // chains per block
 #define HL_OBS 128   // observations staged per LDS pass
 #define HL_KMAX 16
 
-// log(1 + e^e) and sig = 1 / (1 + e^-e) from one exponential and one reciprocal
-__device__ __forceinline__ double hl_log1p_exp(double e, double* sig) {
-  const double t = exp(-fabs(e));
-  double r1;
-  const double l1p = log1p_recip_unit(t, r1);
-  *sig = e >= 0.0 ? r1 : t * r1;
-  return (e > 0.0 ? e : 0.0) + l1p;
-}
-
+// partials of the hyperparameters: column j of group g at ((j G) + g) n + pos
+// (j < K d lp / d mu_k, then d lp / d tau_k, last the log density), so the lanes of
+// a tile store runs of points and kernel 2 reads them back as such
+template <int K, int TC>
 __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
-  __shared__ double sX[HL_OBS * HL_KMAX];
+  constexpr int SPLIT = 256 / TC;  // observations split this many ways
+  __shared__ double sX[HL_OBS * K];
   __shared__ double sY[HL_OBS];
-  __shared__ double sRed[4][HL_TC][HL_KMAX + 1];
+  __shared__ double sRed[SPLIT][TC][K + 1];
   const double* d = a.block;
-  const int K = (int)d[1], G = (int)d[2];
+  const int G = (int)d[2];
   const double* gstart = d + 4;
   const double* X = d + 5 + G;
   const int N = (int)d[0];
@@ -40,20 +40,21 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
   const int g = blockIdx.x % G;
   const int tile = blockIdx.x / G;
   const int n_act = a.n_dev ? min(a.n_rows, *a.n_dev) : a.n_rows;
-  const int p0 = tile * HL_TC;
+  const int p0 = tile * TC;
   if (p0 >= n_act) return;
-  const int t = threadIdx.x, w = t >> 6, lane = t & 63;
+  const int t = threadIdx.x, w = t / TC, lane = t % TC;
   const int pos = p0 + lane;
   const bool live = pos < n_act;
   const int64_t row_in = live ? (a.idx_in ? (int64_t)a.idx[pos] : pos) : 0;
   const double* q = a.Q + row_in * a.ldq;
-  double b[HL_KMAX], gb[HL_KMAX];
+  double b[K], gb[K];
 #pragma unroll
-  for (int k = 0; k < HL_KMAX; ++k) {
-    b[k] = (live && k < K) ? q[2 * K + (int64_t)g * K + k] : 0.0;
+  for (int k = 0; k < K; ++k) {
+    b[k] = live ? q[2 * K + (int64_t)g * K + k] : 0.0;
     gb[k] = 0.0;
   }
   double lp = 0.0;
+  LogProduct lg;
   const int n0 = (int)gstart[g], n1 = (int)gstart[g + 1];
   for (int base = n0; base < n1; base += HL_OBS) {
     const int cnt = min(HL_OBS, n1 - base);
@@ -61,108 +62,135 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
     for (int i = t; i < cnt * K; i += 256) sX[i] = X[(int64_t)base * K + i];
     for (int i = t; i < cnt; i += 256) sY[i] = y[base + i];
     __syncthreads();
-    // two observations per step: independent exp/log chains in flight
-    for (int n = w; n < cnt; n += 8) {
-      const int n2 = n + 4;
+    // two observations per step: independent exponentials in flight
+    for (int n = w; n < cnt; n += 2 * SPLIT) {
+      const int n2 = n + SPLIT;
       const bool two = n2 < cnt;
       const double* xr = sX + n * K;
       const double* xr2 = sX + (two ? n2 : n) * K;
-      double e = 0.0, e2 = 0.0;
+      double x1[K], x2[K], e = 0.0, e2 = 0.0;
 #pragma unroll
-      for (int k = 0; k < HL_KMAX; ++k)
-        if (k < K) { e += xr[k] * b[k]; e2 += xr2[k] * b[k]; }
-      double sig, sig2;
+      for (int k = 0; k < K; ++k) {
+        x1[k] = xr[k];
+        x2[k] = xr2[k];
+        e += x1[k] * b[k];
+        e2 += x2[k] * b[k];
+      }
       const double yy = sY[n], yy2 = two ? sY[n2] : 0.0;
-      const double l1 = hl_log1p_exp(e, &sig);
-      const double l2 = hl_log1p_exp(e2, &sig2);
-      lp += yy * e - l1;
-      const double r = yy - sig;
-      const double r2 = two ? yy2 - sig2 : 0.0;
-      if (two) lp += yy2 * e2 - l2;
+      const double t1 = exp(-fabs(e)), t2 = exp(-fabs(e2));
+      const double d1 = 1.0 + t1, d2 = 1.0 + t2;
+      const double r = yy - (e >= 0.0 ? 1.0 : t1) * recip_small(d1);
+      const double s2 = yy2 - (e2 >= 0.0 ? 1.0 : t2) * recip_small(d2);
+      const double r2 = two ? s2 : 0.0;
+      lp += yy * e - (e > 0.0 ? e : 0.0);
+      lg.times(d1);
+      if (two) {
+        lp += yy2 * e2 - (e2 > 0.0 ? e2 : 0.0);
+        lg.times(d2);
+      }
 #pragma unroll
-      for (int k = 0; k < HL_KMAX; ++k)
-        if (k < K) gb[k] += r * xr[k] + r2 * xr2[k];
+      for (int k = 0; k < K; ++k) gb[k] += r * x1[k] + r2 * x2[k];
     }
+    lg.fold();  // at most 2 HL_OBS / (2 SPLIT) factors since the last
   }
-  // combine the four waves' partial sums
+  // combine the partial sums of the observation split
 #pragma unroll
-  for (int k = 0; k < HL_KMAX; ++k)
-    if (k < K) sRed[w][lane][k] = gb[k];
-  sRed[w][lane][HL_KMAX] = lp;
+  for (int k = 0; k < K; ++k) sRed[w][lane][k] = gb[k];
+  sRed[w][lane][K] = lp - lg.log_value();
   __syncthreads();
-  if (w == 0 && live) {
-    double lpt = 0.0;
-    for (int ww = 0; ww < 4; ++ww) lpt += sRed[ww][lane][HL_KMAX];
-    const int64_t row_out = a.idx_out ? (int64_t)a.idx[pos] : pos;
-    double* gout = a.Gout + row_out * a.ldg;
-    double* part = a.work + ((int64_t)g * a.n_rows + pos) * (2 * K + 1);
-    double lprior = 0.0;
-    for (int k = 0; k < K; ++k) {
-      double s = 0.0;
-      for (int ww = 0; ww < 4; ++ww) s += sRed[ww][lane][k];
-      const double mu = q[k], v = q[K + k];
-      const double tau = exp(v);
-      const double dd = b[k] - mu;
-      const double z = dd / tau;
-      // d lp / d beta = likelihood score - (beta - mu) / tau^2
-      gout[2 * K + (int64_t)g * K + k] = -(s - dd / (tau * tau));
-      part[k] = dd / (tau * tau);                            // d/d mu
-      part[K + k] = -1.0 / tau + dd * dd / (tau * tau * tau);  // d/d tau
-      lprior += -v - 0.5 * z * z;
+  // thread (point, k): beta gradient and the hyperparameters' partials
+  for (int i = t; i < TC * K; i += 256) {
+    const int ln = i % TC, k = i / TC;
+    const int ps = p0 + ln;
+    if (ps >= n_act) continue;
+    const int64_t ri = a.idx_in ? (int64_t)a.idx[ps] : ps, ro = a.idx_out ? (int64_t)a.idx[ps] : ps;
+    const double* qp = a.Q + ri * a.ldq;
+    double s = 0.0;
+#pragma unroll
+    for (int ww = 0; ww < SPLIT; ++ww) s += sRed[ww][ln][k];
+    const double mu = qp[k], v = qp[K + k], bk = qp[2 * K + (int64_t)g * K + k];
+    const double it = exp(-v);  // 1 / tau
+    const double dd = bk - mu;
+    const double z = dd * it;
+    const double dz = z * it;  // (beta - mu) / tau^2
+    // d lp / d beta = likelihood score - (beta - mu) / tau^2
+    a.Gout[ro * a.ldg + 2 * K + (int64_t)g * K + k] = -(s - dz);
+    a.work[((int64_t)k * G + g) * a.n_rows + ps] = dz;                   // d/d mu
+    a.work[((int64_t)(K + k) * G + g) * a.n_rows + ps] = z * dz - it;    // d/d tau
+    if (k == 0) {
+      double lpt = 0.0;
+#pragma unroll
+      for (int ww = 0; ww < SPLIT; ++ww) lpt += sRed[ww][ln][K];
+#pragma unroll
+      for (int kk = 0; kk < K; ++kk) {
+        const double vk = qp[K + kk];
+        const double zk = (qp[2 * K + (int64_t)g * K + kk] - qp[kk]) * exp(-vk);
+        lpt += -vk - 0.5 * zk * zk;
+      }
+      a.work[((int64_t)(2 * K) * G + g) * a.n_rows + ps] = lpt;
     }
-    part[2 * K] = lpt + lprior;
   }
 }
 
-// hyperparameters, one wave per position: lanes take groups g = lane, lane+64,
-// ... and keep the 2K+1 column sums in registers, then combine with butterflies
+// hyperparameters: a block per (column of the partials, 64 points), four waves
+// over the groups (lane = point, so every read is a run of points), then one
+// thread per point; the log density's column also takes the priors
 __global__ void __launch_bounds__(256) hl_hyper_kernel(HlArgs a) {
+  __shared__ double red[4][64];
   const double* d = a.block;
   const int K = (int)d[1], G = (int)d[2];
   const double mu_s = d[3];
   const int n_act = a.n_dev ? min(a.n_rows, *a.n_dev) : a.n_rows;
-  const int pos = blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (pos >= n_act) return;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int p0 = blockIdx.x * 64, j = blockIdx.y;
+  if (p0 >= n_act) return;
+  const int pos = p0 + lane;
+  double s = 0.0;
+  if (pos < n_act) {
+    const double* col = a.work + (int64_t)j * G * a.n_rows + pos;
+#pragma unroll 8
+    for (int g = w; g < G; g += 4) s += col[(int64_t)g * a.n_rows];
+  }
+  red[w][lane] = s;
+  __syncthreads();
+  if (w != 0 || pos >= n_act) return;
+  s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
   const int64_t row_in = a.idx_in ? (int64_t)a.idx[pos] : pos;
   const int64_t row_out = a.idx_out ? (int64_t)a.idx[pos] : pos;
   const double* q = a.Q + row_in * a.ldq;
   double* gout = a.Gout + row_out * a.ldg;
-  const int W = 2 * K + 1;
-  double acc[2 * HL_KMAX + 1];
-#pragma unroll
-  for (int j = 0; j < 2 * HL_KMAX + 1; ++j) acc[j] = 0.0;
-  for (int g = lane; g < G; g += NUTS_WAVE) {
-    const double* pr = a.work + ((int64_t)g * a.n_rows + pos) * W;
-#pragma unroll
-    for (int j = 0; j < 2 * HL_KMAX + 1; ++j)
-      if (j < W) acc[j] += pr[j];
-  }
-  double lp = 0.0;
-#pragma unroll
-  for (int j = 0; j < 2 * HL_KMAX + 1; ++j) {
-    if (j >= W) continue;
-    const double s = wave_sum(acc[j]);
-    if (j < K) {
-      const double mu = q[j];
-      if (lane == 0) gout[j] = -(s - mu / (mu_s * mu_s));
-      lp += -0.5 * mu * mu / (mu_s * mu_s);
-    } else if (j < 2 * K) {
-      const double v = q[j];
-      const double tau = exp(v);
-      if (lane == 0) gout[j] = -(a.jac + tau * (s - tau));
-      lp += -0.5 * tau * tau + a.jac * v;
-    } else {
-      lp += s;
+  if (j < K) {
+    gout[j] = -(s - q[j] / (mu_s * mu_s));
+  } else if (j < 2 * K) {
+    const double tau = exp(q[j]);
+    gout[j] = -(a.jac + tau * (s - tau));
+  } else {
+    double lp = s;
+    for (int k = 0; k < K; ++k) {
+      const double mu = q[k], v = q[K + k], tau = exp(v);
+      lp += -0.5 * mu * mu / (mu_s * mu_s) - 0.5 * tau * tau + a.jac * v;
     }
+    a.Vout[row_out] = -lp;
   }
-  if (lane == 0) a.Vout[row_out] = -lp;
 }
 
-void hl_grad_launch(const HlArgs& a, int G, hipStream_t st) {
-  const int tiles = (a.n_rows + HL_TC - 1) / HL_TC;
-  hipLaunchKernelGGL(hl_group_kernel, dim3(G * tiles), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(hl_hyper_kernel, dim3((a.n_rows + 3) / 4), dim3(256), 0, st, a);
+template <int K>
+static void hl_group_launch(const HlArgs& a, int G, hipStream_t st) {
+  // tiles of 16 points while a 64-point tile would be less than half full
+  if (a.n_rows <= 32)
+    hipLaunchKernelGGL((hl_group_kernel<K, 16>), dim3(G * ((a.n_rows + 15) / 16)), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((hl_group_kernel<K, 64>), dim3(G * ((a.n_rows + 63) / 64)), dim3(256), 0, st, a);
+}
+
+void hl_grad_launch(const HlArgs& a, int G, int K, hipStream_t st) {
+  switch (K) {
+#define HL_CASE(k) case k: hl_group_launch<k>(a, G, st); break;
+    HL_CASE(1) HL_CASE(2) HL_CASE(3) HL_CASE(4) HL_CASE(5) HL_CASE(6) HL_CASE(7) HL_CASE(8)
+    HL_CASE(9) HL_CASE(10) HL_CASE(11) HL_CASE(12) HL_CASE(13) HL_CASE(14) HL_CASE(15) HL_CASE(16)
+#undef HL_CASE
+    default: return;  // the model is refused at K > HL_KMAX
+  }
+  hipLaunchKernelGGL(hl_hyper_kernel, dim3((a.n_rows + 63) / 64, 2 * K + 1), dim3(256), 0, st, a);
 }
 
 size_t hl_work_doubles(int G, int K, int n_rows) { return (size_t)G * n_rows * (2 * K + 1); }
