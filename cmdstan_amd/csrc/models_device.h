@@ -4,8 +4,8 @@
 // (cmdstan src/cmdstan/command_helper.hpp:569-600 evaluates
 // stan::model::log_prob_grad<true, jacobian>) and writes gV = -grad log p.
 // Model data are packed per dataset into one double array; `off[c]` gives the
-// dataset block of chain c.  write_array maps an unconstrained draw to the
-// constrained outputs in Stan's column order.  bind(c) names the chain the next
+// dataset block of chain c.  output(j, q) is the j-th
+// constrained output of an unconstrained draw in Stan's column order.  bind(c) names the chain the next
 // calls are for: it resolves the chain's block once, not once per gradient.
 #pragma once
 #include "device_common.h"
@@ -47,7 +47,7 @@ struct BernoulliFn {
     return -lp;
   }
   __device__ int nout(int) const { return 1; }
-  __device__ void write_array(int, const double* q, double* out) const { out[0] = inv_logit(q[0]); }
+  __device__ double output(int, const double* q) const { return inv_logit(q[0]); }
 };
 
 // q ~ multi_normal_prec(mu, P); block = [D, mu[D], P transposed [D*D] row-major]:
@@ -123,10 +123,7 @@ struct GaussFn {
     return 0.5 * wave_sum(acc);
   }
   __device__ int nout(int c) const { return (int)md.d[0]; }
-  __device__ void write_array(int c, const double* q, double* out) const {
-    const int D = (int)md.d[0];
-    for (int i = 0; i < D; ++i) out[i] = q[i];
-  }
+  __device__ double output(int j, const double* q) const { return q[j]; }
 };
 
 // Eight schools, centered: (mu, tau, theta[J]); theta ~ normal(mu, tau);
@@ -166,11 +163,7 @@ struct EightSchoolsFn {
     return -lp;
   }
   __device__ int nout(int c) const { return (int)md.d[0] + 2; }
-  __device__ void write_array(int c, const double* q, double* out) const {
-    const int J = (int)md.d[0];
-    out[0] = q[0]; out[1] = exp(q[1]);
-    for (int j = 0; j < J; ++j) out[2 + j] = q[2 + j];
-  }
+  __device__ double output(int j, const double* q) const { return j == 1 ? exp(q[1]) : q[j]; }
 };
 
 // Non-centered hierarchical normal: mu ~ normal(0, mu_s); tau ~ cauchy(0, tau_s), tau>0;
@@ -218,11 +211,11 @@ struct HierNormalNCFn {
     return group<NUTS_WAVE>(c, q, gV, lane, [](double x) { return wave_sum(x); });
   }
   __device__ int nout(int c) const { return 2 + 2 * (int)md.d[0]; }
-  __device__ void write_array(int c, const double* q, double* out) const {
+  __device__ double output(int j, const double* q) const {
     const int J = (int)md.d[0];
+    if (j < 2 + J) return j == 1 ? exp(q[1]) : q[j];
     const double tau = exp(q[1]);
-    out[0] = q[0]; out[1] = tau;
-    for (int j = 0; j < J; ++j) { out[2 + j] = q[2 + j]; out[2 + J + j] = q[0] + tau * q[2 + j]; }
+    return q[0] + tau * q[j - J];  // theta of group j - 2 - J
   }
 };
 
@@ -291,12 +284,10 @@ struct HierLogisticFn {
     const double* d = md.d;
     return 2 * (int)d[1] + (int)d[1] * (int)d[2];
   }
-  __device__ void write_array(int c, const double* q, double* out) const {
-    const double* d = md.d;
-    const int K = (int)d[1], G = (int)d[2];
-    for (int k = 0; k < K; ++k) { out[k] = q[k]; out[K + k] = exp(q[K + k]); }
-    for (int k = 0; k < K; ++k)
-      for (int g = 0; g < G; ++g) out[2 * K + k * G + g] = q[2 * K + g * K + k];
+  __device__ double output(int j, const double* q) const {
+    const int K = (int)md.d[1], G = (int)md.d[2];
+    if (j < 2 * K) return j < K ? q[j] : exp(q[j]);
+    return q[2 * K + (j - 2 * K) % G * K + (j - 2 * K) / G];  // beta column-major (group fastest)
   }
 };
 
@@ -343,10 +334,7 @@ struct LogisticFn {
     return -(wave_sum(acc) - 0.5 * s2inv * pr);
   }
   __device__ int nout(int c) const { return (int)md.d[1]; }
-  __device__ void write_array(int c, const double* q, double* out) const {
-    const int D = (int)md.d[1];
-    for (int k = 0; k < D; ++k) out[k] = q[k];
-  }
+  __device__ double output(int j, const double* q) const { return q[j]; }
 };
 
 // runs CALL with `f`, the functor of the model kind over the data md

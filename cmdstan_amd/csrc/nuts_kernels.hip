@@ -60,17 +60,18 @@ __global__ void __launch_bounds__(256) model_grad_rows_kernel(F f, const int* id
   if (lane == 0) VX[r] = v;
 }
 
+// a block per saved row, its threads over the outputs (a thread per row walked
+// them one by one: 1.58 ms for 2560 rows of 4020 outputs)
 template <class F>
-__global__ void write_array_kernel(F f, int C, int rows, const int* D, const int64_t* in_off, const int64_t* out_off,
-                                   const int* nout, const double* in, double* out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (int64_t)C * rows) return;
+__global__ void __launch_bounds__(256) write_array_kernel(F f, int64_t row0, int rows, const int* D,
+                                                          const int64_t* in_off, const int64_t* out_off,
+                                                          const int* nout, const double* in, double* out) {
+  const int64_t t = row0 + blockIdx.x;
   const int c = (int)(t / rows), r = (int)(t % rows);
   const double* src = in + in_off[c] + (int64_t)r * (7 + D[c]);
   double* dst = out + out_off[c] + (int64_t)r * (7 + nout[c]);
-  for (int i = 0; i < 7; ++i) dst[i] = src[i];
   f.bind(c);
-  f.write_array(c, src + 7, dst + 7);
+  for (int i = threadIdx.x; i < 7 + nout[c]; i += 256) dst[i] = i < 7 ? src[i] : f.output(i - 7, src + 7);
 }
 
 static int blocks_for(int C) { return (C + 3) / 4; }
@@ -177,11 +178,12 @@ void launch_model_grad_rows(int kind, const int* idx, const int* n_dev, int n_ro
 void launch_write_array(int kind, int C, int rows, const int* D, const int64_t* in_off, const int64_t* out_off,
                         const int* nout, const double* in, double* out, const ModelDataDev& md, hipStream_t st) {
   const int64_t n = (int64_t)C * rows;
-  if (n == 0) return;
-  const dim3 grid((unsigned)((n + 127) / 128)), blk(128);
-  NUTS_MODEL_SWITCH(kind, md,
-                    hipLaunchKernelGGL((write_array_kernel<decltype(f)>), grid, blk, 0, st, f, C, rows, D, in_off,
-                                       out_off, nout, in, out));
+  for (int64_t r0 = 0; r0 < n; r0 += 1 << 20) {
+    const dim3 grid((unsigned)(n - r0 < (1 << 20) ? n - r0 : 1 << 20)), blk(256);
+    NUTS_MODEL_SWITCH(kind, md,
+                      hipLaunchKernelGGL((write_array_kernel<decltype(f)>), grid, blk, 0, st, f, r0, rows, D, in_off,
+                                         out_off, nout, in, out));
+  }
 }
 
 }  // namespace nutsgpu
