@@ -54,15 +54,24 @@ __device__ __forceinline__ float fg_epi(const GemmDesc& g, float v, int m, int n
 }
 
 // 64x64 tile per block of four waves (2x2), each wave 32x32 = 2x2 MFMA tiles;
-// K in slabs of 64 (each thread stages 16 elements of A and 16 of B per slab,
-// so a slab's loads are in flight together, and the next slab's loads are
-// issued before the current slab's products: a tile waits on memory about
-// once, however long its K range).
+// K in slabs of 64 (each thread stages 16 elements of A and 16 of B per slab).
+// A product here is a few hundred rows by H or D columns: the tile waits for
+// memory, not for the matrix cores, so a slab's 32 loads are issued together --
+// out-of-range elements read a clamped address and count as zero; guarded loads
+// were a branch, an index load and a wait per element (18.6 us for a launch of
+// two slabs) -- and the next slab's before the current slab's products.
+// A_K: A's k are adjacent in memory (else its m), B_N: B's n are adjacent (else
+// its k).  A wave's load takes 64 adjacent elements, and each operand is stored
+// in LDS the way it is read, with a row stride that puts the 64 lanes of an
+// MFMA operand on distinct banks: [m][k] with stride 68, [k][m] with stride 80.
 // f32 16x16x4 operands: lane l gives A[l%16][k=l/16], B[k=l/16][l%16]; result
 // register i of lane l is D[4(l/16)+i][l%16].
+template <bool A_K, bool B_N>
 __global__ void __launch_bounds__(256) flow_gemm_kernel(GemmDesc g) {
-  __shared__ float As[FG_BK][FG_BM + 4];
-  __shared__ float Bs[FG_BK][FG_BN + 4];
+  constexpr int LDA = A_K ? FG_BK + 4 : FG_BM + 16;
+  constexpr int LDB = B_N ? FG_BN + 16 : FG_BK + 4;
+  __shared__ float As[64 * LDA];
+  __shared__ float Bs[64 * LDB];
   const int M = g.Mdev ? min(g.M, *g.Mdev) : g.M;
   const int m0 = blockIdx.y * FG_BM, n0 = blockIdx.x * FG_BN;
   if (m0 >= M) return;
@@ -71,60 +80,71 @@ __global__ void __launch_bounds__(256) flow_gemm_kernel(GemmDesc g) {
   const int ke = min(g.K, kb + g.kper);
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
+  const int lr = l & 15, lk = l >> 4;
   f4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f4{0, 0, 0, 0};
-  const bool a_k = g.sak == 1;
-  const bool b_n = g.sbn == 1;
   float va[16], vb[16];
+  // element e of a thread: the wave's lane along the adjacent index, w + 4 e along the other
   auto fetch = [&](int k0) {
+    int64_t ka[16], ma[16];
+    if (A_K) {
+      const int k = min(k0 + l, ke - 1);
+      const int64_t kc = (g.aidx_k ? g.aidx_k[k] : k) * g.sak;
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      // k-contiguous A: 16 consecutive k of one row; else 4 rows x 4 slab rows
-      const int mm = a_k ? (t >> 2) : ((t & 15) * 4 + (e & 3));
-      const int kk = a_k ? ((t & 3) * 16 + e) : ((t >> 4) + 16 * (e >> 2));
-      const int m = m0 + mm, k = k0 + kk;
-      float v = 0.0f;
-      if (m < M && k < ke) {
-        const int64_t mr = g.aidx_m ? g.aidx_m[m] : m;
-        const int64_t kc = g.aidx_k ? g.aidx_k[k] : k;
-        v = g.A[mr * g.sam + kc * g.sak];
+      for (int e = 0; e < 16; ++e) {
+        const int m = min(m0 + w + 4 * e, M - 1);
+        ma[e] = (int64_t)(g.aidx_m ? g.aidx_m[m] : m) * g.sam;
+        ka[e] = kc;
       }
-      va[e] = v;
+    } else {
+      const int m = min(m0 + l, M - 1);
+      const int64_t mr = (int64_t)(g.aidx_m ? g.aidx_m[m] : m) * g.sam;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int k = min(k0 + w + 4 * e, ke - 1);
+        ka[e] = (int64_t)(g.aidx_k ? g.aidx_k[k] : k) * g.sak;
+        ma[e] = mr;
+      }
     }
 #pragma unroll
+    for (int e = 0; e < 16; ++e) va[e] = g.A[ma[e] + ka[e]];
+#pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int nn = b_n ? ((t & 15) * 4 + (e & 3)) : (t >> 2);
-      const int kk = b_n ? ((t >> 4) + 16 * (e >> 2)) : ((t & 3) * 16 + e);
-      const int n = n0 + nn, k = k0 + kk;
-      vb[e] = (n < g.N && k < ke) ? g.B[(int64_t)k * g.sbk + (int64_t)n * g.sbn] : 0.0f;
+      const int n = min(n0 + (B_N ? l : w + 4 * e), g.N - 1), k = min(k0 + (B_N ? w + 4 * e : l), ke - 1);
+      vb[e] = g.B[(int64_t)k * g.sbk + (int64_t)n * g.sbn];
     }
   };
-  // the next slab's loads are issued before the current slab's products
-  if (kb < ke) fetch(kb);
-  for (int k0 = kb; k0 < ke; k0 += FG_BK) {
+  auto stash = [&](int k0) {
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      const int mm = a_k ? (t >> 2) : ((t & 15) * 4 + (e & 3));
-      const int kk = a_k ? ((t & 3) * 16 + e) : ((t >> 4) + 16 * (e >> 2));
-      As[kk][mm] = va[e];
-      const int nn = b_n ? ((t & 15) * 4 + (e & 3)) : (t >> 2);
-      const int kb2 = b_n ? ((t >> 4) + 16 * (e >> 2)) : ((t & 3) * 16 + e);
-      Bs[kb2][nn] = vb[e];
+      const int mm = A_K ? w + 4 * e : l, ka = A_K ? l : w + 4 * e;
+      As[A_K ? mm * LDA + ka : ka * LDA + mm] = m0 + mm < M && k0 + ka < ke ? va[e] : 0.0f;
+      const int nn = B_N ? l : w + 4 * e, kk = B_N ? w + 4 * e : l;
+      Bs[B_N ? kk * LDB + nn : nn * LDB + kk] = n0 + nn < g.N && k0 + kk < ke ? vb[e] : 0.0f;
     }
+  };
+  if (kb < ke) fetch(kb);
+  for (int k0 = kb; k0 < ke; k0 += FG_BK) {
+    stash(k0);
     __syncthreads();
     if (k0 + FG_BK < ke) fetch(k0 + FG_BK);
 #pragma unroll
     for (int ks = 0; ks < FG_BK / 4; ++ks) {
-      const int kr = ks * 4 + (l >> 4);
-      const float a0 = As[kr][wm + (l & 15)], a1 = As[kr][wm + 16 + (l & 15)];
-      const float b0 = Bs[kr][wn + (l & 15)], b1 = Bs[kr][wn + 16 + (l & 15)];
-      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc[1][1], 0, 0, 0);
+      const int kr = ks * 4 + lk;
+      float a[2], b[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int m = wm + 16 * i + lr, n = wn + 16 * i + lr;
+        a[i] = As[A_K ? m * LDA + kr : kr * LDA + m];
+        b[i] = Bs[B_N ? kr * LDB + n : n * LDB + kr];
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
     }
     __syncthreads();
   }
@@ -134,8 +154,8 @@ __global__ void __launch_bounds__(256) flow_gemm_kernel(GemmDesc g) {
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm + 16 * i + 4 * (l >> 4) + r;
-        const int n = n0 + wn + 16 * j + (l & 15);
+        const int m = m0 + wm + 16 * i + 4 * lk + r;
+        const int n = n0 + wn + 16 * j + lr;
         if (m < M && n < g.N) {
           const float v = acc[i][j][r];
           if (g.splits > 1) g.part[((int64_t)split * g.M + m) * g.N + n] = v;
@@ -649,6 +669,7 @@ __global__ void __launch_bounds__(256) flow_logdet(const float* __restrict__ S, 
   for (int l = 0; l < L; ++l) {
     const int db = Db[l];
     const float* s = S + l * layer_stride + (int64_t)r * db;
+#pragma unroll 8
     for (int j = threadIdx.x; j < db; j += 256) acc += (double)s[j];
   }
   acc = wave_sum(acc);
@@ -754,15 +775,27 @@ __global__ void flow_rows_out(const float* __restrict__ U, int64_t n, double* __
   if (i < n) Z[i] = (double)U[i];
 }
 
-// column sums (bias gradients): out[c] = sum_r A[r][c]
-__global__ void flow_colsum(const float* __restrict__ A, int rows, int cols, float* __restrict__ out) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= cols) return;
+// column sums (bias gradients): out[c] = sum_r A[r][c]; 32 columns x 8 row
+// slices per block, slices added in order (one thread per column walked all
+// rows: 9.8 us at 256 rows, most of it with one block in flight)
+__global__ void __launch_bounds__(256) flow_colsum(const float* __restrict__ A, int rows, int cols,
+                                                   float* __restrict__ out) {
+  __shared__ float red[8][32];
+  const int x = threadIdx.x & 31, z = threadIdx.x >> 5;
+  const int c = blockIdx.x * 32 + x;
   float s = 0.0f;
-  // row order kept; eight loads in flight instead of one
-#pragma unroll 8
-  for (int r = 0; r < rows; ++r) s += A[(int64_t)r * cols + c];
-  out[c] = s;
+  if (c < cols) {
+#pragma unroll 16
+    for (int r = z; r < rows; r += 8) s += A[(int64_t)r * cols + c];
+  }
+  red[z][x] = s;
+  __syncthreads();
+  if (z == 0 && c < cols) {
+    float v = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v += red[k][x];
+    out[c] = v;
+  }
 }
 
 // per-row 0.5|z|^2
@@ -770,6 +803,7 @@ __global__ void flow_half_sq(const float* __restrict__ Z, int D, int n, double* 
   const int r = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (r >= n) return;
   double acc = 0;
+#pragma unroll 8
   for (int j = lane; j < D; j += NUTS_WAVE) {
     const double z = Z[(int64_t)r * D + j];
     acc += z * z;
@@ -1186,7 +1220,13 @@ void FlowNet::gemm(const float* A, int64_t sam, int64_t sak, const float* B, int
     if ((int64_t)splits * M * N > part_n_) throw std::logic_error("flow: split-K workspace too small");
     g.part = part_;
   }
-  hipLaunchKernelGGL(flow_gemm_kernel, dim3(tn, tm, splits), dim3(256), 0, st_, g);
+  // the operand's unit stride picks the variant (every product here has one)
+  const dim3 grid(tn, tm, splits), blk(256);
+  const bool ak = sak == 1, bn = sbn == 1;
+  if (ak && bn) hipLaunchKernelGGL((flow_gemm_kernel<true, true>), grid, blk, 0, st_, g);
+  else if (ak) hipLaunchKernelGGL((flow_gemm_kernel<true, false>), grid, blk, 0, st_, g);
+  else if (bn) hipLaunchKernelGGL((flow_gemm_kernel<false, true>), grid, blk, 0, st_, g);
+  else hipLaunchKernelGGL((flow_gemm_kernel<false, false>), grid, blk, 0, st_, g);
   if (splits > 1) hipLaunchKernelGGL(flow_gemm_reduce, grid1((int64_t)M * N), dim3(256), 0, st_, g);
 }
 
@@ -1414,17 +1454,17 @@ void FlowNet::backward_params(int rows) {
                        S_ + (int64_t)l * R_ * Dmax_b_, ly.ib, ly.Db, D, rows, 1.0f / rows, GO_);
     // W3, b3
     gemm(h2, 1, H, GO_, Db2, 1, G + ly.off[4], Db2, H, Db2, rows, nullptr, FG_EPI_NONE, nullptr, nullptr, 0);
-    hipLaunchKernelGGL(flow_colsum, grid1(Db2), dim3(256), 0, st_, GO_, rows, Db2, G + ly.off[5]);
+    hipLaunchKernelGGL(flow_colsum, grid1(Db2, 32), dim3(256), 0, st_, GO_, rows, Db2, G + ly.off[5]);
     // GP2 = (GO W3^T)(1 - h2^2); W2, b2
     gemm(GO_, Db2, 1, P + ly.off[4], 1, Db2, GP2_, H, rows, H, Db2, nullptr, FG_EPI_DTANH, nullptr, h2, H);
     gemm(h1, 1, H, GP2_, H, 1, G + ly.off[2], H, H, H, rows, nullptr, FG_EPI_NONE, nullptr, nullptr, 0);
-    hipLaunchKernelGGL(flow_colsum, grid1(H), dim3(256), 0, st_, GP2_, rows, H, G + ly.off[3]);
+    hipLaunchKernelGGL(flow_colsum, grid1(H, 32), dim3(256), 0, st_, GP2_, rows, H, G + ly.off[3]);
     // GP1 = (GP2 W2^T)(1 - h1^2); W1 from the layer's conditioner input, b1
     gemm(GP2_, H, 1, P + ly.off[2], 1, H, GP1_, H, rows, H, H, nullptr, FG_EPI_DTANH, nullptr, h1, H);
     // W1: A(j, r) = U_[l+1][r][ia[j]] (row gather on the conditioner columns)
     gemm(U_ + (l + 1) * RD, 1, D, GP1_, H, 1, G + ly.off[0], H, ly.Da, H, rows, nullptr, FG_EPI_NONE, nullptr, nullptr,
          0, nullptr, ly.ia);
-    hipLaunchKernelGGL(flow_colsum, grid1(H), dim3(256), 0, st_, GP1_, rows, H, G + ly.off[1]);
+    hipLaunchKernelGGL(flow_colsum, grid1(H, 32), dim3(256), 0, st_, GP1_, rows, H, G + ly.off[1]);
     // cotangent of the conditioner input: GC[:, ia] += GP1 W1^T
     gemm(GP1_, H, 1, P + ly.off[0], 1, H, GC_, D, rows, ly.Da, H, nullptr, FG_EPI_ADD, nullptr, nullptr, 0, nullptr,
          nullptr, ly.ia);
