@@ -23,6 +23,14 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 #define FG_BK 64
 enum { FG_EPI_NONE = 0, FG_EPI_BIAS = 1, FG_EPI_BIAS_TANH = 2, FG_EPI_DTANH = 3, FG_EPI_ADD = 4 };
 
+// Element-wise kernels over rows x columns: 256 columns of a row per block, so the
+// row is one scalar division per block (a 64-bit division per element was most
+// of these kernels' instructions).  Launched with grid_rc(rows, columns).
+#define FLOW_RC(r, j, cols)                                  \
+  const unsigned rc_tiles_ = ((unsigned)(cols) + 255u) / 256u; \
+  const int r = (int)(blockIdx.x / rc_tiles_);               \
+  const int j = (int)(blockIdx.x % rc_tiles_) * 256 + (int)threadIdx.x
+
 struct GemmDesc {
   const float* A; int64_t sam, sak;  // A(m, k) = A[m*sam + k*sak]
   const float* B; int64_t sbk, sbn;  // B(k, n) = B[k*sbk + n*sbn]
@@ -148,27 +156,54 @@ __global__ void __launch_bounds__(256) flow_gemm_kernel(GemmDesc g) {
     }
     __syncthreads();
   }
+  // what the epilogue reads, all loads together (clamped), before the guarded stores
+  const int mb = m0 + wm + 4 * lk, nb = n0 + wn + lr;
+  const bool whole = g.splits == 1;
+  int64_t cn[2];
+  float bias[2] = {0.0f, 0.0f}, x[2][2][4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const int n = min(nb + 16 * j, g.N - 1);
+    cn[j] = whole && g.cidx_n ? g.cidx_n[n] : n;
+    if (whole && (g.epi == FG_EPI_BIAS || g.epi == FG_EPI_BIAS_TANH)) bias[j] = g.bias[n];
+  }
+  if (whole && (g.epi == FG_EPI_DTANH || g.epi == FG_EPI_ADD)) {
+    const float* src = g.epi == FG_EPI_DTANH ? g.aux : g.C;
+    const int64_t ld = g.epi == FG_EPI_DTANH ? g.ldaux : g.ldc;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const int64_t n = g.epi == FG_EPI_DTANH ? min(nb + 16 * j, g.N - 1) : cn[j];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) x[i][j][r] = src[min(mb + 16 * i + r, M - 1) * ld + n];
+      }
+  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const int m = m0 + wm + 16 * i + 4 * lk + r;
-        const int n = n0 + wn + 16 * j + lr;
+        const int m = mb + 16 * i + r, n = nb + 16 * j;
+        float v = acc[i][j][r];
+        if (whole) {
+          if (g.epi == FG_EPI_BIAS) v = v + bias[j];
+          else if (g.epi == FG_EPI_BIAS_TANH) v = tanhf(v + bias[j]);
+          else if (g.epi == FG_EPI_DTANH) v = v * (1.0f - x[i][j][r] * x[i][j][r]);
+          else if (g.epi == FG_EPI_ADD) v = x[i][j][r] + v;
+        }
         if (m < M && n < g.N) {
-          const float v = acc[i][j][r];
-          if (g.splits > 1) g.part[((int64_t)split * g.M + m) * g.N + n] = v;
-          else g.C[fg_cidx(g, m, n)] = fg_epi(g, v, m, n);
+          if (whole) g.C[(int64_t)m * g.ldc + cn[j]] = v;
+          else g.part[((int64_t)split * g.M + m) * g.N + n] = v;
         }
       }
 }
 
 __global__ void flow_gemm_reduce(GemmDesc g) {
   const int M = g.Mdev ? min(g.M, *g.Mdev) : g.M;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)M * g.N) return;
-  const int m = (int)(i / g.N), n = (int)(i % g.N);
+  FLOW_RC(m, n, g.N);
+  if (m >= M || n >= g.N) return;
   float s = 0.0f;
   // split order kept; eight loads in flight instead of one
 #pragma unroll 8
@@ -613,9 +648,9 @@ __global__ void __launch_bounds__(256) fb_in(const float* __restrict__ GP1, int 
 // U0[r][j] = Q[idx[r]][j]
 __global__ void flow_gather_z(const double* __restrict__ Q, int64_t ldq, const int* __restrict__ idx,
                               const int* __restrict__ n_dev, int n, int D, float* __restrict__ U0) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= rows_of(n_dev, n)) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= rows_of(n_dev, n)) return;
+  const int64_t i = (int64_t)r * D + j;
   const int64_t c = idx ? idx[r] : r;
   U0[i] = (float)Q[c * ldq + j];
 }
@@ -624,9 +659,9 @@ __global__ void flow_gather_z(const double* __restrict__ Q, int64_t ldq, const i
 __global__ void flow_couple_fwd(const float* __restrict__ U, const float* __restrict__ O, const int* __restrict__ ia,
                                 const int* __restrict__ ib, int Da, int Db, int D, const int* __restrict__ n_dev, int n,
                                 float* __restrict__ S, float* __restrict__ Un) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= rows_of(n_dev, n)) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= rows_of(n_dev, n)) return;
+  const int64_t i = (int64_t)r * D + j;
   const int64_t row = (int64_t)r * D;
   if (j < Da) {
     Un[row + ia[j]] = U[row + ia[j]];
@@ -643,9 +678,9 @@ __global__ void flow_couple_fwd(const float* __restrict__ U, const float* __rest
 __global__ void flow_couple_inv(const float* __restrict__ V, const float* __restrict__ O, const int* __restrict__ ia,
                                 const int* __restrict__ ib, int Da, int Db, int D, int n, float* __restrict__ S,
                                 float* __restrict__ Vn) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= n) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= n) return;
+  const int64_t i = (int64_t)r * D + j;
   const int64_t row = (int64_t)r * D;
   if (j < Da) {
     Vn[row + ia[j]] = V[row + ia[j]];
@@ -684,9 +719,9 @@ __global__ void __launch_bounds__(256) flow_logdet(const float* __restrict__ S, 
 // X = loc + scale * U (FP64 out)
 __global__ void flow_to_x(const float* __restrict__ U, const double* __restrict__ loc, const double* __restrict__ scale,
                           int D, const int* __restrict__ n_dev, int n, double* __restrict__ X) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= rows_of(n_dev, n)) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= rows_of(n_dev, n)) return;
+  const int64_t i = (int64_t)r * D + j;
   X[i] = loc[j] + scale[j] * (double)U[i];
 }
 
@@ -694,9 +729,9 @@ __global__ void flow_to_x(const float* __restrict__ U, const double* __restrict_
 __global__ void flow_standardize(const double* __restrict__ X, const int64_t* __restrict__ pick,
                                  const double* __restrict__ loc, const double* __restrict__ scale, int D, int n,
                                  float* __restrict__ V0) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= n) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= n) return;
+  const int64_t i = (int64_t)r * D + j;
   const int64_t src = pick ? pick[r] : r;
   V0[i] = (float)((X[src * D + j] - loc[j]) / scale[j]);
 }
@@ -704,9 +739,9 @@ __global__ void flow_standardize(const double* __restrict__ X, const int64_t* __
 // GC = GX * scale (cotangent of the last layer's output)
 __global__ void flow_bwd_init(const double* __restrict__ GX, const double* __restrict__ scale, int D,
                               const int* __restrict__ n_dev, int n, float* __restrict__ GC) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= rows_of(n_dev, n)) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= rows_of(n_dev, n)) return;
+  const int64_t i = (int64_t)r * D + j;
   GC[i] = (float)(GX[i] * scale[j]);
 }
 
@@ -715,9 +750,9 @@ __global__ void flow_bwd_init(const double* __restrict__ GX, const double* __res
 __global__ void flow_couple_bwd_pull(float* __restrict__ GC, const float* __restrict__ U, const float* __restrict__ S,
                                      const int* __restrict__ ib, int Db, int D, const int* __restrict__ n_dev, int n,
                                      float* __restrict__ GO) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / Db), j = (int)(i % Db);
-  if (r >= rows_of(n_dev, n)) return;
+  FLOW_RC(r, j, Db);
+  if (j >= Db || r >= rows_of(n_dev, n)) return;
+  const int64_t i = (int64_t)r * Db + j;
   const int64_t e = (int64_t)r * D + ib[j];
   const float s = S[i];
   const float es = expf(s);
@@ -734,9 +769,9 @@ __global__ void flow_couple_bwd_pull(float* __restrict__ GC, const float* __rest
 __global__ void flow_couple_bwd_train(float* __restrict__ GC, const float* __restrict__ Uz, const float* __restrict__ S,
                                       const int* __restrict__ ib, int Db, int D, int n, float inv_b,
                                       float* __restrict__ GO) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / Db), j = (int)(i % Db);
-  if (r >= n) return;
+  FLOW_RC(r, j, Db);
+  if (j >= Db || r >= n) return;
+  const int64_t i = (int64_t)r * Db + j;
   const int64_t e = (int64_t)r * D + ib[j];
   const float s = S[i];
   const float ems = expf(-s);
@@ -751,9 +786,9 @@ __global__ void flow_couple_bwd_train(float* __restrict__ GC, const float* __res
 __global__ void flow_finish(const float* __restrict__ GC, const double* __restrict__ VX,
                             const double* __restrict__ logdet, const int* __restrict__ idx, const int* __restrict__ n_dev,
                             int n, int D, double* __restrict__ G, int64_t ldg, double* __restrict__ V) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= rows_of(n_dev, n)) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= rows_of(n_dev, n)) return;
+  const int64_t i = (int64_t)r * D + j;
   const int64_t c = idx ? idx[r] : r;
   G[c * ldg + j] = (double)GC[i];
   if (j == 0) V[c] = VX[r] - logdet[r];
@@ -762,9 +797,9 @@ __global__ void flow_finish(const float* __restrict__ GC, const double* __restri
 // sampler rows: columns 7.. <- X, column 0 -= logdet
 __global__ void flow_store_rows(const double* __restrict__ X, const double* __restrict__ logdet, int n, int D,
                                 double* __restrict__ rows, int64_t ld) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int r = (int)(i / D), j = (int)(i % D);
-  if (r >= n) return;
+  FLOW_RC(r, j, D);
+  if (j >= D || r >= n) return;
+  const int64_t i = (int64_t)r * D + j;
   rows[r * ld + 7 + j] = X[i];
   if (j == 0) rows[r * ld] -= logdet[r];
 }
@@ -1026,6 +1061,7 @@ __global__ void __launch_bounds__(256) flow_bwd_persistent(FpArgs a) {
   fp_depart(a);
 }
 
+static dim3 grid_rc(int64_t rows, int64_t cols) { return dim3((unsigned)(rows * ((cols + 255) / 256))); }
 static dim3 grid1(int64_t n, int b = 256) { return dim3((unsigned)((n + b - 1) / b)); }
 
 #define HIPF(x)                                                                         \
@@ -1227,7 +1263,7 @@ void FlowNet::gemm(const float* A, int64_t sam, int64_t sak, const float* B, int
   else if (ak) hipLaunchKernelGGL((flow_gemm_kernel<true, false>), grid, blk, 0, st_, g);
   else if (bn) hipLaunchKernelGGL((flow_gemm_kernel<false, true>), grid, blk, 0, st_, g);
   else hipLaunchKernelGGL((flow_gemm_kernel<false, false>), grid, blk, 0, st_, g);
-  if (splits > 1) hipLaunchKernelGGL(flow_gemm_reduce, grid1((int64_t)M * N), dim3(256), 0, st_, g);
+  if (splits > 1) hipLaunchKernelGGL(flow_gemm_reduce, grid_rc(M, N), dim3(256), 0, st_, g);
 }
 
 // MLP of layer l on UA (rows x Da): H1, H2 of the layer, O = [s_raw, t]
@@ -1329,7 +1365,7 @@ void FlowNet::forward(const double* Q, int64_t ldq, const int* idx, const int* n
     ran_persistent_ = true;
     return;
   }
-  hipLaunchKernelGGL(flow_gather_z, grid1((int64_t)n_rows * D), dim3(256), 0, st_, Q, ldq, idx, n_dev, n_rows, D, U_);
+  hipLaunchKernelGGL(flow_gather_z, grid_rc(n_rows, D), dim3(256), 0, st_, Q, ldq, idx, n_dev, n_rows, D, U_);
   if (fused_ok(n_rows)) {
     const float* P = params_;
     const int tm = (n_rows + 63) / 64, th = (H + 63) / 64, tmax = (Dmax_b_ + 63) / 64;
@@ -1356,12 +1392,12 @@ void FlowNet::forward(const double* Q, int64_t ldq, const int* idx, const int* n
     const Layer& ly = layers_[l];
     float* U = U_ + l * RD;
     mlp(l, U, D, ly.ia, n_dev, n_rows);
-    hipLaunchKernelGGL(flow_couple_fwd, grid1((int64_t)n_rows * D), dim3(256), 0, st_, U, O_, ly.ia, ly.ib, ly.Da,
+    hipLaunchKernelGGL(flow_couple_fwd, grid_rc(n_rows, D), dim3(256), 0, st_, U, O_, ly.ia, ly.ib, ly.Da,
                        ly.Db, D, n_dev, n_rows, S_ + (int64_t)l * R_ * Dmax_b_, U + RD);
   }
   hipLaunchKernelGGL(flow_logdet, dim3(n_rows), dim3(256), 0, st_, S_, (int64_t)R_ * Dmax_b_, db_dev_, L, n_dev,
                      n_rows, log_scale_sum_, logdet, 1);
-  hipLaunchKernelGGL(flow_to_x, grid1((int64_t)n_rows * D), dim3(256), 0, st_, U_ + L * RD, loc_, scale_, D, n_dev,
+  hipLaunchKernelGGL(flow_to_x, grid_rc(n_rows, D), dim3(256), 0, st_, U_ + L * RD, loc_, scale_, D, n_dev,
                      n_rows, X);
 }
 
@@ -1377,7 +1413,7 @@ void FlowNet::pullback(const double* GX, const double* VX, const double* logdet,
     ran_persistent_ = true;
     return;
   }
-  hipLaunchKernelGGL(flow_bwd_init, grid1((int64_t)n_rows * D), dim3(256), 0, st_, GX, scale_, D, n_dev, n_rows, GC_);
+  hipLaunchKernelGGL(flow_bwd_init, grid_rc(n_rows, D), dim3(256), 0, st_, GX, scale_, D, n_dev, n_rows, GC_);
   if (fused_ok(n_rows)) {
     const float* P = params_;
     const int tm = (n_rows + 63) / 64, th = (H + 63) / 64;
@@ -1393,7 +1429,7 @@ void FlowNet::pullback(const double* GX, const double* VX, const double* logdet,
       hipLaunchKernelGGL(fb_in, dim3((ly.Da + 63) / 64, tm), dim3(256), 0, st_, GP1_, H, P + ly.off[0], ly.ia, ly.Da,
                          D, GC_, n_dev, n_rows);
     }
-    hipLaunchKernelGGL(flow_finish, grid1((int64_t)n_rows * D), dim3(256), 0, st_, GC_, VX, logdet, idx, n_dev,
+    hipLaunchKernelGGL(flow_finish, grid_rc(n_rows, D), dim3(256), 0, st_, GC_, VX, logdet, idx, n_dev,
                        n_rows, D, G, ldg, V);
     return;
   }
@@ -1402,7 +1438,7 @@ void FlowNet::pullback(const double* GX, const double* VX, const double* logdet,
     const float* P = params_;
     const float* h1 = H1_ + (int64_t)l * R_ * H;
     const float* h2 = H2_ + (int64_t)l * R_ * H;
-    hipLaunchKernelGGL(flow_couple_bwd_pull, grid1((int64_t)n_rows * ly.Db), dim3(256), 0, st_, GC_, U_ + l * RD,
+    hipLaunchKernelGGL(flow_couple_bwd_pull, grid_rc(n_rows, ly.Db), dim3(256), 0, st_, GC_, U_ + l * RD,
                        S_ + (int64_t)l * R_ * Dmax_b_, ly.ib, ly.Db, D, n_dev, n_rows, GO_);
     // GP2 = (GO W3^T) (1 - h2^2); GP1 = (GP2 W2^T) (1 - h1^2); GUA = GP1 W1^T
     gemm(GO_, 2 * ly.Db, 1, P + ly.off[4], 1, 2 * ly.Db, GP2_, H, n_rows, H, 2 * ly.Db, n_dev, FG_EPI_DTANH, nullptr,
@@ -1412,7 +1448,7 @@ void FlowNet::pullback(const double* GX, const double* VX, const double* logdet,
     gemm(GP1_, H, 1, P + ly.off[0], 1, H, GC_, D, n_rows, ly.Da, H, n_dev, FG_EPI_ADD, nullptr, nullptr, 0, nullptr,
          nullptr, ly.ia);
   }
-  hipLaunchKernelGGL(flow_finish, grid1((int64_t)n_rows * D), dim3(256), 0, st_, GC_, VX, logdet, idx, n_dev, n_rows,
+  hipLaunchKernelGGL(flow_finish, grid_rc(n_rows, D), dim3(256), 0, st_, GC_, VX, logdet, idx, n_dev, n_rows,
                      D, G, ldg, V);
 }
 
@@ -1425,7 +1461,7 @@ void FlowNet::inverse_pass(int rows) {
     const Layer& ly = layers_[l];
     const float* Vin = U_ + (l + 1) * RD;
     mlp(l, Vin, D, ly.ia, nullptr, rows);
-    hipLaunchKernelGGL(flow_couple_inv, grid1((int64_t)rows * D), dim3(256), 0, st_, Vin, O_, ly.ia, ly.ib, ly.Da,
+    hipLaunchKernelGGL(flow_couple_inv, grid_rc(rows, D), dim3(256), 0, st_, Vin, O_, ly.ia, ly.ib, ly.Da,
                        ly.Db, D, rows, S_ + (int64_t)l * R_ * Dmax_b_, U_ + l * RD);
   }
 }
@@ -1450,7 +1486,7 @@ void FlowNet::backward_params(int rows) {
     const int Db2 = 2 * ly.Db;
     const float* h1 = H1_ + (int64_t)l * R_ * H;
     const float* h2 = H2_ + (int64_t)l * R_ * H;
-    hipLaunchKernelGGL(flow_couple_bwd_train, grid1((int64_t)rows * ly.Db), dim3(256), 0, st_, GC_, U_ + l * RD,
+    hipLaunchKernelGGL(flow_couple_bwd_train, grid_rc(rows, ly.Db), dim3(256), 0, st_, GC_, U_ + l * RD,
                        S_ + (int64_t)l * R_ * Dmax_b_, ly.ib, ly.Db, D, rows, 1.0f / rows, GO_);
     // W3, b3
     gemm(h2, 1, H, GO_, Db2, 1, G + ly.off[4], Db2, H, Db2, rows, nullptr, FG_EPI_NONE, nullptr, nullptr, 0);
@@ -1474,14 +1510,14 @@ void FlowNet::backward_params(int rows) {
 void FlowNet::map_rows(double* rows, int64_t ld, int n_rows) {
   if (n_rows > R_) throw std::invalid_argument("flow: too many rows");
   forward(rows + 7, ld, nullptr, nullptr, n_rows, xrows_, rowbuf_);
-  hipLaunchKernelGGL(flow_store_rows, grid1((int64_t)n_rows * spec_.D), dim3(256), 0, st_, xrows_, rowbuf_, n_rows,
+  hipLaunchKernelGGL(flow_store_rows, grid_rc(n_rows, spec_.D), dim3(256), 0, st_, xrows_, rowbuf_, n_rows,
                      spec_.D, rows, ld);
 }
 
 void FlowNet::inverse(const double* X, int n_rows, double* Z, double* logdet) {
   if (n_rows > R_) throw std::invalid_argument("flow: too many rows");
   const int D = spec_.D, L = spec_.L;
-  hipLaunchKernelGGL(flow_standardize, grid1((int64_t)n_rows * D), dim3(256), 0, st_, X, nullptr, loc_, scale_, D,
+  hipLaunchKernelGGL(flow_standardize, grid_rc(n_rows, D), dim3(256), 0, st_, X, nullptr, loc_, scale_, D,
                      n_rows, U_ + (int64_t)L * R_ * D);
   inverse_pass(n_rows);
   hipLaunchKernelGGL(flow_rows_out, grid1((int64_t)n_rows * D), dim3(256), 0, st_, U_, (int64_t)n_rows * D, Z);
@@ -1493,7 +1529,7 @@ void FlowNet::inverse(const double* X, int n_rows, double* Z, double* logdet) {
 double FlowNet::loss_grad(const double* X, int n_rows, float* grad_host) {
   if (n_rows > R_) throw std::invalid_argument("flow: too many rows");
   const int D = spec_.D, L = spec_.L;
-  hipLaunchKernelGGL(flow_standardize, grid1((int64_t)n_rows * D), dim3(256), 0, st_, X, nullptr, loc_, scale_, D,
+  hipLaunchKernelGGL(flow_standardize, grid_rc(n_rows, D), dim3(256), 0, st_, X, nullptr, loc_, scale_, D,
                      n_rows, U_ + (int64_t)L * R_ * D);
   inverse_pass(n_rows);
   row_losses(n_rows);
@@ -1517,7 +1553,7 @@ double FlowNet::train(const double* draws, int64_t n_draws, int steps, int batch
   std::vector<double> lrow(batch);
   for (int t = 1; t <= steps; ++t) {
     hipLaunchKernelGGL(flow_pick_rows, grid1(batch), dim3(256), 0, st_, seed, (uint32_t)t, batch, n_draws, pick_);
-    hipLaunchKernelGGL(flow_standardize, grid1((int64_t)batch * D), dim3(256), 0, st_, draws, pick_, loc_, scale_, D,
+    hipLaunchKernelGGL(flow_standardize, grid_rc(batch, D), dim3(256), 0, st_, draws, pick_, loc_, scale_, D,
                        batch, U_ + (int64_t)L * R_ * D);
     inverse_pass(batch);
     backward_params(batch);
