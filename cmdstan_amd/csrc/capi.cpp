@@ -1936,6 +1936,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
     PoolSpan span(M.ws);
     DevPool* const ws = &M.ws;
     DevBuf<double> Q(ws, (size_t)C * D), G(ws, (size_t)C * D), V(ws, C), L(ws, C), work(ws);
+    bool finish = true;  // V and grad V still to be turned into lp and its gradient
     DevBuf<int> dD(ws);
     DevBuf<int64_t> doff(ws), ddso(ws);
     GlScratch gs(ws);
@@ -1945,7 +1946,9 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
         throw std::runtime_error("plugin log_prob_grad failed");
       HIPC(hipDeviceSynchronize());  // whatever stream the callback worked on
     } else if ((M.glm || (M.glm_large && (precision != 0 || M.glm_wide))) && dataset == 0) {
-      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, C, 0, M.glm_s2inv, Q.p, D, G.p, V.p, nullptr};
+      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, C, 0, M.glm_s2inv, Q.p, D, G.p, L.p, nullptr};
+      ga.sign = -1.0;
+      finish = false;
       // reduced precision: the kernel the sampler's autotuner picks for this many points
       const ModelImpl::GlmTune tn = M.glm && precision != 0 ? glm_autotune(M, C, precision, 0) : ModelImpl::GlmTune{};
       int rcg = 0;
@@ -1953,7 +1956,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
         const GlLargePlan gp = gl_large_plan(M.glmN, C, D, num_cus());
         GlLargeArgs a;
         gl_bind(M, a, gp, gs, precision, 0);
-        a.C = C; a.Q = Q.p; a.ldq = D; a.G = G.p; a.V = V.p;
+        a.C = C; a.Q = Q.p; a.ldq = D; a.G = G.p; a.V = L.p; a.sign = -1.0;
         gl_large_grad(a, gp, M.low_x(precision, 0), precision, 0);
       } else if (M.glm_wide) {
         const GlmWidePlan gp = glm_wide_plan(M.glmN, C, D, num_cus());
@@ -1977,7 +1980,9 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
       HlArgs a{};
       a.block = M.d_data.p + M.ds_off[dataset];
       a.Q = Q.p; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = C;
-      a.Gout = G.p; a.ldg = D; a.Vout = V.p; a.work = work.p; a.jac = jacobian ? 1.0 : 0.0;
+      a.Gout = G.p; a.ldg = D; a.Vout = L.p; a.work = work.p; a.jac = jacobian ? 1.0 : 0.0;
+      a.sign = -1.0;
+      finish = false;
       hl_grad_launch(a, hd.groups, hd.group_size, 0);
     } else {
       dD.alloc(C);
@@ -1989,7 +1994,8 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
       launch_model_grad(M.kind, C, dD.p, doff.p, Q.p, G.p, V.p, nullptr, md, 0);
     }
     const int64_t tot = std::max<int64_t>((int64_t)C * D, C);
-    hipLaunchKernelGGL(noalloc_finish, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, 0, V.p, L.p, G.p, C, D);
+    if (finish)
+      hipLaunchKernelGGL(noalloc_finish, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, 0, V.p, L.p, G.p, C, D);
     HIPC(hipGetLastError());
     HIPC(hipMemcpy(grad, G.p, (size_t)C * D * sizeof(double), hipMemcpyDeviceToHost));
     HIPC(hipMemcpy(lp, L.p, C * sizeof(double), hipMemcpyDeviceToHost));
@@ -2040,6 +2046,7 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
                                     std::to_string(doubles * 8) + " bytes of scratch, more than the " +
                                     std::to_string(work_cap * 8) + " available; use fewer points");
     };
+    bool finish = true;  // V and grad V still to be turned into lp and its gradient
     if (M.plugin) {
       if (M.pl.log_prob_grad(M.pl.user, d_q, D, nullptr, nullptr, n, jacobian ? 1 : 0, d_grad, V, st))
         throw std::runtime_error("plugin log_prob_grad failed");
@@ -2047,12 +2054,16 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       // the plan of nuts_log_prob_grad, so both give the same sums
       const GlmPlan gp = glm_mfma_plan(M.glmN, n, D, num_cus());
       need(gp.work_doubles);
-      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, gp.rows_per_chunk, M.glm_s2inv, d_q, D, d_grad, V, work};
+      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, gp.rows_per_chunk, M.glm_s2inv, d_q, D, d_grad, d_lp, work};
+      ga.sign = -1.0;
+      finish = false;
       if (glm_grad_mfma_f64(ga, gp, st)) throw std::runtime_error("GLM kernel: unsupported D");
     } else if (M.glm_wide && dataset == 0) {
       const GlmWidePlan gp = glm_wide_plan(M.glmN, n, D, num_cus(), work_cap);
       need(gp.work_doubles);
-      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, 0, M.glm_s2inv, d_q, D, d_grad, V, work};
+      GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, 0, M.glm_s2inv, d_q, D, d_grad, d_lp, work};
+      ga.sign = -1.0;
+      finish = false;
       if (glm_grad_wide_f64(ga, gp, st)) throw std::runtime_error("GLM kernel: unsupported D");
     } else if (M.kind == MK_HIER_LOGISTIC) {
       const Dataset& hd = M.ds[dataset];
@@ -2060,7 +2071,9 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       HlArgs a{};
       a.block = M.d_data.p + M.ds_off[dataset];
       a.Q = d_q; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = n;
-      a.Gout = d_grad; a.ldg = D; a.Vout = V; a.work = work; a.jac = jacobian ? 1.0 : 0.0;
+      a.Gout = d_grad; a.ldg = D; a.Vout = d_lp; a.work = work; a.jac = jacobian ? 1.0 : 0.0;
+      a.sign = -1.0;
+      finish = false;
       hl_grad_launch(a, hd.groups, hd.group_size, st);
     } else {
       hipLaunchKernelGGL(noalloc_tables, dim3((n + 255) / 256), dim3(256), 0, st, Dv, off, dso, n, D,
@@ -2069,7 +2082,8 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       launch_model_grad(M.kind, n, Dv, off, d_q, d_grad, V, nullptr, md, st);
     }
     const int64_t tot = std::max<int64_t>((int64_t)n * D, n);
-    hipLaunchKernelGGL(noalloc_finish, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, V, d_lp, d_grad, n, D);
+    if (finish)
+      hipLaunchKernelGGL(noalloc_finish, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, st, V, d_lp, d_grad, n, D);
     HIPC(hipGetLastError());
     return NUTS_OK;
   });

@@ -26,6 +26,7 @@ struct GlLargeArgs {
   unsigned short* Rb = nullptr;          // [3][Cp][ldn]
   const unsigned short* Xt = nullptr;    // [Dp][ldn]
   hipEvent_t ev_begin = nullptr, ev_end = nullptr;  // optional, around the two passes
+  double sign = 1.0;  // as GlmArgs::sign
 };
 
 struct GlLargePlan {

@@ -243,7 +243,7 @@ __global__ void gl_reduce(GlLargeArgs a, int splits, int row_tiles) {
     // split order kept; eight loads in flight instead of one
 #pragma unroll 8
     for (int sp = 0; sp < splits; ++sp) s += a.Wg[((int64_t)sp * a.C + pos) * a.D + k];
-    g[k] = s + a.s2inv * q[k];
+    g[k] = a.sign * (s + a.s2inv * q[k]);
   }
   if (threadIdx.x < 64) {
     double lpv = 0.0, pr = 0.0;
@@ -251,7 +251,7 @@ __global__ void gl_reduce(GlLargeArgs a, int splits, int row_tiles) {
     for (int k = threadIdx.x; k < a.D; k += 64) pr += q[k] * q[k];
     lpv = wave_sum(lpv);
     pr = wave_sum(pr);
-    if (threadIdx.x == 0) a.V[c] = -(lpv - 0.5 * a.s2inv * pr);
+    if (threadIdx.x == 0) a.V[c] = -a.sign * (lpv - 0.5 * a.s2inv * pr);
   }
 }
 

@@ -232,7 +232,7 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
 __global__ void __launch_bounds__(512)
 glm_mfma_reduce(const double* __restrict__ Wg, const double* __restrict__ Wlp, int N, int total_blocks, int C, int D,
                 double s2inv, const double* __restrict__ Q, int64_t ldq, const int* __restrict__ idx,
-                const int* __restrict__ n_active, double* __restrict__ G, double* __restrict__ V) {
+                const int* __restrict__ n_active, double sign, double* __restrict__ G, double* __restrict__ V) {
   __shared__ double red[8][64];
   const int pos = blockIdx.x;
   const int n_act = idx ? *n_active : C;
@@ -254,7 +254,7 @@ glm_mfma_reduce(const double* __restrict__ Wg, const double* __restrict__ Wlp, i
     double t = 0.0;
 #pragma unroll
     for (int v = 0; v < 8; v += 2) t += red[v][lane] + red[v + 1][lane];
-    g[k] = t + s2inv * q[k];
+    g[k] = sign * (t + s2inv * q[k]);
   }
   if (blockIdx.y == 0 && z == 1) {
     double lpv = 0.0, pr = 0.0;
@@ -262,7 +262,7 @@ glm_mfma_reduce(const double* __restrict__ Wg, const double* __restrict__ Wlp, i
     for (int i = lane; i < D; i += 64) pr += q[i] * q[i];
     lpv = wave_sum(lpv);
     pr = wave_sum(pr);
-    if (lane == 0) V[c] = -(lpv - 0.5 * s2inv * pr);
+    if (lane == 0) V[c] = -sign * (lpv - 0.5 * s2inv * pr);
   }
 }
 
@@ -370,7 +370,7 @@ void glm_reduce_launch(const GlmArgs& a, const GlmPlan& p, hipStream_t st) {
   double* Wg = a.work;
   double* Wlp = a.work + (size_t)p.total_blocks * GM_TC * a.D;
   hipLaunchKernelGGL(glm_mfma_reduce, dim3(a.C, (a.D + 63) / 64), dim3(512), 0, st, Wg, Wlp, a.N, p.total_blocks, a.C,
-                     a.D, a.s2inv, a.Q, a.ldq, a.idx, a.n_active, a.G, a.V);
+                     a.D, a.s2inv, a.Q, a.ldq, a.idx, a.n_active, a.sign, a.G, a.V);
 }
 
 }  // namespace nutsgpu

@@ -203,7 +203,7 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
       for (int t = 0; t < TW; ++t) {
         const int d = col0(t) + lr;
         if (d >= D) continue;
-        if (whole) a.G[row + d] = gacc[g][t][i] + a.s2inv * a.Q[row + d];
+        if (whole) a.G[row + d] = a.sign * (gacc[g][t][i] + a.s2inv * a.Q[row + d]);
         else Wg[(base + p) * D + d] = gacc[g][t][i];
       }
     }
@@ -251,7 +251,7 @@ glm_wide_reduce(GlmArgs a, int total_blocks, int max_chunks, int gp, const doubl
       double t = 0.0;
 #pragma unroll
       for (int y = 0; y < 8; y += 2) t += red[y][lane] + red[y + 1][lane];
-      a.G[(int64_t)c * a.ldq + k] = t + a.s2inv * q[k];
+      a.G[(int64_t)c * a.ldq + k] = a.sign * (t + a.s2inv * q[k]);
     }
   }
   if (blockIdx.y == 0 && z == 1) {
@@ -260,7 +260,7 @@ glm_wide_reduce(GlmArgs a, int total_blocks, int max_chunks, int gp, const doubl
     for (int k = lane; k < a.D; k += 64) pr += q[k] * q[k];
     lpv = wave_sum(lpv);
     pr = wave_sum(pr);
-    if (lane == 0) a.V[c] = -(lpv - 0.5 * a.s2inv * pr);
+    if (lane == 0) a.V[c] = -a.sign * (lpv - 0.5 * a.s2inv * pr);
   }
 }
 

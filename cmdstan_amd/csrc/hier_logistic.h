@@ -20,6 +20,7 @@ struct HlArgs {
   double* Vout;
   double* work;          // hl_work_doubles(G, K, n_rows)
   double jac;            // 1: add the log-Jacobian of tau = exp(v)
+  double sign = 1.0;     // Gout, Vout as they are (V = -lp), or -1: log density and its gradient
 };
 
 void hl_grad_launch(const HlArgs& a, int G, int K, hipStream_t st);

@@ -114,7 +114,7 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
     const double z = dd * it;
     const double dz = z * it;  // (beta - mu) / tau^2
     // d lp / d beta = likelihood score - (beta - mu) / tau^2
-    a.Gout[ro * a.ldg + 2 * K + (int64_t)g * K + k] = -(s - dz);
+    a.Gout[ro * a.ldg + 2 * K + (int64_t)g * K + k] = a.sign * (dz - s);
     a.work[((int64_t)k * G + g) * a.n_rows + ps] = dz;                   // d/d mu
     a.work[((int64_t)(K + k) * G + g) * a.n_rows + ps] = z * dz - it;    // d/d tau
     if (k == 0) {
@@ -160,17 +160,17 @@ __global__ void __launch_bounds__(256) hl_hyper_kernel(HlArgs a) {
   const double* q = a.Q + row_in * a.ldq;
   double* gout = a.Gout + row_out * a.ldg;
   if (j < K) {
-    gout[j] = -(s - q[j] / (mu_s * mu_s));
+    gout[j] = a.sign * (q[j] / (mu_s * mu_s) - s);
   } else if (j < 2 * K) {
     const double tau = exp(q[j]);
-    gout[j] = -(a.jac + tau * (s - tau));
+    gout[j] = -a.sign * (a.jac + tau * (s - tau));
   } else {
     double lp = s;
     for (int k = 0; k < K; ++k) {
       const double mu = q[k], v = q[K + k], tau = exp(v);
       lp += -0.5 * mu * mu / (mu_s * mu_s) - 0.5 * tau * tau + a.jac * v;
     }
-    a.Vout[row_out] = -lp;
+    a.Vout[row_out] = -a.sign * lp;
   }
 }
 

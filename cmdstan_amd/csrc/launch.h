@@ -77,6 +77,7 @@ struct GlmArgs {
   const int* n_active = nullptr;  // its length (device)
   hipEvent_t ev_begin = nullptr;  // optional events recorded around the contraction kernel alone
   hipEvent_t ev_end = nullptr;
+  double sign = 1.0;  // V and G as they are (V = -lp), or -1: log density and its gradient
 };
 
 // FP64 matrix-core version (the sampler's default for logistic regression).
