@@ -893,6 +893,11 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     throw std::invalid_argument("this model has no block-per-chain fused kernel");
   const char* fbc = std::getenv("CMDSTAN_AMD_FUSED_BLOCK_CHAINS");  // threshold override (chains still running)
   const int fused_block_chains = fbc ? std::atoi(fbc) : 2 * num_cus();
+  // The FP64 gradient kernels find the chains that wait for a gradient from the
+  // request flags themselves while one wave's ballot holds them all: a step of
+  // few chains is its launches, and compact_active is one of four (3.2 us of 24
+  // per step at 4 chains, N = 10000, D = 25).  More chains would need a scan per block.
+  const bool by_flags = C <= 64 && !R.flow && (hl_ok || gw_ok || (glm_ok && cfg.precision == 0));
   DevBuf<double> hlwork(ws);
   HlArgs hla{};
   if (hl_ok && !fused) {
@@ -901,11 +906,13 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     act_idx.alloc(C);
     n_act.alloc(1);
     hla.block = M.d_data.p + M.ds_off[R.first_dataset];
-    hla.idx = act_idx.p; hla.n_dev = n_act.p; hla.n_rows = C; hla.work = hlwork.p; hla.jac = 1.0;
+    hla.n_rows = C; hla.work = hlwork.p; hla.jac = 1.0;
     if (R.flow) {  // packed rows x = T(z) in, packed gradient out
-      hla.idx_in = false; hla.idx_out = false;
+      hla.n_dev = n_act.p;
     } else {
-      hla.Q = Q.p; hla.ldq = Dp[0]; hla.idx_in = true; hla.idx_out = true;
+      if (by_flags) hla.need = dneed.p;
+      else { hla.idx = act_idx.p; hla.n_dev = n_act.p; }
+      hla.Q = Q.p; hla.ldq = Dp[0];
       hla.Gout = G.p; hla.ldg = Dp[0]; hla.Vout = V.p;
     }
   }
@@ -955,7 +962,8 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     work.alloc(gplan.work_doubles);
     ga.X = M.d_X; ga.y = M.d_y; ga.N = M.glmN; ga.D = M.glmD; ga.C = C; ga.rows_per_chunk = gplan.rows_per_chunk;
     ga.s2inv = M.glm_s2inv; ga.Q = Q.p; ga.ldq = Dp[0]; ga.G = G.p; ga.V = V.p; ga.work = work.p;
-    ga.idx = act_idx.p; ga.n_active = n_act.p;
+    if (by_flags) ga.need = dneed.p;
+    else { ga.idx = act_idx.p; ga.n_active = n_act.p; }
     if (R.flow) {
       ga.Q = fX.p; ga.ldq = D[0]; ga.G = fGX.p; ga.V = fVX.p; ga.idx = ident.p;
     }
@@ -972,7 +980,8 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     work.alloc(gwplan.work_doubles);
     ga.X = M.d_X; ga.y = M.d_y; ga.N = M.glmN; ga.D = M.glmD; ga.C = C; ga.rows_per_chunk = 0;
     ga.s2inv = M.glm_s2inv; ga.Q = Q.p; ga.ldq = Dp[0]; ga.G = G.p; ga.V = V.p; ga.work = work.p;
-    ga.idx = act_idx.p; ga.n_active = n_act.p;
+    if (by_flags) ga.need = dneed.p;
+    else { ga.idx = act_idx.p; ga.n_active = n_act.p; }
     if (R.flow) {
       ga.Q = fX.p; ga.ldq = D[0]; ga.G = fGX.p; ga.V = fVX.p; ga.idx = ident.p;
     }
@@ -1063,7 +1072,8 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
         R.flow->pullback(fGX.p, fVX.p, fLD.p, act_idx.p, n_act.p, C, G.p, Dp[0], V.p);
         if (with_events) HIPC(hipEventRecord(ev.b[k], st));
       } else if (glm_ok || gw_ok) {
-        launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
+        if (by_flags) ga.tally = tal;
+        else launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
         ga.ev_begin = with_events ? ev.a[k] : nullptr;
         ga.ev_end = with_events ? ev.b[k] : nullptr;
         glm_grad();
@@ -1073,7 +1083,8 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
         gla.ev_end = with_events ? ev.b[k] : nullptr;
         gl_large_grad(gla, glp, xlow, cfg.precision, st);
       } else if (hl_ok) {
-        launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
+        if (by_flags) hla.tally = tal;
+        else launch_compact_active(dneed.p, C, act_idx.p, n_act.p, tal, st);
         if (with_events) HIPC(hipEventRecord(ev.a[k], st));
         hl_grad_launch(hla, hl_groups, hl_k, st);
         if (with_events) HIPC(hipEventRecord(ev.b[k], st));
@@ -1979,7 +1990,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
       work.alloc(hl_work_doubles(hd.groups, hd.group_size, C));
       HlArgs a{};
       a.block = M.d_data.p + M.ds_off[dataset];
-      a.Q = Q.p; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = C;
+      a.Q = Q.p; a.ldq = D; a.n_rows = C;
       a.Gout = G.p; a.ldg = D; a.Vout = L.p; a.work = work.p; a.jac = jacobian ? 1.0 : 0.0;
       a.sign = -1.0;
       finish = false;
@@ -2070,7 +2081,7 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       need(hl_work_doubles(hd.groups, hd.group_size, n));
       HlArgs a{};
       a.block = M.d_data.p + M.ds_off[dataset];
-      a.Q = d_q; a.ldq = D; a.idx = nullptr; a.idx_in = false; a.idx_out = false; a.n_dev = nullptr; a.n_rows = n;
+      a.Q = d_q; a.ldq = D; a.n_rows = n;
       a.Gout = d_grad; a.ldg = D; a.Vout = d_lp; a.work = work; a.jac = jacobian ? 1.0 : 0.0;
       a.sign = -1.0;
       finish = false;

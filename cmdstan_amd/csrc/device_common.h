@@ -107,6 +107,39 @@ __device__ __forceinline__ double wave_sum(double v) {
   return a[0];
 }
 
+// Positions of a batched gradient -> chains.  With the chains' request flags
+// (`need`, at most 64 chains) every wave finds them by one ballot: position p is
+// the p-th chain whose flag is set, so the launch needs no compaction kernel
+// before it.  Otherwise the list idx (null: position = row) of *n_active (null:
+// C) chains.
+struct ActiveChains {
+  int n;            // active positions
+  int chain;        // flags: the chain of position `lane`
+  bool flags;
+  const int* idx;
+  __device__ __forceinline__ ActiveChains(const int* need, const int* idx_, const int* n_active, int C)
+      : chain(0), flags(need != nullptr), idx(idx_) {
+    if (flags) {
+      const int l = threadIdx.x & 63;
+      const bool f = l < C && need[l] != 0;
+      const unsigned long long m = __ballot(f);
+      n = __popcll(m);
+      const int r = __popcll(m & ((1ull << l) - 1));  // set flags below this lane
+      chain = __builtin_amdgcn_ds_permute(4 * (f ? r : n + l - r), l);  // lane -> position, a permutation
+    } else {
+      n = n_active ? *n_active : C;
+    }
+  }
+  // chain of a position, 0 past the last one; every lane of the wave takes part
+  __device__ __forceinline__ int at(int pos) const {
+    if (flags) {
+      const int c = __shfl(chain, pos & 63, 64);
+      return pos < n ? c : 0;
+    }
+    return pos < n ? (idx ? idx[pos] : pos) : 0;
+  }
+};
+
 // and of 0/1 flags
 __device__ __forceinline__ int wave_and(int v) { return __all(v != 0) ? 1 : 0; }
 

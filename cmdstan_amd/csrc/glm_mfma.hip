@@ -60,8 +60,9 @@ __device__ __forceinline__ double gm_residual(double e, double yy, bool live, do
 template <int DT, int R, int SPLIT>
 __global__ void __launch_bounds__(256, 2)
 glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, int D, int total_blocks,
-             const double* __restrict__ Q, int64_t ldq, int C, const int* __restrict__ idx,
-             const int* __restrict__ n_active, double* __restrict__ Wg, double* __restrict__ Wlp) {
+             const double* __restrict__ Q, int64_t ldq, int C, const int* __restrict__ need,
+             const int* __restrict__ idx, const int* __restrict__ n_active, double* __restrict__ Wg,
+             double* __restrict__ Wlp) {
   constexpr int KS = 4 * DT - R;              // phase-1 steps
   constexpr int XS = 16 * DT + 2;             // LDS row stride
   constexpr int TR = SPLIT == 1 ? 32 : 16;    // rows per tile
@@ -77,7 +78,8 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
   const int lk = l >> 4;   // k index inside a 4-deep step
 
   // XCD-aware mapping: consecutive linear ids go to consecutive XCDs.
-  const int n_act = idx ? *n_active : C;
+  const ActiveChains act(need, idx, n_active, C);
+  const int n_act = act.n;
   const GlmSplit sp = glm_split(n_act, N, total_blocks);
   const int lin = blockIdx.x;
   const int xcd = lin & 7;
@@ -91,13 +93,13 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
   double qreg[KS];
   {
     const int pos = c0 + lr;
-    const int c = pos < n_act ? (idx ? idx[pos] : pos) : -1;
-    const double* qr = Q + (int64_t)(c < 0 ? 0 : c) * ldq;
+    const bool live = pos < n_act;
+    const double* qr = Q + (int64_t)act.at(pos) * ldq;
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
       const int k = 4 * ks + lk;
       const double v = qr[k < D ? k : 0];
-      qreg[ks] = c >= 0 && k < D ? v : 0.0;
+      qreg[ks] = live && k < D ? v : 0.0;
     }
   }
   d4 gacc[DT];
@@ -231,14 +233,17 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
 // per column walking all chunks took 8.0 us at 160 chunks.
 __global__ void __launch_bounds__(512)
 glm_mfma_reduce(const double* __restrict__ Wg, const double* __restrict__ Wlp, int N, int total_blocks, int C, int D,
-                double s2inv, const double* __restrict__ Q, int64_t ldq, const int* __restrict__ idx,
-                const int* __restrict__ n_active, double sign, double* __restrict__ G, double* __restrict__ V) {
+                double s2inv, const double* __restrict__ Q, int64_t ldq, const int* __restrict__ need,
+                const int* __restrict__ idx, const int* __restrict__ n_active, long long* __restrict__ tally,
+                double sign, double* __restrict__ G, double* __restrict__ V) {
   __shared__ double red[8][64];
   const int pos = blockIdx.x;
-  const int n_act = idx ? *n_active : C;
+  const ActiveChains act(need, idx, n_active, C);
+  const int n_act = act.n;
   if (pos >= n_act) return;
   const GlmSplit sp = glm_split(n_act, N, total_blocks);
-  const int c = idx ? idx[pos] : pos;
+  const int c = __builtin_amdgcn_readfirstlane(act.at(pos));
+  if (tally && pos == 0 && blockIdx.y == 0 && threadIdx.x == 0) *tally += n_act;
   const double* q = Q + (int64_t)c * ldq;
   double* g = G + (int64_t)c * ldq;
   const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
@@ -330,10 +335,10 @@ static void gm_launch(const GlmArgs& a, const GlmPlan& p, double* Wg, double* Wl
   // at most 16 points: the waves split the rows (see the top of the file)
   if (a.C <= 16)
     hipLaunchKernelGGL((glm_mfma_f64<DT, R, 4>), dim3(p.total_blocks), dim3(256), 0, st, a.X, a.y, a.N, a.D,
-                       p.total_blocks, a.Q, a.ldq, a.C, a.idx, a.n_active, Wg, Wlp);
+                       p.total_blocks, a.Q, a.ldq, a.C, a.need, a.idx, a.n_active, Wg, Wlp);
   else
     hipLaunchKernelGGL((glm_mfma_f64<DT, R, 1>), dim3(p.total_blocks), dim3(256), 0, st, a.X, a.y, a.N, a.D,
-                       p.total_blocks, a.Q, a.ldq, a.C, a.idx, a.n_active, Wg, Wlp);
+                       p.total_blocks, a.Q, a.ldq, a.C, a.need, a.idx, a.n_active, Wg, Wlp);
 }
 
 template <int DT>
@@ -370,7 +375,8 @@ void glm_reduce_launch(const GlmArgs& a, const GlmPlan& p, hipStream_t st) {
   double* Wg = a.work;
   double* Wlp = a.work + (size_t)p.total_blocks * GM_TC * a.D;
   hipLaunchKernelGGL(glm_mfma_reduce, dim3(a.C, (a.D + 63) / 64), dim3(512), 0, st, Wg, Wlp, a.N, p.total_blocks, a.C,
-                     a.D, a.s2inv, a.Q, a.ldq, a.idx, a.n_active, a.sign, a.G, a.V);
+                     a.D, a.s2inv, a.Q, a.ldq, a.need, a.idx, a.n_active, a.tally, a.sign, a.G,
+                     a.V);
 }
 
 }  // namespace nutsgpu

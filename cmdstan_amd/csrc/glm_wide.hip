@@ -67,7 +67,8 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
   const int tid = threadIdx.x;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l = tid & 63, lr = l & 15, lk = l >> 4;
-  const int n_act = a.idx ? *a.n_active : a.C;
+  const ActiveChains act(a.need, a.idx, a.n_active, a.C);
+  const int n_act = act.n;
   const GwSplit sp = gw_split(n_act, a.N, total_blocks, max_chunks, GP);
   // blocks of one row chunk (all groups) on one XCD, so X is fetched once per L2
   const int lin = blockIdx.x;
@@ -90,11 +91,12 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
 #pragma unroll
   for (int g = 0; g < NG; ++g) {
     const int pos = p0 + 16 * g + lr;
-    const int c = pos < n_act ? (a.idx ? a.idx[pos] : pos) : -1;
+    const bool live = pos < n_act;
+    const double* q = a.Q + (int64_t)act.at(pos) * a.ldq;
 #pragma unroll
     for (int ks = 0; ks < 4 * TW; ++ks) {
       const int k = col0(ks >> 2) + 4 * (ks & 3) + lk;
-      qreg[g][ks] = (c >= 0 && k < D) ? a.Q[(int64_t)c * a.ldq + k] : 0.0;
+      qreg[g][ks] = (live && k < D) ? q[k] : 0.0;
     }
   }
   d4 gacc[NG][TW];
@@ -197,8 +199,8 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int p = p0 + 16 * g + 4 * i + lk;
+      const int64_t row = whole ? (int64_t)act.at(p) * a.ldq : 0;
       if (p >= n_act) continue;
-      const int64_t row = whole ? (int64_t)(a.idx ? a.idx[p] : p) * a.ldq : 0;
 #pragma unroll
       for (int t = 0; t < TW; ++t) {
         const int d = col0(t) + lr;
@@ -231,11 +233,13 @@ __global__ void __launch_bounds__(512)
 glm_wide_reduce(GlmArgs a, int total_blocks, int max_chunks, int gp, const double* __restrict__ Wg, const double* __restrict__ Wlp) {
   __shared__ double red[8][64];
   const int pos = blockIdx.x;
-  const int n_act = a.idx ? *a.n_active : a.C;
+  const ActiveChains act(a.need, a.idx, a.n_active, a.C);
+  const int n_act = act.n;
   if (pos >= n_act) return;
   const GwSplit sp = gw_split(n_act, a.N, total_blocks, max_chunks, gp);
   const int64_t stride = gp * sp.groups;
-  const int c = a.idx ? a.idx[pos] : pos;
+  const int c = __builtin_amdgcn_readfirstlane(act.at(pos));
+  if (a.tally && pos == 0 && blockIdx.y == 0 && threadIdx.x == 0) *a.tally += n_act;
   const double* q = a.Q + (int64_t)c * a.ldq;
   const int lane = threadIdx.x & 63, z = threadIdx.x >> 6;
   if (sp.chunks > 1) {

@@ -9,11 +9,14 @@ namespace nutsgpu {
 
 struct HlArgs {
   const double* block;   // device dataset block [N, K, G, mu_s, gstart[G+1], X, y]
-  const double* Q;       // positions: row idx[pos] (idx_in) or pos, stride ldq
+  const double* Q;       // positions: row of the chain (idx or need) or of the position, stride ldq
   int64_t ldq;
-  const int* idx;        // active positions -> chains
-  bool idx_in, idx_out;  // rows of Q / of Gout and Vout are chains (true) or positions
+  const int* idx;        // active positions -> chains; null: rows are positions
   const int* n_dev;      // active count (device) or null for n_rows
+  // in place of idx, at most 64 chains: the chains' request flags (left as they
+  // are); tally (optional) accumulates their number
+  const int* need = nullptr;
+  long long* tally = nullptr;
   int n_rows;
   double* Gout;          // gradient of V = -lp, stride ldg
   int64_t ldg;

@@ -31,6 +31,7 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
   __shared__ double sX[HL_OBS * K];
   __shared__ double sY[HL_OBS];
   __shared__ double sRed[SPLIT][TC][K + 1];
+  __shared__ int sRow[TC];  // rows of the tile's points
   const double* d = a.block;
   const int G = (int)d[2];
   const double* gstart = d + 4;
@@ -39,14 +40,16 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
   const double* y = X + (int64_t)N * K;
   const int g = blockIdx.x % G;
   const int tile = blockIdx.x / G;
-  const int n_act = a.n_dev ? min(a.n_rows, *a.n_dev) : a.n_rows;
+  const ActiveChains act(a.need, a.idx, a.n_dev, a.n_rows);
+  const int n_act = min(a.n_rows, act.n);
   const int p0 = tile * TC;
   if (p0 >= n_act) return;
   const int t = threadIdx.x, w = t / TC, lane = t % TC;
   const int pos = p0 + lane;
   const bool live = pos < n_act;
-  const int64_t row_in = live ? (a.idx_in ? (int64_t)a.idx[pos] : pos) : 0;
-  const double* q = a.Q + row_in * a.ldq;
+  const int64_t row = act.at(pos);
+  if (t < TC) sRow[t] = (int)row;
+  const double* q = a.Q + row * a.ldq;
   double b[K], gb[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -103,8 +106,8 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
     const int ln = i % TC, k = i / TC;
     const int ps = p0 + ln;
     if (ps >= n_act) continue;
-    const int64_t ri = a.idx_in ? (int64_t)a.idx[ps] : ps, ro = a.idx_out ? (int64_t)a.idx[ps] : ps;
-    const double* qp = a.Q + ri * a.ldq;
+    const int64_t ro = sRow[ln];
+    const double* qp = a.Q + ro * a.ldq;
     double s = 0.0;
 #pragma unroll
     for (int ww = 0; ww < SPLIT; ++ww) s += sRed[ww][ln][k];
@@ -140,11 +143,14 @@ __global__ void __launch_bounds__(256) hl_hyper_kernel(HlArgs a) {
   const double* d = a.block;
   const int K = (int)d[1], G = (int)d[2];
   const double mu_s = d[3];
-  const int n_act = a.n_dev ? min(a.n_rows, *a.n_dev) : a.n_rows;
+  const ActiveChains act(a.need, a.idx, a.n_dev, a.n_rows);
+  const int n_act = min(a.n_rows, act.n);
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int p0 = blockIdx.x * 64, j = blockIdx.y;
   if (p0 >= n_act) return;
+  if (a.tally && p0 == 0 && j == 0 && threadIdx.x == 0) *a.tally += n_act;
   const int pos = p0 + lane;
+  const int64_t row = act.at(pos);
   double s = 0.0;
   if (pos < n_act) {
     const double* col = a.work + (int64_t)j * G * a.n_rows + pos;
@@ -155,10 +161,8 @@ __global__ void __launch_bounds__(256) hl_hyper_kernel(HlArgs a) {
   __syncthreads();
   if (w != 0 || pos >= n_act) return;
   s = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
-  const int64_t row_in = a.idx_in ? (int64_t)a.idx[pos] : pos;
-  const int64_t row_out = a.idx_out ? (int64_t)a.idx[pos] : pos;
-  const double* q = a.Q + row_in * a.ldq;
-  double* gout = a.Gout + row_out * a.ldg;
+  const double* q = a.Q + row * a.ldq;
+  double* gout = a.Gout + row * a.ldg;
   if (j < K) {
     gout[j] = a.sign * (q[j] / (mu_s * mu_s) - s);
   } else if (j < 2 * K) {
@@ -170,7 +174,7 @@ __global__ void __launch_bounds__(256) hl_hyper_kernel(HlArgs a) {
       const double mu = q[k], v = q[K + k], tau = exp(v);
       lp += -0.5 * mu * mu / (mu_s * mu_s) - 0.5 * tau * tau + a.jac * v;
     }
-    a.Vout[row_out] = -a.sign * lp;
+    a.Vout[row] = -a.sign * lp;
   }
 }
 

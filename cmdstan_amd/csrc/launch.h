@@ -75,6 +75,10 @@ struct GlmArgs {
   double* work;
   const int* idx = nullptr;       // optional compacted chain list (positions -> chains)
   const int* n_active = nullptr;  // its length (device)
+  // in place of idx, FP64 kernels and at most 64 chains: the chains' request
+  // flags (left as they are); tally (optional) accumulates their number
+  const int* need = nullptr;
+  long long* tally = nullptr;
   hipEvent_t ev_begin = nullptr;  // optional events recorded around the contraction kernel alone
   hipEvent_t ev_end = nullptr;
   double sign = 1.0;  // V and G as they are (V = -lp), or -1: log density and its gradient

@@ -1452,7 +1452,11 @@ struct NutsWave {
   __device__ void run() {
     int budget = GradFn::fused ? P.fused_budget : 1;
     for (;;) {
-      if (s.phase >= PH_PAUSED) return;
+      if (s.phase >= PH_PAUSED) {
+        // lockstep: the request flag is whole after every launch (the gradient kernels may leave it set)
+        if constexpr (!GradFn::fused) { if (tid == 0) B.need[c] = 0; converge(); }
+        return;
+      }
       const bool req = dispatch();
       if (!req) continue;
       if constexpr (!GradFn::fused) {
