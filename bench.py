@@ -567,9 +567,7 @@ def main():
         flops_per_launch = 4.0 * args.N * D * fit.grad_chains_per_launch
         ach = flops_per_launch / t / 1e12
         if args.precision == "fp64":
-            # even D runs the double-buffered LDS-copy variant
-            kname = "glm_mfma_f64_lds" if D % 2 == 0 else "glm_mfma_f64"
-            peak, nprod = PEAK_FP64_TFLOPS, 1
+            kname, peak, nprod = "glm_mfma_f64", PEAK_FP64_TFLOPS, 1
         else:
             kname, peak, nprod = reduced_kernel(args.precision, fit.tuned_path, D)
         roof = dict(bound="mfma", achieved=ach, peak=peak, unit="TFLOP/s", frac=ach / peak,
