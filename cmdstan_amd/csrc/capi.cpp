@@ -5,6 +5,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <exception>
 #include <cmath>
 #include <limits>
 #include <cstdio>
@@ -49,8 +50,9 @@ struct HipError : std::runtime_error {
 // Device workspace of a handle (a model or a flow), kept from call to call: a
 // call's buffers cost a hipMalloc and a hipFree each (tens of microseconds, and
 // hipFree waits for the device), more than a small call's kernels.  Blocks are
-// the handle's own -- one handle is used by one host thread -- and go with it;
-// at most kKeep bytes stay cached, larger buffers are freed at once.
+// the handle's own and go with it; at most kKeep bytes stay cached, larger
+// buffers are freed at once.  A block belongs to one call until its work has
+// finished, so calls of several threads on one handle share none.
 class DevPool {
  public:
   static constexpr size_t kKeep = (size_t)1 << 30;
@@ -58,14 +60,19 @@ class DevPool {
   DevPool(const DevPool&) = delete;
   DevPool& operator=(const DevPool&) = delete;
   ~DevPool() { clear(); }
-  // Around a call's use.  A call that left by an exception may have work in
-  // flight on its buffers: the next one waits for the device first.
+  // Around a call's use.  A call that left early may have work in flight on its
+  // buffers: the next one waits for the device first.
   void begin() {
+    std::lock_guard<std::mutex> lock(mu_);
     if (open_) (void)hipDeviceSynchronize();
     open_ = true;
   }
-  void end() { open_ = false; }
+  void end() {
+    std::lock_guard<std::mutex> lock(mu_);
+    open_ = false;
+  }
   void* get(size_t bytes, size_t* got) {
+    std::lock_guard<std::mutex> lock(mu_);
     size_t best = free_.size();
     for (size_t i = 0; i < free_.size(); ++i)
       if (free_[i].n >= bytes && free_[i].n <= 2 * bytes + 65536 && (best == free_.size() || free_[i].n < free_[best].n))
@@ -88,7 +95,9 @@ class DevPool {
     return p;
   }
   void put(void* p, size_t n) {
-    if (held_ + n > kKeep) {
+    std::lock_guard<std::mutex> lock(mu_);
+    // on the way out of an exception work may be in flight: hipFree waits for it
+    if (held_ + n > kKeep || std::uncaught_exceptions() > 0) {
       (void)hipFree(p);
       return;
     }
@@ -103,6 +112,7 @@ class DevPool {
     free_.clear();
     held_ = 0;
   }
+  std::mutex mu_;
   std::vector<Block> free_;
   size_t held_ = 0;
   bool open_ = false;
