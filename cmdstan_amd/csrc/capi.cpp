@@ -277,10 +277,10 @@ struct ModelImpl {
 // residuals as three BF16 terms; CMDSTAN_AMD_GL_BF16=0 keeps them on FP32
 // matrix cores.
 struct GlScratch {
-  DevBuf<float> qf, r;
+  DevBuf<float> qf, r, wg;
   DevBuf<unsigned short> qb, rb;
-  DevBuf<double> wg, wlp;
-  explicit GlScratch(DevPool* p) : qf(p), r(p), qb(p), rb(p), wg(p), wlp(p) {}
+  DevBuf<double> wlp;
+  explicit GlScratch(DevPool* p) : qf(p), r(p), wg(p), qb(p), rb(p), wlp(p) {}
 };
 bool gl_bf16_enabled(int precision, int D) {
   if (precision != 2 || !gl_large_bf16_ok(D)) return false;
@@ -288,7 +288,7 @@ bool gl_bf16_enabled(int precision, int D) {
   return !e || std::atoi(e) != 0;
 }
 void gl_bind(ModelImpl& M, GlLargeArgs& a, const GlLargePlan& p, GlScratch& s, int precision, hipStream_t st) {
-  s.wg.alloc(p.wg_doubles);
+  s.wg.alloc(p.wg_floats);
   s.wlp.alloc(p.wlp_doubles);
   a.y = M.d_y; a.N = M.glmN; a.D = M.glmD; a.s2inv = M.glm_s2inv;
   a.Wg = s.wg.p; a.Wlp = s.wlp.p; a.Dq = p.Dq; a.ldr = p.ldr;

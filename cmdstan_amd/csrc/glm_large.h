@@ -18,7 +18,7 @@ struct GlLargeArgs {
   const int* n_active = nullptr;
   float* Qf = nullptr; int Dq = 0;       // packed FP32 positions [C][Dq]
   float* R = nullptr; int64_t ldr = 0;   // residuals [N][ldr]
-  double* Wg = nullptr;                  // [splits][C][D]
+  float* Wg = nullptr;                   // [splits][C][D], each value the FP32 sum it was formed as
   double* Wlp = nullptr;                 // [row tiles][C]
   // BF16 matrix-core variant (X stored in BF16): positions and residuals as
   // three BF16 terms, and X transposed [Dp][ldn]
@@ -32,7 +32,7 @@ struct GlLargeArgs {
 struct GlLargePlan {
   int row_tiles = 0, Dq = 0, splits = 0, rows_per_split = 0;
   int64_t ldr = 0;
-  size_t r_floats = 0, q_floats = 0, wg_doubles = 0, wlp_doubles = 0;
+  size_t r_floats = 0, q_floats = 0, wg_floats = 0, wlp_doubles = 0;
   // BF16 variant: rows padded to whole 128-row tiles (ldn), chains to whole
   // 128-chain tiles (Cp), coefficients to 64 (Dk, pass-1 K) and 128 (Dp)
   int64_t ldn = 0;

@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(256) gl_grad_kernel(GlLargeArgs a, const XT* _
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wr + 16 * i + 4 * (l >> 4) + r;  // chain position
         const int n = n0 + wc + 16 * j + (l & 15);           // coefficient
-        if (m < n_act && n < a.D) a.Wg[((int64_t)sp * a.C + m) * a.D + n] = (double)acc[i][j][r];
+        if (m < n_act && n < a.D) a.Wg[((int64_t)sp * a.C + m) * a.D + n] = acc[i][j][r];
       }
 }
 
@@ -238,15 +238,20 @@ __global__ void gl_reduce(GlLargeArgs a, int splits, int row_tiles) {
   const int c = a.idx ? a.idx[pos] : pos;
   const double* q = a.Q + (int64_t)c * a.ldq;
   double* g = a.G + (int64_t)c * a.ldq;
-  for (int k = threadIdx.x; k < a.D; k += blockDim.x) {
+  // a block per 256 columns of a position, its last block the log density: as one
+  // block's loop the columns' and the log density's waits added up (D = 1000,
+  // 512 points: 21.4 -> 14.6 us; 23.7 when the partials were FP64)
+  if (blockIdx.y + 1 < gridDim.y) {
+    const int k = blockIdx.y * 256 + threadIdx.x;
+    if (k >= a.D) return;
     double s = 0.0;
     // split order kept; eight loads in flight instead of one
 #pragma unroll 8
-    for (int sp = 0; sp < splits; ++sp) s += a.Wg[((int64_t)sp * a.C + pos) * a.D + k];
+    for (int sp = 0; sp < splits; ++sp) s += (double)a.Wg[((int64_t)sp * a.C + pos) * a.D + k];
     g[k] = a.sign * (s + a.s2inv * q[k]);
-  }
-  if (threadIdx.x < 64) {
+  } else if (threadIdx.x < 64) {
     double lpv = 0.0, pr = 0.0;
+#pragma unroll 8
     for (int rt = threadIdx.x; rt < row_tiles; rt += 64) lpv += a.Wlp[(int64_t)rt * a.C + pos];
     for (int k = threadIdx.x; k < a.D; k += 64) pr += q[k] * q[k];
     lpv = wave_sum(lpv);
@@ -272,7 +277,7 @@ GlLargePlan gl_large_plan(int N, int C, int D, int num_cus) {
   p.ldr = (C + 3) / 4 * 4;
   p.r_floats = (size_t)N * p.ldr;
   p.q_floats = (size_t)C * p.Dq;
-  p.wg_doubles = (size_t)p.splits * C * D;
+  p.wg_floats = (size_t)p.splits * C * D;
   p.wlp_doubles = (size_t)p.row_tiles * C;
   p.Cp = (C + GL_BM - 1) / GL_BM * GL_BM;
   p.Dk = (D + 63) / 64 * 64;
@@ -305,7 +310,7 @@ void gl_large_grad(const GlLargeArgs& a, const GlLargePlan& p, const void* X, in
 }
 
 void gl_reduce_launch(const GlLargeArgs& a, const GlLargePlan& p, hipStream_t st) {
-  hipLaunchKernelGGL(gl_reduce, dim3(a.C), dim3(128), 0, st, a, p.splits, p.row_tiles);
+  hipLaunchKernelGGL(gl_reduce, dim3(a.C, (a.D + 255) / 256 + 1), dim3(256), 0, st, a, p.splits, p.row_tiles);
 }
 
 }  // namespace nutsgpu

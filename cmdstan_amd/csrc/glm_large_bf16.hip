@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(256, 2) gbl_grad_kernel(GlLargeArgs a, GlLarge
       for (int r = 0; r < 4; ++r) {
         const int m = m0 + wr + 16 * i + 4 * (l >> 4) + r;  // chain position
         const int n = n0 + wc + 16 * j + (l & 15);           // coefficient
-        if (m < n_act && n < a.D) a.Wg[((int64_t)sp * a.C + m) * a.D + n] = (double)acc[i][j][r];
+        if (m < n_act && n < a.D) a.Wg[((int64_t)sp * a.C + m) * a.D + n] = acc[i][j][r];
       }
 }
 
