@@ -75,3 +75,19 @@ def test_wide_transition_replay(driver):
         qo, io = o.transition_replay(q0[k], u[k], z[k], 0.05, metric=1, minv=np.ones(150))
         assert (info[k]["depth"], info[k]["n_leapfrog"]) == (io["depth"], io["n_leapfrog"])
         assert np.allclose(q[k], qo, rtol=1e-10, atol=1e-12)
+
+
+@pytest.mark.parametrize("N,D", [(10000, 500), (3000, 200)])
+def test_wide_gradient_against_extended_precision(N, D):
+    """The error against 80-bit sums is no larger than that of the same closed form in 64 bits."""
+    d = logistic(seed=11, N=N, D=D)
+    rng = np.random.default_rng(4)
+    q = np.linalg.lstsq(d["X"], 3.0 * (d["y"] - 0.5), rcond=None)[0] + np.sqrt(5.0 / N) * rng.standard_normal((4, D))
+    X, Q = d["X"].astype(np.longdouble), q.astype(np.longdouble)
+    eta = X @ Q.T
+    g_ext = (X.T @ (d["y"][:, None] - 1 / (1 + np.exp(-eta)))).T - Q / np.longdouble(6.25)
+    _, g = ca.Model("logistic_regression", d).log_prob_grad(q)
+    g64 = _closed_form(d, q)[1]
+    err, err64 = (float(np.linalg.norm(v - g_ext) / np.linalg.norm(g_ext)) for v in (g, g64))
+    print(f"error {err:.2e}, in 64 bits {err64:.2e}")
+    assert err <= err64
