@@ -1790,8 +1790,9 @@ int nuts_sample(nuts_model* m, const nuts_config* cfg, const double* init, const
     RunResult r = cfg->flow ? run_with_flow(m->impl, R, rep) : run_batch(m->impl, R);
     const int C = (int)r.st.size();
     if (out) {
-      // vectors that are not empty: results of an earlier phase of a flow run
-      if (out->draws && !r.draws.empty()) std::memcpy(out->draws, r.draws.data(), r.draws.size() * sizeof(double));
+      // The run wrote its rows into out->draws.  A flow run whose plain phase fails ends
+      // with that phase, whose rows and columns are not the requested ones: the
+      // caller's array stays as it was; the metric has the caller's size.
       int64_t moff = 0;
       for (int c = 0; c < C; ++c) {
         const ChainState& s = r.st[c];

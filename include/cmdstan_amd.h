@@ -202,7 +202,8 @@ int nuts_output_rows(const nuts_config* cfg);
  * dataset, num_chains per dataset; chain k of dataset m is chain m*num_chains+k.
  *   draws:     chains back to back, each rows x (7 + num_outputs of its dataset):
  *              lp__, accept_stat__, stepsize__, treedepth__, n_leapfrog__,
- *              divergent__, energy__, then the constrained parameters
+ *              divergent__, energy__, then the constrained parameters (left as it
+ *              was when the plain phase of a flow run fails)
  *   stepsize:  [chains] adapted (or given) step size
  *   inv_metric:[chains] blocks of D (diag_e/unit_e) or D*D (dense_e)
  *   n_leapfrog:[chains] total leapfrog steps; grad_evals: [chains] all gradient
