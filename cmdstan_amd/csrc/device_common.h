@@ -153,20 +153,26 @@ __device__ __forceinline__ double recip_small(double d) {
   return __builtin_fma(x, __builtin_fma(-d, x, 1.0), x);
 }
 
-// Sum of log(1 + t) over many t in [0, 1] as the logarithm of their product: a
-// multiplication per term and one logarithm at the end.  fold() after at most
-// 900 terms keeps the mantissa in range.  Each factor and product rounds by
-// 1e-16 of itself, so the sum is off by about 2e-16 per term, below the rounding
-// of adding the terms up one by one.
+// Sum of log(1 + t) over many t in [0, 1] as the logarithm of their product: one
+// fused multiply-add per term and one logarithm at the end.  u is the product
+// minus one, (1 + u)(1 + t) - 1 = u (1 + t) + t, so a t far below the rounding
+// of 1 counts in full; fold() after at most 900 terms brings 1 + u back into
+// [1, 2) (u stays as it is while it is below 1).  Every operand is positive and
+// rounds by 2^-53 of itself, so after n terms u, and with it log1p(u), is off by
+// at most n 2^-52 of itself: like adding up n logarithms, measured no worse
+// than 5e-15 (sum 5e-15) for 3000 terms up to |eta| = 10 and 2e-14 (sum 1e-14)
+// at 50.  The product of the rounded 1 + t itself loses what of t lies below
+// 2^-53: 1e-13 of the sum at |eta| = 10, all of it above 37.
 struct LogProduct {
-  double m = 1.0;
+  double u = 0.0;
   int e = 0;
-  __device__ __forceinline__ void times(double one_plus_t) { m *= one_plus_t; }
+  __device__ __forceinline__ void times(double t, double one_plus_t) { u = __builtin_fma(u, one_plus_t, t); }
   __device__ __forceinline__ void fold() {
-    e += __builtin_amdgcn_frexp_exp(m);
-    m = __builtin_amdgcn_frexp_mant(m);
+    const int x = __builtin_amdgcn_frexp_exp(1.0 + u) - 1;
+    e += x;
+    u = __builtin_amdgcn_ldexp(u, -x) + (__builtin_amdgcn_ldexp(1.0, -x) - 1.0);
   }
-  __device__ __forceinline__ double log_value() const { return log(m) + (double)e * 0.69314718055994531; }
+  __device__ __forceinline__ double log_value() const { return log1p(u) + (double)e * 0.69314718055994531; }
 };
 
 __device__ __forceinline__ double log1p_exp(double a) {

@@ -53,7 +53,7 @@ __device__ __forceinline__ double gm_residual(double e, double yy, bool live, do
   const double d = 1.0 + t;
   const double r = (e >= 0.0 ? 1.0 : t) * recip_small(d) - yy;
   lp += live ? yy * e - (e > 0.0 ? e : 0.0) : 0.0;
-  lg.times(live ? d : 1.0);
+  if (live) lg.times(t, d);
   return live ? r : 0.0;
 }
 
@@ -107,6 +107,7 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
   for (int t = 0; t < DT; ++t) gacc[t] = d4{0, 0, 0, 0};
   double lp = 0.0;
   LogProduct lg;
+  int tile = 0;
   const int n_begin = chunk * sp.rows;
   const int n_end = min(N, n_begin + sp.rows);
 
@@ -170,7 +171,6 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
         const int rr = 16 * rb + 4 * i + lk;
         eta[rb][i] = gm_residual(eta[rb][i], sy[rr], nb + roff + rr < n_end, lp, lg);
       }
-    lg.fold();
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
@@ -181,6 +181,7 @@ glm_mfma_f64(const double* __restrict__ X, const double* __restrict__ y, int N, 
           gacc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(eta[rb][i], xrow[16 * t], gacc[t], 0, 0, 0);
       }
     if (more) {
+      if (++tile % 64 == 0) lg.fold();   // at most 512 factors since the last
       if constexpr (SPLIT == 1) b ^= 1;  // the other buffer: its readers passed this iteration's barrier
       else {
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");

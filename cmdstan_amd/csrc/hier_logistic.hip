@@ -87,15 +87,15 @@ __global__ void __launch_bounds__(256) hl_group_kernel(HlArgs a) {
       const double s2 = yy2 - (e2 >= 0.0 ? 1.0 : t2) * recip_small(d2);
       const double r2 = two ? s2 : 0.0;
       lp += yy * e - (e > 0.0 ? e : 0.0);
-      lg.times(d1);
+      lg.times(t1, d1);
       if (two) {
         lp += yy2 * e2 - (e2 > 0.0 ? e2 : 0.0);
-        lg.times(d2);
+        lg.times(t2, d2);
       }
 #pragma unroll
       for (int k = 0; k < K; ++k) gb[k] += r * x1[k] + r2 * x2[k];
     }
-    lg.fold();  // at most 2 HL_OBS / (2 SPLIT) factors since the last
+    lg.fold();  // at most HL_OBS / SPLIT factors since the last
   }
   // combine the partial sums of the observation split
 #pragma unroll
