@@ -233,42 +233,59 @@ struct ModelImpl {
   // caller-supplied model (nuts_model_create_plugin)
   bool plugin = false;
   nuts_model_plugin pl{};
-  DevBuf<unsigned char> xlow;  // X converted to FP32 or BF16 (lazily)
-  int xlow_prec = 0;
-  DevBuf<unsigned short> xbf;  // X as BF16 terms for the BF16-split kernel (lazily)
-  int xbf_prec = 0;
-  const unsigned short* bf16_x(int precision, hipStream_t st) {
+  // Tuning results and converted copies of X, made by the first call that needs
+  // them: one thread at a time.  A copy of another precision takes the place of
+  // the one kept; a call holds its own copy until its work has finished, so a
+  // call beside it on another precision frees nothing it reads.
+  std::mutex tune_mu;
+  std::recursive_mutex x_mu;
+  using XCopy = std::shared_ptr<const void>;
+  XCopy xlow, xbf;  // X in FP32 or BF16; X as BF16 terms for the BF16-split kernel
+  int xlow_prec = 0, xbf_prec = 0;
+  template <class T>
+  static XCopy x_copy(std::shared_ptr<DevBuf<T>> b) { return XCopy(b, b->p); }
+  XCopy bf16_x(int precision, hipStream_t st) {
+    std::lock_guard<std::recursive_mutex> lock(x_mu);
     if (xbf_prec != precision) {
+      xbf.reset();
+      xbf_prec = 0;
       const int64_t n = (int64_t)glmN * glm_bf16_ldx(glmD);
-      xbf.alloc((size_t)n * (precision == 1 ? 3 : 1));
-      glm_bf16_prepare_x(d_X, glmN, glmD, precision, xbf.p, st);
+      auto b = std::make_shared<DevBuf<unsigned short>>((size_t)n * (precision == 1 ? 3 : 1));
+      glm_bf16_prepare_x(d_X, glmN, glmD, precision, b->p, st);
       HIPC(hipStreamSynchronize(st));
+      xbf = x_copy(b);
       xbf_prec = precision;
     }
-    return xbf.p;
+    return xbf;
   }
-  const void* low_x(int precision, hipStream_t st) {
+  XCopy low_x(int precision, hipStream_t st) {
+    std::lock_guard<std::recursive_mutex> lock(x_mu);
     if (xlow_prec != precision) {
+      xlow.reset();
+      xlow_prec = 0;
       const int64_t n = (int64_t)glmN * glmD;
-      xlow.alloc((size_t)n * (precision == 1 ? 4 : 2));
-      glm_convert_x(d_X, xlow.p, n, precision, st);
+      auto b = std::make_shared<DevBuf<unsigned char>>((size_t)n * (precision == 1 ? 4 : 2));
+      glm_convert_x(d_X, b->p, n, precision, st);
       HIPC(hipStreamSynchronize(st));
+      xlow = x_copy(b);
       xlow_prec = precision;
     }
-    return xlow.p;
+    return xlow;
   }
   // BF16 X transposed [Dp][ldn] for pass 2 of the BF16 large-D kernels (made
   // once from the BF16 X, kept beside it: both fit HBM many times over)
-  DevBuf<unsigned short> xt;
+  std::unique_ptr<DevBuf<unsigned short>> xt;
   const unsigned short* bf16_xt(hipStream_t st) {
-    if (!xt.p) {
+    std::lock_guard<std::recursive_mutex> lock(x_mu);
+    if (!xt) {
       const GlLargePlan gp = gl_large_plan(glmN, 1, glmD, 0);
-      const unsigned short* xb = static_cast<const unsigned short*>(low_x(2, st));
-      xt.alloc(gp.xt_elems);
-      gl_large_prepare_xt(xb, glmN, glmD, xt.p, gp, st);
+      const XCopy xb = low_x(2, st);
+      auto b = std::make_unique<DevBuf<unsigned short>>(gp.xt_elems);
+      gl_large_prepare_xt(static_cast<const unsigned short*>(xb.get()), glmN, glmD, b->p, gp, st);
       HIPC(hipStreamSynchronize(st));
+      xt = std::move(b);
     }
-    return xt.p;
+    return xt->p;
   }
 };
 
@@ -566,12 +583,13 @@ __global__ void resume_kernel(ChainState* st, int C) {
 // blocks per CU, and for FP32/BF16 the two-pass kernels.
 ModelImpl::GlmTune glm_autotune(ModelImpl& M, int C, int precision, hipStream_t st) {
   const auto key = std::make_pair(C, precision);
+  std::lock_guard<std::mutex> lock(M.tune_mu);
   auto it = M.glm_tune.find(key);
   if (it != M.glm_tune.end()) return it->second;
   const int N = M.glmN, D = M.glmD, Dp = (D + 15) / 16 * 16;
   DevBuf<double> Q((size_t)C * Dp), G((size_t)C * Dp), V(C);
   HIPC(hipMemsetAsync(Q.p, 0, (size_t)C * Dp * sizeof(double), st));
-  const void* xl = precision ? M.low_x(precision, st) : nullptr;
+  const ModelImpl::XCopy xl = precision ? M.low_x(precision, st) : nullptr;
   hipEvent_t e0, e1;
   HIPC(hipEventCreate(&e0));
   HIPC(hipEventCreate(&e1));
@@ -593,12 +611,13 @@ ModelImpl::GlmTune glm_autotune(ModelImpl& M, int C, int precision, hipStream_t 
     GlmArgs ga{M.d_X, M.d_y, N, D, C, gp.rows_per_chunk, M.glm_s2inv, Q.p, Dp, G.p, V.p, work.p};
     const double ms = time_it([&]() {
       if (precision == 0) glm_grad_mfma_f64(ga, gp, st);
-      else glm_grad_mfma_f32(ga, gp, xl, precision, kF32Layout, st);
+      else glm_grad_mfma_f32(ga, gp, xl.get(), precision, kF32Layout, st);
     });
     if (ms < best.ms) { best.ms = ms; best.path = 0; best.blocks_per_cu = bpc; }
   }
   if (precision != 0) {
-    const unsigned short* xb = M.bf16_x(precision, st);
+    const ModelImpl::XCopy xbc = M.bf16_x(precision, st);
+    const auto* xb = static_cast<const unsigned short*>(xbc.get());
     for (int bpc = 1; bpc <= 4; ++bpc) {
       const GlmPlan gp = glm_mfma_plan(N, C, D, num_cus(), bpc);
       DevBuf<double> work(gp.work_doubles);
@@ -611,7 +630,7 @@ ModelImpl::GlmTune glm_autotune(ModelImpl& M, int C, int precision, hipStream_t 
     GlLargeArgs a;
     gl_bind(M, a, gp, gs, precision, st);
     a.C = C; a.Q = Q.p; a.ldq = Dp; a.G = G.p; a.V = V.p;
-    const double ms = time_it([&]() { gl_large_grad(a, gp, xl, precision, st); });
+    const double ms = time_it([&]() { gl_large_grad(a, gp, xl.get(), precision, st); });
     if (ms < best.ms) { best.ms = ms; best.path = 1; }
   }
   (void)hipEventDestroy(e0);
@@ -875,6 +894,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
 
   DevBuf<double> work(ws);
   DevBuf<int> act_idx(ws), n_act(ws);
+  ModelImpl::XCopy xcopy;  // the copy of X this run reads
   const void* xlow = nullptr;
   const unsigned short* xbf = nullptr;  // BF16 terms of X (path 2)
   GlmArgs ga;
@@ -963,7 +983,8 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     if (R.flow) {
       gla.Q = fX.p; gla.ldq = D[0]; gla.G = fGX.p; gla.V = fVX.p; gla.idx = ident.p;
     }
-    xlow = M.low_x(cfg.precision, st);
+    xcopy = M.low_x(cfg.precision, st);
+    xlow = xcopy.get();
   }
   if (!fused && glm_ok) {
     act_idx.alloc(C);
@@ -978,8 +999,9 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
       ga.Q = fX.p; ga.ldq = D[0]; ga.G = fGX.p; ga.V = fVX.p; ga.idx = ident.p;
     }
     if (cfg.precision != 0) {
-      if (tune.path == 2) xbf = M.bf16_x(cfg.precision, st);
-      else xlow = M.low_x(cfg.precision, st);
+      xcopy = tune.path == 2 ? M.bf16_x(cfg.precision, st) : M.low_x(cfg.precision, st);
+      if (tune.path == 2) xbf = static_cast<const unsigned short*>(xcopy.get());
+      else xlow = xcopy.get();
     }
   }
   GlmWidePlan gwplan;
@@ -1962,6 +1984,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
     DevBuf<int> dD(ws);
     DevBuf<int64_t> doff(ws), ddso(ws);
     GlScratch gs(ws);
+    ModelImpl::XCopy x;  // the copy of X this call reads
     Q.upload(q, (size_t)C * D);
     if (M.plugin) {
       if (M.pl.log_prob_grad(M.pl.user, Q.p, D, nullptr, nullptr, C, jacobian ? 1 : 0, G.p, V.p, nullptr))
@@ -1979,7 +2002,8 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
         GlLargeArgs a;
         gl_bind(M, a, gp, gs, precision, 0);
         a.C = C; a.Q = Q.p; a.ldq = D; a.G = G.p; a.V = L.p; a.sign = -1.0;
-        gl_large_grad(a, gp, M.low_x(precision, 0), precision, 0);
+        x = M.low_x(precision, 0);
+        gl_large_grad(a, gp, x.get(), precision, 0);
       } else if (M.glm_wide) {
         const GlmWidePlan gp = glm_wide_plan(M.glmN, C, D, num_cus());
         work.alloc(gp.work_doubles);
@@ -1990,9 +2014,10 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
         work.alloc(gp.work_doubles);
         ga.work = work.p;
         ga.rows_per_chunk = gp.rows_per_chunk;
+        if (precision != 0) x = tn.path == 2 ? M.bf16_x(precision, 0) : M.low_x(precision, 0);
         rcg = precision == 0 ? glm_grad_mfma_f64(ga, gp, 0)
-              : tn.path == 2 ? glm_grad_mfma_bf16(ga, gp, M.bf16_x(precision, 0), precision, 0)
-                             : glm_grad_mfma_f32(ga, gp, M.low_x(precision, 0), precision, kF32Layout, 0);
+              : tn.path == 2 ? glm_grad_mfma_bf16(ga, gp, static_cast<const unsigned short*>(x.get()), precision, 0)
+                             : glm_grad_mfma_f32(ga, gp, x.get(), precision, kF32Layout, 0);
       }
       if (rcg) throw std::runtime_error("GLM kernel: unsupported D");
     } else if (M.kind == MK_HIER_LOGISTIC) {
