@@ -2139,6 +2139,8 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
 // ------------------------------------------------------------------ flow
 struct nuts_flow {
   DevPool ws;  // workspace of this handle's calls
+  // the net's activations and parameters are the handle's own: one call at a time
+  mutable std::mutex mu;
   std::unique_ptr<FlowNet> net;
 };
 
@@ -2161,15 +2163,27 @@ void nuts_flow_destroy(nuts_flow* f) { delete f; }
 int64_t nuts_flow_num_params(const nuts_flow* f) { return f ? f->net->num_params() : -1; }
 
 int nuts_flow_get_params(const nuts_flow* f, float* out) {
-  return guarded([&]() { f->net->get_params(out); return NUTS_OK; });
+  return guarded([&]() {
+    std::lock_guard<std::mutex> lock(f->mu);
+    f->net->get_params(out);
+    return NUTS_OK;
+  });
 }
 
 int nuts_flow_set_params(nuts_flow* f, const float* in) {
-  return guarded([&]() { f->net->set_params(in); return NUTS_OK; });
+  return guarded([&]() {
+    std::lock_guard<std::mutex> lock(f->mu);
+    f->net->set_params(in);
+    return NUTS_OK;
+  });
 }
 
 int nuts_flow_set_standardization(nuts_flow* f, const double* loc, const double* scale) {
-  return guarded([&]() { f->net->set_standardization(loc, scale); return NUTS_OK; });
+  return guarded([&]() {
+    std::lock_guard<std::mutex> lock(f->mu);
+    f->net->set_standardization(loc, scale);
+    return NUTS_OK;
+  });
 }
 
 static void flow_rows_check(const nuts_flow* f, int n) {
@@ -2182,6 +2196,7 @@ int nuts_flow_forward(nuts_flow* f, const double* z, int n, double* x, double* l
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
+    std::lock_guard<std::mutex> lock(f->mu);
     PoolSpan span(f->ws);
     DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dl(&f->ws, n);
     dz.upload(z, (size_t)n * D, st);
@@ -2200,6 +2215,7 @@ int nuts_flow_inverse(nuts_flow* f, const double* x, int n, double* z, double* l
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
+    std::lock_guard<std::mutex> lock(f->mu);
     PoolSpan span(f->ws);
     DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dl(&f->ws, n);
     dx.upload(x, (size_t)n * D, st);
@@ -2217,6 +2233,7 @@ int nuts_flow_pullback_grad(nuts_flow* f, const double* z, const double* gx, int
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
+    std::lock_guard<std::mutex> lock(f->mu);
     PoolSpan span(f->ws);
     DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dgx(&f->ws, (size_t)n * D), dgz(&f->ws, (size_t)n * D), dl(&f->ws, n), dvx(&f->ws, n), dv(&f->ws, n);
     dz.upload(z, (size_t)n * D, st);
@@ -2237,6 +2254,7 @@ int nuts_flow_loss_grad(nuts_flow* f, const double* x, int n, double* loss, floa
     flow_rows_check(f, n);
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
+    std::lock_guard<std::mutex> lock(f->mu);
     PoolSpan span(f->ws);
     DevBuf<double> dx(&f->ws, (size_t)n * D);
     dx.upload(x, (size_t)n * D, st);
@@ -2254,6 +2272,7 @@ int nuts_flow_train(nuts_flow* f, const double* x, int64_t n, int steps, int bat
       throw std::invalid_argument("flow: bad training arguments");
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
+    std::lock_guard<std::mutex> lock(f->mu);
     PoolSpan span(f->ws);
     DevBuf<double> dx(&f->ws, (size_t)n * D);
     dx.upload(x, (size_t)n * D, st);

@@ -1,11 +1,12 @@
 """Calls of several threads on one handle that build or share the handle's own state: the converted
-copies of X and the tuning results of reduced-precision calls."""
+copies of X and the tuning results of reduced-precision calls, a flow's activations."""
 import threading
 
 import numpy as np
 import pytest
 
 import cmdstan_amd as ca
+from cmdstan_amd.sampler import Flow
 from tests.model_cases import EIGHT, logistic
 
 pytestmark = pytest.mark.gpu
@@ -56,3 +57,15 @@ def test_sampling_shares_a_handle():
     jobs = [(lambda s=s: m.sample(seed=s, **opts).draws, m.sample(seed=s, **opts).draws) for s in (1, 2)]
     jobs.append((lambda: m.log_prob_grad(q), m.log_prob_grad(q)))
     assert run_together(jobs, 5) == []
+
+
+def test_threads_share_a_flow():
+    D, n = 37, 20
+    f = Flow(D, n_layers=4, hidden=16, max_rows=32)
+    rng = np.random.default_rng(3)
+    f.set_params(f.get_params() + 0.05 * rng.standard_normal(f.n_params).astype(np.float32))
+    z, gx = rng.standard_normal((4, n, D)), rng.standard_normal((n, D))
+    calls = [lambda: f.forward(z[0]), lambda: f.inverse(z[1]), lambda: (f.pullback_grad(z[2], gx),),
+             lambda: f.loss_grad(z[3])]
+    jobs = [(c, c()) for c in calls]
+    assert run_together(jobs, 20) == []
