@@ -104,6 +104,7 @@ SIGNATURES = {
     "nuts_flow_pullback_grad": (C.c_int, [C.c_void_p, DP, DP, C.c_int, DP]),
     "nuts_flow_loss_grad": (C.c_int, [C.c_void_p, DP, C.c_int, DP, C.POINTER(C.c_float)]),
     "nuts_flow_train": (C.c_int, [C.c_void_p, DP, C.c_int64, C.c_int, C.c_int, C.c_double, C.c_uint64, DP]),
+    "nuts_release_workspaces": (C.c_size_t, []),
     "nuts_last_error": (C.c_char_p, []),
     "nuts_version": (C.c_char_p, []),
 }

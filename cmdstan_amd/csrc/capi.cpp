@@ -5,7 +5,6 @@
 
 #include <algorithm>
 #include <chrono>
-#include <exception>
 #include <cmath>
 #include <limits>
 #include <cstdio>
@@ -23,6 +22,7 @@
 #include "json.h"
 #include "rdump.h"
 #include "launch.h"
+#include "dev_pool.h"
 #include "flow.h"
 #include "hier_logistic.h"
 #include "glm_large.h"
@@ -47,84 +47,6 @@ struct HipError : std::runtime_error {
                      std::to_string(__LINE__));                                                         \
   } while (0)
 
-// Device workspace of a handle (a model or a flow), kept from call to call: a
-// call's buffers cost a hipMalloc and a hipFree each (tens of microseconds, and
-// hipFree waits for the device), more than a small call's kernels.  Blocks are
-// the handle's own and go with it; at most kKeep bytes stay cached, larger
-// buffers are freed at once.  A block belongs to one call until its work has
-// finished, so calls of several threads on one handle share none.
-class DevPool {
- public:
-  static constexpr size_t kKeep = (size_t)1 << 30;
-  DevPool() {}
-  DevPool(const DevPool&) = delete;
-  DevPool& operator=(const DevPool&) = delete;
-  ~DevPool() { clear(); }
-  // Around a call's use.  A call that left early may have work in flight on its
-  // buffers: the next one waits for the device first.
-  void begin() {
-    std::lock_guard<std::mutex> lock(mu_);
-    if (open_) (void)hipDeviceSynchronize();
-    open_ = true;
-  }
-  void end() {
-    std::lock_guard<std::mutex> lock(mu_);
-    open_ = false;
-  }
-  void* get(size_t bytes, size_t* got) {
-    std::lock_guard<std::mutex> lock(mu_);
-    size_t best = free_.size();
-    for (size_t i = 0; i < free_.size(); ++i)
-      if (free_[i].n >= bytes && free_[i].n <= 2 * bytes + 65536 && (best == free_.size() || free_[i].n < free_[best].n))
-        best = i;
-    if (best < free_.size()) {
-      void* p = free_[best].p;
-      *got = free_[best].n;
-      held_ -= free_[best].n;
-      free_.erase(free_.begin() + best);
-      return p;
-    }
-    bytes = (bytes + 511) & ~size_t(511);
-    void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-      (void)hipGetLastError();
-      clear();
-      HIPC(hipMalloc(&p, bytes));
-    }
-    *got = bytes;
-    return p;
-  }
-  void put(void* p, size_t n) {
-    std::lock_guard<std::mutex> lock(mu_);
-    // on the way out of an exception work may be in flight: hipFree waits for it
-    if (held_ + n > kKeep || std::uncaught_exceptions() > 0) {
-      (void)hipFree(p);
-      return;
-    }
-    free_.push_back({p, n});
-    held_ += n;
-  }
-
- private:
-  struct Block { void* p; size_t n; };
-  void clear() {
-    for (auto& b : free_) (void)hipFree(b.p);
-    free_.clear();
-    held_ = 0;
-  }
-  std::mutex mu_;
-  std::vector<Block> free_;
-  size_t held_ = 0;
-  bool open_ = false;
-};
-
-// a call's span of the handle's workspace: done() once its work has finished
-struct PoolSpan {
-  DevPool& p;
-  explicit PoolSpan(DevPool& p_) : p(p_) { p.begin(); }
-  void done() { p.end(); }
-};
-
 template <class T>
 struct DevBuf {
   T* p = nullptr;
@@ -137,8 +59,8 @@ struct DevBuf {
     free();
     n = n_;
     if (!n) return;
-    if (pool_) p = static_cast<T*>(pool_->get(n * sizeof(T), &bytes_));
-    else HIPC(hipMalloc(&p, n * sizeof(T)));
+    p = static_cast<T*>(pool_ ? pool_->get(n * sizeof(T), &bytes_) : DevPool::alloc(n * sizeof(T)));
+    if (!p) HIPC(DevMem::error());
   }
   void upload(const T* h, size_t cnt, hipStream_t st = 0) {
     if (cnt) HIPC(hipMemcpyAsync(p, h, cnt * sizeof(T), hipMemcpyHostToDevice, st));
@@ -688,7 +610,6 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   }
 
   DevPool* const ws = &M.ws;
-  PoolSpan span(M.ws);
   hipStream_t st;
   HIPC(hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
   struct StreamGuard { hipStream_t s; ~StreamGuard() { (void)hipStreamDestroy(s); } } sg{st};
@@ -1368,7 +1289,6 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   }
   HIPC(hipStreamSynchronize(st));
   HIPC(hipGetLastError());
-  span.done();
   return res;
 }
 
@@ -1559,6 +1479,7 @@ struct nuts_model {
 extern "C" {
 
 const char* nuts_last_error(void) { return g_err.c_str(); }
+size_t nuts_release_workspaces(void) { return DevPool::release(); }
 const char* nuts_version(void) { return "cmdstan_amd 0.1 (gfx950)"; }
 
 nuts_data* nuts_data_create(void) { return new nuts_data(); }
@@ -1977,7 +1898,6 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
     const int D = M.ds[dataset].D, C = n_points;
     if (precision != 0 && !((M.glm || M.glm_large) && dataset == 0))
       throw std::invalid_argument("reduced precision is available for the batched logistic regression only");
-    PoolSpan span(M.ws);
     DevPool* const ws = &M.ws;
     DevBuf<double> Q(ws, (size_t)C * D), G(ws, (size_t)C * D), V(ws, C), L(ws, C), work(ws);
     bool finish = true;  // V and grad V still to be turned into lp and its gradient
@@ -2046,7 +1966,6 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
     HIPC(hipGetLastError());
     HIPC(hipMemcpy(grad, G.p, (size_t)C * D * sizeof(double), hipMemcpyDeviceToHost));
     HIPC(hipMemcpy(lp, L.p, C * sizeof(double), hipMemcpyDeviceToHost));
-    span.done();
     return NUTS_OK;
   });
 }
@@ -2197,7 +2116,6 @@ int nuts_flow_forward(nuts_flow* f, const double* z, int n, double* x, double* l
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
     std::lock_guard<std::mutex> lock(f->mu);
-    PoolSpan span(f->ws);
     DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dl(&f->ws, n);
     dz.upload(z, (size_t)n * D, st);
     f->net->forward(dz.p, D, nullptr, nullptr, n, dx.p, dl.p);
@@ -2205,7 +2123,6 @@ int nuts_flow_forward(nuts_flow* f, const double* z, int n, double* x, double* l
     HIPC(hipMemcpyAsync(logdet, dl.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
     f->net->check_barriers();
-    span.done();
     return NUTS_OK;
   });
 }
@@ -2216,14 +2133,12 @@ int nuts_flow_inverse(nuts_flow* f, const double* x, int n, double* z, double* l
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
     std::lock_guard<std::mutex> lock(f->mu);
-    PoolSpan span(f->ws);
     DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dl(&f->ws, n);
     dx.upload(x, (size_t)n * D, st);
     f->net->inverse(dx.p, n, dz.p, dl.p);
     HIPC(hipMemcpyAsync(z, dz.p, (size_t)n * D * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipMemcpyAsync(logdet, dl.p, n * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
-    span.done();
     return NUTS_OK;
   });
 }
@@ -2234,7 +2149,6 @@ int nuts_flow_pullback_grad(nuts_flow* f, const double* z, const double* gx, int
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
     std::lock_guard<std::mutex> lock(f->mu);
-    PoolSpan span(f->ws);
     DevBuf<double> dz(&f->ws, (size_t)n * D), dx(&f->ws, (size_t)n * D), dgx(&f->ws, (size_t)n * D), dgz(&f->ws, (size_t)n * D), dl(&f->ws, n), dvx(&f->ws, n), dv(&f->ws, n);
     dz.upload(z, (size_t)n * D, st);
     dgx.upload(gx, (size_t)n * D, st);
@@ -2244,7 +2158,6 @@ int nuts_flow_pullback_grad(nuts_flow* f, const double* z, const double* gx, int
     HIPC(hipMemcpyAsync(gz, dgz.p, (size_t)n * D * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPC(hipStreamSynchronize(st));
     f->net->check_barriers();
-    span.done();
     return NUTS_OK;
   });
 }
@@ -2255,12 +2168,10 @@ int nuts_flow_loss_grad(nuts_flow* f, const double* x, int n, double* loss, floa
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
     std::lock_guard<std::mutex> lock(f->mu);
-    PoolSpan span(f->ws);
     DevBuf<double> dx(&f->ws, (size_t)n * D);
     dx.upload(x, (size_t)n * D, st);
     const double l = f->net->loss_grad(dx.p, n, grad);
     if (loss) *loss = l;
-    span.done();
     return NUTS_OK;
   });
 }
@@ -2273,13 +2184,11 @@ int nuts_flow_train(nuts_flow* f, const double* x, int64_t n, int steps, int bat
     const int D = f->net->dim();
     hipStream_t st = f->net->own_stream();
     std::lock_guard<std::mutex> lock(f->mu);
-    PoolSpan span(f->ws);
     DevBuf<double> dx(&f->ws, (size_t)n * D);
     dx.upload(x, (size_t)n * D, st);
     HIPC(hipStreamSynchronize(st));
     const double l = f->net->train(dx.p, n, steps, batch, (float)lr, seed, std::min(20, std::max(1, steps)));
     if (final_loss) *final_loss = l;
-    span.done();
     return NUTS_OK;
   });
 }

@@ -8,6 +8,7 @@
 #include <stdexcept>
 #include <string>
 
+#include "dev_pool.h"
 #include "device_common.h"
 #include "flow.h"
 #include "launch.h"
@@ -1072,9 +1073,10 @@ static dim3 grid1(int64_t n, int b = 256) { return dim3((unsigned)((n + b - 1) /
 
 template <class T>
 static T* dalloc(int64_t n) {
-  T* p = nullptr;
-  if (n > 0) HIPF(hipMalloc(&p, n * sizeof(T)));
-  return p;
+  if (n <= 0) return nullptr;
+  void* p = DevPool::alloc(n * sizeof(T));
+  if (!p) HIPF(DevMem::error());
+  return static_cast<T*>(p);
 }
 
 // ------------------------------------------------------------------- masks

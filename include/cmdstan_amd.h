@@ -16,7 +16,14 @@
  *
  * Conventions: plain pointers to caller-owned host memory; device memory is
  * owned by the library.  Every function returns NUTS_OK (0) or NUTS_NOT_OK (1)
- * and leaves a message for nuts_last_error().  One handle per host thread.
+ * and leaves a message for nuts_last_error().  Threads may share a handle: calls
+ * on one model run side by side (a plugin's callbacks have to allow it), calls
+ * on one flow one after the other; nuts_log_prob_grad_noalloc as it states.
+ *
+ * Workspaces: a model or flow handle keeps the device buffers of its calls for the
+ * next one, at most 1 GiB idle per handle and 4 GiB over all handles of the
+ * process.  They go with the handle, are given back when an allocation of this
+ * library fails, and on nuts_release_workspaces().
  */
 #ifndef CMDSTAN_AMD_H
 #define CMDSTAN_AMD_H
@@ -352,6 +359,9 @@ int nuts_flow_loss_grad(nuts_flow* f, const double* x, int n, double* loss, floa
 /* Adam on minibatches of `batch` rows drawn from the n rows of x */
 int nuts_flow_train(nuts_flow* f, const double* x, int64_t n, int steps, int batch, double lr, uint64_t seed,
                     double* final_loss);
+
+/* Frees the idle device workspaces of every handle (see above); their bytes. */
+size_t nuts_release_workspaces(void);
 
 const char* nuts_last_error(void);
 const char* nuts_version(void);
