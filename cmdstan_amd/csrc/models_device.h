@@ -33,7 +33,8 @@ struct BernoulliFn {
     s = md.d[1];
   }
   template <class T>
-  __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
+  __device__ __forceinline__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int,
+                                               int lane) const {
     // log1p_exp(u), log1p_exp(-u) and inv_logit(u) share e^-|u| and log1p of it
     const double u = q[0];
     const double e = exp(u >= 0 ? -u : u);
@@ -113,7 +114,8 @@ struct GaussFn {
     return acc;
   }
   template <class T>
-  __device__ double operator()(int, const T* __restrict__ q, T* __restrict__ gV, int D, int lane) const {
+  __device__ __forceinline__ double operator()(int, const T* __restrict__ q, T* __restrict__ gV, int D,
+                                               int lane) const {
     double acc = 0;
     if (D <= NUTS_WAVE) {
       acc = rows<1>(q, gV, D, lane, 0, acc);
@@ -136,7 +138,8 @@ struct EightSchoolsFn {
   ModelData md;
   __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
   template <class T>
-  __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
+  __device__ __forceinline__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int,
+                                               int lane) const {
     const double* d = md.d;
     const int J = (int)d[0];
     const double mu_s = d[1], tau_s = d[2];
@@ -178,7 +181,8 @@ struct HierNormalNCFn {
   // the gradient with TPC threads per chain (thread tid); sum reduces a
   // per-thread partial over the chain's threads in a fixed order
   template <int TPC, class T, class Sum>
-  __device__ double group(int c, const T* __restrict__ q, T* __restrict__ gV, int tid, const Sum& sum) const {
+  __device__ __forceinline__ double group(int c, const T* __restrict__ q, T* __restrict__ gV, int tid,
+                                          const Sum& sum) const {
     const double* d = md.d;
     const int J = (int)d[0];
     const double mu_s = d[1], tau_s = d[2];
@@ -207,7 +211,8 @@ struct HierNormalNCFn {
     return -lp;
   }
   template <class T>
-  __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
+  __device__ __forceinline__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int,
+                                               int lane) const {
     return group<NUTS_WAVE>(c, q, gV, lane, [](double x) { return wave_sum(x); });
   }
   __device__ int nout(int c) const { return 2 + 2 * (int)md.d[0]; }
@@ -230,7 +235,8 @@ struct HierLogisticFn {
   ModelData md;
   __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
   template <class T>
-  __device__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int, int lane) const {
+  __device__ __forceinline__ double operator()(int c, const T* __restrict__ q, T* __restrict__ gV, int,
+                                               int lane) const {
     const double* d = md.d;
     const int N = (int)d[0], K = (int)d[1], G = (int)d[2];
     const double mu_s = d[3];
@@ -300,7 +306,8 @@ struct LogisticFn {
   static constexpr bool vec32 = false;
   ModelData md;
   __device__ __forceinline__ void bind(int c) { md.d = md.data + md.off[c]; }
-  __device__ double operator()(int c, const double* __restrict__ q, double* __restrict__ gV, int D, int lane) const {
+  __device__ __forceinline__ double operator()(int c, const double* __restrict__ q, double* __restrict__ gV, int D,
+                                               int lane) const {
     const double* d = md.d;
     const int N = (int)d[0];
     const double s2inv = d[2];

@@ -25,6 +25,16 @@
 // sharp companion, computed once per leaf by a matvec with the per-chain D×D
 // inverse metric, and momenta p = L⁻ᵀ z are drawn with the chain's Cholesky
 // factor Minv = L Lᵀ, whose buffer also holds L⁻¹ (see dense_factor).
+//
+// Out-of-line functions.  A device function that can see a pointer or reference
+// to LDS or private memory (the state s, the LDS machine's vectors, a model
+// functor, arrays of sums) is forced inline.  An LDS address that every caller
+// passes alike is otherwise folded into the out-of-line copy, which then finds
+// the variable through the compiler's table of the calling kernels instead of
+// through its argument, and flat accesses take the place of LDS ones.  Out of
+// line are only stream_normal (scalars) and, on global-memory vectors,
+// dense_matvec, dense_matvec2 and dense_inverse; a test reads the built
+// library's symbols for any other.
 #pragma once
 #include "device_common.h"
 #include "nuts_types.h"
@@ -423,10 +433,7 @@ __device__ __forceinline__ void dense_matvec_lds(const double* __restrict__ M, c
 // into p_i when i < j and into ps_i when i > j; the diagonal terms z_i / L_ii
 // and L_ii z_i come last.  Every element of F is read once, columns
 // coalesced, with no sequential dependency between rows.  Inlined, not an
-// out-of-line call like the matvecs: z lives in the caller's LDS strip, and
-// an out-of-line copy that every caller passes the same strip was built with
-// that strip's address folded in as LDS offset 0, which is not where the
-// calling kernel placed it.
+// out-of-line call like the matvecs: z lives in the caller's LDS strip.
 template <int TPC, class VT>
 __device__ __forceinline__ void dense_tri_sample(const double* __restrict__ F, const double* __restrict__ z,
                                               VT* __restrict__ p, VT* __restrict__ ps, int D, int tid) {
@@ -610,13 +617,13 @@ struct NutsWave {
       }
     }
   }
-  static __device__ double gsum(double v) {
+  static __device__ __forceinline__ double gsum(double v) {
     double a[1] = {v};
     gsum_n(a);
     return a[0];
   }
   // global vector writes of the group visible to its other threads
-  static __device__ void gsync() {
+  static __device__ __forceinline__ void gsync() {
     if constexpr (TPC == NUTS_WAVE) {
       wave_sync();
     } else {
@@ -625,7 +632,7 @@ struct NutsWave {
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     }
   }
-  static __device__ int gand(int v) {
+  static __device__ __forceinline__ int gand(int v) {
     v = wave_and(v);
     if constexpr (TPC == NUTS_WAVE) {
       return v;
@@ -644,39 +651,41 @@ struct NutsWave {
   // that follow run with the full wave, never duplicated into the divergent
   // exits of the loop (where a read-modify-write of the shared state would
   // be applied once per lane group).
-  static __device__ void converge() { __builtin_amdgcn_wave_barrier(); }
-  static __device__ void lsync() {
+  static __device__ __forceinline__ void converge() { __builtin_amdgcn_wave_barrier(); }
+  static __device__ __forceinline__ void lsync() {
     if constexpr (TPC == NUTS_WAVE) lds_sync();
     else __syncthreads();
   }
 
-  __device__ VT* vecp(int id) const { return blk + (int64_t)id * Dp; }
-  __device__ VT* Lbeg(int k) const { return vecp(PV_FIXED + s.L_beg_vec[k]); }
-  __device__ VT* Lend(int k) const { return vecp(PV_FIXED + P.maxd + k); }
-  __device__ VT* Lrho(int k) const { return vecp(PV_FIXED + 2 * P.maxd + k); }
-  __device__ VT* Sq(int k) const { return vecp(PV_FIXED + 3 * P.maxd + k); }
-  __device__ VT* Sg(int k) const { return vecp(PV_FIXED + 3 * P.maxd + P.nslots + k); }
-  __device__ VT* LSbeg(int k) const { return vecp(PV_FIXED + 3 * P.maxd + 2 * P.nslots + k); }
-  __device__ VT* LSend(int k) const { return vecp(PV_FIXED + 4 * P.maxd + 2 * P.nslots + k); }
+  __device__ __forceinline__ VT* vecp(int id) const { return blk + (int64_t)id * Dp; }
+  __device__ __forceinline__ VT* Lbeg(int k) const { return vecp(PV_FIXED + s.L_beg_vec[k]); }
+  __device__ __forceinline__ VT* Lend(int k) const { return vecp(PV_FIXED + P.maxd + k); }
+  __device__ __forceinline__ VT* Lrho(int k) const { return vecp(PV_FIXED + 2 * P.maxd + k); }
+  __device__ __forceinline__ VT* Sq(int k) const { return vecp(PV_FIXED + 3 * P.maxd + k); }
+  __device__ __forceinline__ VT* Sg(int k) const { return vecp(PV_FIXED + 3 * P.maxd + P.nslots + k); }
+  __device__ __forceinline__ VT* LSbeg(int k) const { return vecp(PV_FIXED + 3 * P.maxd + 2 * P.nslots + k); }
+  __device__ __forceinline__ VT* LSend(int k) const { return vecp(PV_FIXED + 4 * P.maxd + 2 * P.nslots + k); }
   // momentum of a proposal slot (kept only for the diagnostic rows)
-  __device__ VT* Sp(int k) const { return vecp(PV_FIXED + (DENSE ? 5 : 3) * P.maxd + 2 * P.nslots + k); }
+  __device__ __forceinline__ VT* Sp(int k) const {
+    return vecp(PV_FIXED + (DENSE ? 5 : 3) * P.maxd + 2 * P.nslots + k);
+  }
 
   // ------------------------------------------------------------- metric
-  __device__ double mi(int i) const { return METRIC == METRIC_UNIT ? 1.0 : (double)minv[i]; }
+  __device__ __forceinline__ double mi(int i) const { return METRIC == METRIC_UNIT ? 1.0 : (double)minv[i]; }
   // sharp momentum element: x = momentum, xs = its stored companion (dense)
-  __device__ double sh(const VT* x, const VT* xs, int i) const {
+  __device__ __forceinline__ double sh(const VT* x, const VT* xs, int i) const {
     if (DENSE) return xs[i];
     return METRIC == METRIC_UNIT ? (double)x[i] : (double)minv[i] * (double)x[i];
   }
   // out = Minv x (dense)
-  __device__ void matvec(const VT* x, VT* out) const {
+  __device__ __forceinline__ void matvec(const VT* x, VT* out) const {
     gsync();
     if constexpr (LV) dense_matvec_lds<1>(dM, x, (const VT*)nullptr, out, (VT*)nullptr, D, lane);
     else dense_matvec<TPC, VT>(dM, x, out, D, tid);
     gsync();
   }
   // T = 1/2 p·Minv p; for dense ps must hold Minv p
-  __device__ double kinetic(const VT* p, const VT* ps) const {
+  __device__ __forceinline__ double kinetic(const VT* p, const VT* ps) const {
     const VT* __restrict__ pr = p;
     const VT* __restrict__ sr = DENSE ? ps : (METRIC == METRIC_UNIT ? p : minv);
     double a = 0;
@@ -690,22 +699,22 @@ struct NutsWave {
   }
 
   // ------------------------------------------------------------- draws
-  __device__ double uniform() {
+  __device__ __forceinline__ double uniform() {
     const uint64_t k = s.uctr++;
     if (B.inj_u) return k < (uint64_t)B.n_inj_u ? B.inj_u[(int64_t)c * B.n_inj_u + k] : 0.5;
     return stream_uniform(P.seed, uid, STREAM_UNIFORM, k);
   }
-  __device__ double normal_draw(int i) const {
+  __device__ __forceinline__ double normal_draw(int i) const {
     if (B.inj_z) {
       const uint64_t k = s.nctr + (uint64_t)i;
       return k < (uint64_t)B.n_inj_z ? B.inj_z[(int64_t)c * B.n_inj_z + k] : 0.0;
     }
     return stream_normal(P.seed, uid, s.nctr + (uint64_t)(i >> 1), i & 1);
   }
-  __device__ void advance_normals() { s.nctr += B.inj_z ? (uint64_t)D : (uint64_t)((D + 1) / 2); }
+  __device__ __forceinline__ void advance_normals() { s.nctr += B.inj_z ? (uint64_t)D : (uint64_t)((D + 1) / 2); }
 
   // {unit,diag,dense}_e_metric::sample_p; for dense also sets ps = Minv p
-  __device__ void sample_p(VT* p, VT* ps) {
+  __device__ __forceinline__ void sample_p(VT* p, VT* ps) {
     if (!DENSE) {
       for (int i = tid; i < D; i += TPC) {
         const double z = normal_draw(i);
@@ -730,16 +739,16 @@ struct NutsWave {
   // ------------------------------------------------------------- vectors
   // the pool vectors never alias each other: restrict lets the unrolled loops
   // issue several independent loads before their stores
-  __device__ void copy(VT* __restrict__ dst, const VT* __restrict__ src) const {
+  __device__ __forceinline__ void copy(VT* __restrict__ dst, const VT* __restrict__ src) const {
 #pragma unroll(UN)
     for (int i = tid; i < D; i += TPC) dst[i] = src[i];
     converge();
   }
-  __device__ void swap(VT* a, VT* b) const {
+  __device__ __forceinline__ void swap(VT* a, VT* b) const {
     for (int i = tid; i < D; i += TPC) { const VT t = a[i]; a[i] = b[i]; b[i] = t; } converge();
   }
   // expl_leapfrog: begin_update_p(eps/2), update_q(eps)
-  __device__ void leap_begin(double e) const {
+  __device__ __forceinline__ void leap_begin(double e) const {
     VT* p = vecp(PV_P);
     const double h = 0.5 * e;
     if (DENSE) {
@@ -761,7 +770,7 @@ struct NutsWave {
     converge();
   }
   // end_update_p(eps/2); dense: also the leaf's sharp momentum
-  __device__ void leap_end(double e) const {
+  __device__ __forceinline__ void leap_end(double e) const {
     VT* __restrict__ p = vecp(PV_P);
     const VT* __restrict__ gr = g;
     const double h = 0.5 * e;
@@ -773,7 +782,7 @@ struct NutsWave {
 
   // dense_e leaf: end_update_p(eps/2), then the sharp momentum M p and M g in
   // one pass over the metric; M g stays in PV_TMP for leap_begin_mg
-  __device__ void leap_end_mg(double e) const {
+  __device__ __forceinline__ void leap_end_mg(double e) const {
     VT* __restrict__ p = vecp(PV_P);
     const VT* __restrict__ gr = g;
     const double h = 0.5 * e;
@@ -787,7 +796,7 @@ struct NutsWave {
   // dense_e: begin_update_p(eps/2) and update_q(eps) of the next leaf, with
   // M (p - h g) = M p - h M g from the products leap_end_mg left (g unchanged
   // in between): no second pass over the metric
-  __device__ void leap_begin_mg(double e) const {
+  __device__ __forceinline__ void leap_begin_mg(double e) const {
     VT* __restrict__ p = vecp(PV_P);
     const VT* __restrict__ ps = vecp(PV_PS);
     VT* __restrict__ t = vecp(PV_TMP);
@@ -803,14 +812,14 @@ struct NutsWave {
   }
 
   // ------------------------------------------------------------- slots
-  __device__ int alloc_slot() {
+  __device__ __forceinline__ int alloc_slot() {
     const uint32_t m = s.free_mask;
     const int k = __builtin_ctz(m);  // a free slot always exists (<= maxd+1 live)
     s.free_mask = m & ~(1u << k);
     return k;
   }
-  __device__ void free_slot(int k) { if (k >= 0) s.free_mask |= (1u << k); }
-  __device__ int store_leaf_slot() {
+  __device__ __forceinline__ void free_slot(int k) { if (k >= 0) s.free_mask |= (1u << k); }
+  __device__ __forceinline__ int store_leaf_slot() {
     const int k = alloc_slot();
     copy(Sq(k), q);
     copy(Sg(k), g);
@@ -820,10 +829,10 @@ struct NutsWave {
     return k;
   }
 
-  __device__ double pending_V() const { return have_v ? v_new : B.V[c]; }
+  __device__ __forceinline__ double pending_V() const { return have_v ? v_new : B.V[c]; }
 
   // -------------------------------------------------------- control flow
-  __device__ bool request(int next) {
+  __device__ __forceinline__ bool request(int next) {
     s.phase = next;
     s.n_grad++;
     return true;
@@ -831,21 +840,21 @@ struct NutsWave {
   // the machine goes on at `phase`: steps reached from several places are
   // phases of their own, so their code is there once (the loop's instructions
   // are fetched through a 64 KB cache)
-  __device__ bool then(int phase) {
+  __device__ __forceinline__ bool then(int phase) {
     s.phase = phase;
     return false;
   }
-  __device__ void stop(int phase) {
+  __device__ __forceinline__ void stop(int phase) {
     s.phase = phase;
     if (tid == 0) atomicAdd(B.n_stopped, 1); converge();
   }
-  __device__ void fail(int code) {
+  __device__ __forceinline__ void fail(int code) {
     s.failure = code;
     stop(PH_FAILED);
   }
 
   // services::util::initialize
-  __device__ bool init_try() {
+  __device__ __forceinline__ bool init_try() {
     const int t = s.init_tries;
     for (int i = tid; i < D; i += TPC) {
       double v;
@@ -860,7 +869,7 @@ struct NutsWave {
     } converge();
     return request(PH_INIT_CHECK);
   }
-  __device__ bool init_check() {
+  __device__ __forceinline__ bool init_check() {
     const double V = pending_V();
     int ok = 1;
     for (int i = tid; i < D; i += TPC) ok &= isfinite(g[i]) ? 1 : 0; converge();
@@ -884,7 +893,7 @@ struct NutsWave {
   }
 
   // base_hmc::init_stepsize
-  __device__ bool ss_probe_begin() {
+  __device__ __forceinline__ bool ss_probe_begin() {
     const int k = s.sample_slot;
     copy(q, Sq(k));
     copy(g, Sg(k));
@@ -896,13 +905,13 @@ struct NutsWave {
     leap_begin(s.nom_eps);
     return request(PH_SS_PROBE);
   }
-  __device__ bool ss_start() {
+  __device__ __forceinline__ bool ss_start() {
     const double e = s.nom_eps;
     if (e == 0 || e > 1e7 || isnan(e)) { ss_finish(); return false; }
     s.ss_first = 1;
     return then(PH_SS_BEGIN);
   }
-  __device__ bool ss_probe() {
+  __device__ __forceinline__ bool ss_probe() {
     s.Vz = pending_V();
     leap_end(s.nom_eps);
     double h = kinetic(vecp(PV_P), vecp(PV_PS)) + s.Vz;
@@ -921,7 +930,7 @@ struct NutsWave {
     if (s.nom_eps == 0) { fail(FAIL_STEPSIZE_ZERO); return false; }
     return then(PH_SS_BEGIN);
   }
-  __device__ void ss_finish() {
+  __device__ __forceinline__ void ss_finish() {
     if (s.ss_return == SS_RET_WINDOW) {
       s.sa_mu = log(10 * s.nom_eps);
       s.sa_counter = 0; s.sa_sbar = 0; s.sa_xbar = 0;
@@ -932,7 +941,7 @@ struct NutsWave {
   }
 
   // base_nuts::transition, set-up part
-  __device__ void trans_begin() {
+  __device__ __forceinline__ void trans_begin() {
     if (s.iter >= P.iter_target) { stop(PH_PAUSED); return; }
     s.eps = s.nom_eps;
     if (P.jitter != 0) s.eps *= 1.0 + P.jitter * (2.0 * uniform() - 1.0);
@@ -974,7 +983,7 @@ struct NutsWave {
     s.phase = PH_DOUBLING_BEGIN;
   }
 
-  __device__ bool doubling_begin() {
+  __device__ __forceinline__ bool doubling_begin() {
     const int fwd = uniform() > 0.5 ? 1 : 0;
     if (fwd != s.z_is_fwd) {
       swap(q, vecp(PV_OQ));
@@ -1018,7 +1027,7 @@ struct NutsWave {
   // into (K = the trailing one bits of the leaf index), or in p and srho at
   // the doubling's last leaf.  When a check fails, the transition ends and
   // those stores are never read.
-  __device__ bool leaf() {
+  __device__ __forceinline__ bool leaf() {
     if constexpr (DENSE) {
       return leaf_dense();
     } else {
@@ -1129,7 +1138,7 @@ struct NutsWave {
 
   // build_tree base case and merges for dense_e (the sharp momenta are kept
   // beside the momenta in every checkpoint)
-  __device__ bool leaf_dense() {
+  __device__ __forceinline__ bool leaf_dense() {
     const double e = s.dir * s.eps;
     s.Vz = pending_V();
     VT* p = vecp(PV_P);
@@ -1239,7 +1248,7 @@ struct NutsWave {
   }
 
   // top-level merge of a complete, valid subtree (biased progressive sampling)
-  __device__ void doubling_end() {
+  __device__ __forceinline__ void doubling_end() {
     s.depth++;
     bool take;
     if (s.S_logw > s.log_w) take = true;
@@ -1278,12 +1287,14 @@ struct NutsWave {
   }
 
   // window logic of stan::mcmc::windowed_adaptation (unsigned arithmetic)
-  __device__ bool in_window() const {
+  __device__ __forceinline__ bool in_window() const {
     return (s.w_counter >= P.w_init_buffer) && (s.w_counter < P.w_num_warmup - P.w_term_buffer) &&
            (s.w_counter != P.w_num_warmup);
   }
-  __device__ bool end_window() const { return (s.w_counter == s.w_next) && (s.w_counter != P.w_num_warmup); }
-  __device__ void next_window() {
+  __device__ __forceinline__ bool end_window() const {
+    return (s.w_counter == s.w_next) && (s.w_counter != P.w_num_warmup);
+  }
+  __device__ __forceinline__ void next_window() {
     if (s.w_next == P.w_num_warmup - P.w_term_buffer - 1) return;
     s.w_size *= 2;
     s.w_next = s.w_counter + s.w_size;
@@ -1294,7 +1305,7 @@ struct NutsWave {
   }
   // var_adaptation::learn_variance / covar_adaptation::learn_covariance;
   // returns true at a window end
-  __device__ bool learn_metric(const VT* qs) {
+  __device__ __forceinline__ bool learn_metric(const VT* qs) {
     VT* wm = vecp(PV_WM);
     VT* wm2 = vecp(PV_WM2);
     if (in_window()) {
@@ -1366,7 +1377,7 @@ struct NutsWave {
   }
 
   // end of base_nuts::transition + adapt_*_e_nuts::transition + writer
-  __device__ void trans_end() {
+  __device__ __forceinline__ void trans_end() {
     const double accept = s.sum_metro / (double)s.n_leapfrog;
     const int k = s.sample_slot;
     s.n_leapfrog_total += s.n_leapfrog;
@@ -1422,7 +1433,7 @@ struct NutsWave {
     iteration_next();
   }
 
-  __device__ void iteration_next() {
+  __device__ __forceinline__ void iteration_next() {
     s.iter++;
     if (s.iter == P.num_warmup && s.adapt_flag) {
       s.adapt_flag = 0;
@@ -1433,7 +1444,7 @@ struct NutsWave {
   }
 
   // One step of the machine; true when V, G at Q are needed next.
-  __device__ bool dispatch() {
+  __device__ __forceinline__ bool dispatch() {
     switch (s.phase) {
       case PH_INIT_TRY: return init_try();
       case PH_INIT_CHECK: return init_check();
@@ -1449,7 +1460,7 @@ struct NutsWave {
     }
   }
 
-  __device__ void run() {
+  __device__ __forceinline__ void run() {
     int budget = GradFn::fused ? P.fused_budget : 1;
     for (;;) {
       if (s.phase >= PH_PAUSED) {
@@ -1478,7 +1489,7 @@ struct NutsWave {
   // Lower Cholesky factor of the column-major SPD matrix A into L (column-major),
   // left-looking, one column per step with the wave splitting the rows.
   // Returns false if a pivot is not positive.
-  static __device__ bool dense_factor(const double* A, double* L, int D, int tid) {
+  static __device__ __forceinline__ bool dense_factor(const double* A, double* L, int D, int tid) {
     for (int j = 0; j < D; ++j) {
       // pivot: A[j][j] - sum_k L[j][k]^2 (row j of L = element j of columns k < j)
       double sq = 0;
