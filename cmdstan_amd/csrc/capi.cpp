@@ -244,9 +244,6 @@ void gl_bind(ModelImpl& M, GlLargeArgs& a, const GlLargePlan& p, GlScratch& s, i
   }
 }
 
-// Register layout of the 16x16 f32 MFMA result (0: row 4*(l/16)+i, 1: row 4i + l/16).
-constexpr int kF32Layout = 0;
-
 std::vector<std::string> idx_names(const std::string& base, int n) {
   std::vector<std::string> r;
   for (int i = 0; i < n; ++i) r.push_back(base + "." + std::to_string(i + 1));
@@ -533,7 +530,7 @@ ModelImpl::GlmTune glm_autotune(ModelImpl& M, int C, int precision, hipStream_t 
     GlmArgs ga{M.d_X, M.d_y, N, D, C, gp.rows_per_chunk, M.glm_s2inv, Q.p, Dp, G.p, V.p, work.p};
     const double ms = time_it([&]() {
       if (precision == 0) glm_grad_mfma_f64(ga, gp, st);
-      else glm_grad_mfma_f32(ga, gp, xl.get(), precision, kF32Layout, st);
+      else glm_grad_mfma_f32(ga, gp, xl.get(), precision, st);
     });
     if (ms < best.ms) { best.ms = ms; best.path = 0; best.blocks_per_cu = bpc; }
   }
@@ -929,7 +926,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
   if (!fused && gw_ok) {
     act_idx.alloc(C);
     n_act.alloc(1);
-    gwplan = glm_wide_plan(M.glmN, C, M.glmD, num_cus());
+    gwplan = glm_wide_plan(C, M.glmD, num_cus());
     work.alloc(gwplan.work_doubles);
     ga.X = M.d_X; ga.y = M.d_y; ga.N = M.glmN; ga.D = M.glmD; ga.C = C; ga.rows_per_chunk = 0;
     ga.s2inv = M.glm_s2inv; ga.Q = Q.p; ga.ldq = Dp[0]; ga.G = G.p; ga.V = V.p; ga.work = work.p;
@@ -947,7 +944,7 @@ RunResult run_batch(ModelImpl& M, const RunSpec& R) {
     }
     const int rcg = cfg.precision == 0 ? glm_grad_mfma_f64(ga, gplan, st)
                     : xbf ? glm_grad_mfma_bf16(ga, gplan, xbf, cfg.precision, st)
-                          : glm_grad_mfma_f32(ga, gplan, xlow, cfg.precision, kF32Layout, st);
+                          : glm_grad_mfma_f32(ga, gplan, xlow, cfg.precision, st);
     if (rcg) throw std::runtime_error("GLM kernel: unsupported D");
   };
 
@@ -1925,7 +1922,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
         x = M.low_x(precision, 0);
         gl_large_grad(a, gp, x.get(), precision, 0);
       } else if (M.glm_wide) {
-        const GlmWidePlan gp = glm_wide_plan(M.glmN, C, D, num_cus());
+        const GlmWidePlan gp = glm_wide_plan(C, D, num_cus());
         work.alloc(gp.work_doubles);
         ga.work = work.p;
         rcg = glm_grad_wide_f64(ga, gp, 0);
@@ -1937,7 +1934,7 @@ static int log_prob_grad_impl(nuts_model* m, int dataset, const double* q, int n
         if (precision != 0) x = tn.path == 2 ? M.bf16_x(precision, 0) : M.low_x(precision, 0);
         rcg = precision == 0 ? glm_grad_mfma_f64(ga, gp, 0)
               : tn.path == 2 ? glm_grad_mfma_bf16(ga, gp, static_cast<const unsigned short*>(x.get()), precision, 0)
-                             : glm_grad_mfma_f32(ga, gp, x.get(), precision, kF32Layout, 0);
+                             : glm_grad_mfma_f32(ga, gp, x.get(), precision, 0);
       }
       if (rcg) throw std::runtime_error("GLM kernel: unsupported D");
     } else if (M.kind == MK_HIER_LOGISTIC) {
@@ -2025,7 +2022,7 @@ extern "C" int nuts_log_prob_grad_noalloc(nuts_model* m, int dataset, const doub
       finish = false;
       if (glm_grad_mfma_f64(ga, gp, st)) throw std::runtime_error("GLM kernel: unsupported D");
     } else if (M.glm_wide && dataset == 0) {
-      const GlmWidePlan gp = glm_wide_plan(M.glmN, n, D, num_cus(), work_cap);
+      const GlmWidePlan gp = glm_wide_plan(n, D, num_cus(), work_cap);
       need(gp.work_doubles);
       GlmArgs ga{M.d_X, M.d_y, M.glmN, D, n, 0, M.glm_s2inv, d_q, D, d_grad, d_lp, work};
       ga.sign = -1.0;

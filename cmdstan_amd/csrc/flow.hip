@@ -1258,13 +1258,13 @@ void FlowNet::gemm(const float* A, int64_t sam, int64_t sak, const float* B, int
     if ((int64_t)splits * M * N > part_n_) throw std::logic_error("flow: split-K workspace too small");
     g.part = part_;
   }
-  // the operand's unit stride picks the variant (every product here has one)
+  // the operands' unit strides pick the variant; every product here has one in A's k or B's n
   const dim3 grid(tn, tm, splits), blk(256);
   const bool ak = sak == 1, bn = sbn == 1;
   if (ak && bn) hipLaunchKernelGGL((flow_gemm_kernel<true, true>), grid, blk, 0, st_, g);
   else if (ak) hipLaunchKernelGGL((flow_gemm_kernel<true, false>), grid, blk, 0, st_, g);
   else if (bn) hipLaunchKernelGGL((flow_gemm_kernel<false, true>), grid, blk, 0, st_, g);
-  else hipLaunchKernelGGL((flow_gemm_kernel<false, false>), grid, blk, 0, st_, g);
+  else throw std::logic_error("flow: product without a unit stride");
   if (splits > 1) hipLaunchKernelGGL(flow_gemm_reduce, grid_rc(M, N), dim3(256), 0, st_, g);
 }
 

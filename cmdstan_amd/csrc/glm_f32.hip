@@ -272,12 +272,10 @@ static void gf_launch_tiles(const GlmArgs& a, const GlmPlan& p, const void* Xlow
 }
 
 // The reduce kernel of the FP64 path sums the chunk partials in FP64.
-int glm_grad_mfma_f32(const GlmArgs& a, const GlmPlan& p, const void* Xlow, int precision, int layout,
-                      hipStream_t st) {
+int glm_grad_mfma_f32(const GlmArgs& a, const GlmPlan& p, const void* Xlow, int precision, hipStream_t st) {
   if (a.D > GF_KMAX || a.D < 1) return 1;
   double* Wg = a.work;
   double* Wlp = a.work + (size_t)p.total_blocks * GF_TC * a.D;
-  (void)layout;  // the 16x16 f32 result layout measured on gfx950 is layout 0
   if (a.ev_begin) (void)hipEventRecord(a.ev_begin, st);
   if (precision == 1) gf_launch_tiles<float>(a, p, Xlow, Wg, Wlp, st);
   else gf_launch_tiles<unsigned short>(a, p, Xlow, Wg, Wlp, st);

@@ -15,7 +15,7 @@ struct GlmWidePlan {
 
 bool glm_wide_ok(int D);
 // max_doubles bounds the workspace of the gradient partials
-GlmWidePlan glm_wide_plan(int N, int C, int D, int num_cus, size_t max_doubles = (size_t)1 << 40);
+GlmWidePlan glm_wide_plan(int C, int D, int num_cus, size_t max_doubles = (size_t)1 << 40);
 int glm_grad_wide_f64(const GlmArgs& a, const GlmWidePlan& p, hipStream_t st);
 
 }  // namespace nutsgpu

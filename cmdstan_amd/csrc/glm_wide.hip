@@ -18,7 +18,7 @@
 // per tile.  Splitting the columns over the waves, not the points, keeps 16 or
 // 32 points enough to fill a block, so a few points still spread over every CU
 // by row chunks.  Measured, N = 10000, D = 500: 64 points 24.0 ms with a wave
-// per point (LogisticFn) -> 64 us (52 us in this kernel, 24.5 TFLOP/s), 4
+// per point (LogisticFn) -> 57 us (51.6 us in this kernel, 24.8 TFLOP/s), 4
 // points 36 us, 1024 points 601 us (34 TFLOP/s).  One block of eight waves per
 // CU: two blocks of four waves (8 tiles each) spilled and took 98 us, and
 // skipping the tiles past D by branches cost 90 us (the operand reads no
@@ -274,9 +274,8 @@ glm_wide_reduce(GlmArgs a, int total_blocks, int max_chunks, int gp, const doubl
 
 bool glm_wide_ok(int D) { return D > 128 && D <= 1024; }
 
-GlmWidePlan glm_wide_plan(int N, int C, int D, int num_cus, size_t max_doubles) {
+GlmWidePlan glm_wide_plan(int C, int D, int num_cus, size_t max_doubles) {
   GlmWidePlan p;
-  (void)N;
   // 32 points per block feed each operand read to two products; 16 where that
   // holds every point, and above 512 columns (registers)
   p.gp = C > 16 && D <= 512 ? 32 : 16;

@@ -20,7 +20,6 @@
 namespace nutsgpu {
 
 #define HL_OBS 128   // observations staged per LDS pass
-#define HL_KMAX 16
 #define HL_HW 16     // waves of a hyperparameter block
 
 // partials of the hyperparameters: column j of group g at ((j G) + g) n + pos
@@ -197,7 +196,7 @@ void hl_grad_launch(const HlArgs& a, int G, int K, hipStream_t st) {
     HL_CASE(1) HL_CASE(2) HL_CASE(3) HL_CASE(4) HL_CASE(5) HL_CASE(6) HL_CASE(7) HL_CASE(8)
     HL_CASE(9) HL_CASE(10) HL_CASE(11) HL_CASE(12) HL_CASE(13) HL_CASE(14) HL_CASE(15) HL_CASE(16)
 #undef HL_CASE
-    default: return;  // the model is refused at K > HL_KMAX
+    default: return;  // the model is refused at K > 16
   }
   hipLaunchKernelGGL(hl_hyper_kernel, dim3((a.n_rows + 63) / 64, 2 * K + 1), dim3(64 * HL_HW), 0, st, a);
 }
