@@ -129,7 +129,6 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
   LogProduct lg[IT];
 #pragma unroll
   for (int m = 0; m < IT; ++m) lp[m] = 0.0;
-  int tile = 0;
   if (n_begin < n_end) fetch(n_begin);
   for (int nb = n_begin; nb < n_end; nb += 16) {
 #pragma unroll
@@ -171,6 +170,7 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
           const double d = 1.0 + t;
           lp[m] += yy * e - (e > 0.0 ? e : 0.0);
           lg[m].times(t, d);
+          lg[m].fold();
           r = (e >= 0.0 ? 1.0 : t) * recip_small(d) - yy;
         }
         sR[64 * item + l] = r;
@@ -189,10 +189,6 @@ glm_wide_f64(GlmArgs a, int total_blocks, int max_chunks, double* __restrict__ W
         for (int g = 0; g < NG; ++g)
           gacc[g][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(r[g], x, gacc[g][t], 0, 0, 0);
       }
-    }
-    if (++tile % 512 == 0) {
-#pragma unroll
-      for (int m = 0; m < IT; ++m) lg[m].fold();
     }
   }
   // gacc[g][t] register i = G[point 16 g + 4i + lk][col0(t) + lr]; a single chunk is the whole sum
