@@ -172,7 +172,14 @@ struct LogProduct {
     e += x;
     u = __builtin_amdgcn_ldexp(u, -x) + (__builtin_amdgcn_ldexp(1.0, -x) - 1.0);
   }
-  __device__ __forceinline__ double log_value() const { return log1p(u) + (double)e * 0.69314718055994531; }
+  // log1p(u) for u in [0, 1): log of the rounded d = 1 + u, plus what d leaves out
+  // of u (over d, but that is within half a rounding of the result).  log1p's own
+  // code is longer: glm_mfma_f64 at N = 10000, D = 25, 4 points 5.63 us with it, 5.47.
+  __device__ __forceinline__ double log_value() {
+    fold();
+    const double d = 1.0 + u;
+    return (log(d) + (u - (d - 1.0))) + (double)e * 0.69314718055994531;
+  }
 };
 
 __device__ __forceinline__ double log1p_exp(double a) {
